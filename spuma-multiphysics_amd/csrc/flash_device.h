@@ -201,12 +201,38 @@ enum CandidateFlags : uint32_t {
     kRestartsSearched = 1u,  // the search ran the restart temperatures
     kOverflow = 2u,          // more distinct candidates than the set holds
     kSeedsPruned = 4u,       // the stable-gas pruning skipped the seeds
+    kDirect = 8u,            // the directed search's (saturation table): one candidate or none
 };
+enum StartBits : uint32_t {
+    kStartFound = 1u,   // converged, or stalled near convergence
+    kStartStable = 2u,  // converged and stable in single precision
+};
+constexpr int kStarts = 7, kRestarts = 20;  // all gas, all liquid, five seeds; the seeds from four temperatures
 struct CandidateSet {
     uint32_t count, flags;
     Candidate c[kMaxCandidates];
 };
 static_assert(sizeof(CandidateSet) == 104, "candidate set layout");
+
+// Appends a converged candidate to the set; dedupe: unless one of its kind
+// lies within 1e-4 of it.
+RD void noteCandidate(CandidateSet& set, int16_t kind, int16_t index, const float* x, bool dedupe) {
+    if (dedupe)
+        for (uint32_t i = 0; i < set.count; ++i) {
+            const Candidate& o = set.c[i];
+            if (o.kind == kind && ab(x[0] - o.x[0]) <= 1e-4f && ab(x[1] - o.x[1]) <= 1e-4f &&
+                ab(x[2] - o.x[2]) <= 1e-4f)
+                return;
+        }
+    if (set.count == kMaxCandidates) {
+        set.flags |= kOverflow;
+        return;
+    }
+    Candidate& o = set.c[set.count++];
+    o.x[0] = x[0]; o.x[1] = x[1]; o.x[2] = x[2];
+    o.kind = kind;
+    o.index = index;
+}
 
 // Full-pivot LU with Eigen's rank rule (reactiveDeviceFlash.h:111-139), n fixed.
 template <int n, class R>
@@ -1463,22 +1489,49 @@ struct Flash : FlashCap<CAP, R> {
     // entropy are judged here only to decide, as the reference does, whether
     // the restart temperatures run; the FP64 refinement judges them again.
     RD void note(int16_t kind, int16_t index, const R* x, bool dedupe) {
-        CandidateSet& set = *record;
-        if (dedupe)
-            for (uint32_t i = 0; i < set.count; ++i) {
-                const Candidate& o = set.c[i];
-                if (o.kind == kind && ab(float(x[0]) - o.x[0]) <= 1e-4f && ab(float(x[1]) - o.x[1]) <= 1e-4f &&
-                    ab(float(x[2]) - o.x[2]) <= 1e-4f)
-                    return;
+        const float at[3] = {float(x[0]), float(x[1]), float(x[2])};
+        noteCandidate(*record, kind, index, at, dedupe);
+    }
+    // One start of the search on its own (searchStartsKernel): 0 the all-gas
+    // solve, 1 the all-liquid one, 2 + j seed j, 7 + 5 t + j seed j from restart
+    // temperature t, in searchRecord's order.  Every start begins at the
+    // cell's own inputs, so running them apart finds what the sequence finds.
+    // x: the point reached; returns kStart* bits (0: no such start, or no candidate).
+    // `start` is the same in every lane that calls: where lanes take both
+    // sides of a branch around calls, the compiler may keep a call's saved
+    // scalar registers, written for the whole wave, in the stack slot of a
+    // value that the lanes of the other side still need.
+    RAMD_NOINLINE uint32_t searchStart(int start, R* x) {
+        if (!fin(energy) || !(density() > 0)) return 0;
+        for (int k = 0; k < NS; ++k)
+            if (!fin(q[k]) || q[k] < 0) return 0;
+        E candidate;
+        bool ok;
+        if (start < 2) {
+            if (start == 1) {
+                if (!NL) return 0;
+                R other = 0;
+                for (int k = 0; k < NS; ++k)
+                    if (k != mod().condensable) other += q[k];
+                if (other != 0) return 0;
             }
-        if (set.count == kMaxCandidates) {
-            set.flags |= kOverflow;
-            return;
+            ok = frozen(start == 0 ? R(0) : q[mod().condensable], candidate, 0);
+            if (!ok && !stalled) return 0;
+            x[0] = m_log(candidate.p);
+            x[1] = m_log(candidate.T);
+            x[2] = 0;
+        } else {
+            if (!NL || !(q[mod().condensable] > 0)) return 0;
+            const bool restart = start >= 7;
+            const int j = restart ? (start - 7) % 5 : start - 2;
+            const R seed = j == 0 ? R(-1) : j == 1 ? R(.5) : j == 2 ? R(.95) : j == 3 ? R(.1) : R(.9999);
+            R scale;
+            ++n.candidates;
+            activeStart(seed, restart, restart ? restartTemperature((start - 7) / 5) : R(0), x, scale);
+            ok = activeNewton(x, scale, candidate, 0);
+            if (!ok && !stalled) return 0;
         }
-        Candidate& o = set.c[set.count++];
-        o.x[0] = float(x[0]); o.x[1] = float(x[1]); o.x[2] = float(x[2]);
-        o.kind = kind;
-        o.index = index;
+        return kStartFound | (ok && stable(candidate) ? kStartStable : 0u);
     }
     RAMD_NOINLINE void searchRecord(CandidateSet& set) {
         record = &set;
@@ -1654,6 +1707,8 @@ struct Flash : FlashCap<CAP, R> {
     // FP64 restart search inline, the refinement stops with *deferred = true;
     // the caller reruns such cells with deferred == nullptr in a launch of
     // their own, so the long searches do not hold up the other lanes of a wave.
+    // A set of the saturation table (kDirect) is only tried: where none of its
+    // candidates is confirmed, *deferred = true and the cell is searched.
     RAMD_NOINLINE bool refine(const CandidateSet& set, E& best, bool* deferred = nullptr) {
         if (!fin(energy) || !(density() > 0)) return false;
         for (int k = 0; k < NS; ++k)
@@ -1665,6 +1720,7 @@ struct Flash : FlashCap<CAP, R> {
         bool have = false;
         E candidate;
         bool gasStable = false;
+        const bool direct = deferred && (set.flags & kDirect);
         const bool prunable = mod().stableGasPrune != 0;
         uint32_t i = 0;
         const bool recorded = i < set.count && set.c[i].kind == kGasCandidate;
@@ -1709,6 +1765,10 @@ struct Flash : FlashCap<CAP, R> {
         for (; i < set.count && set.c[i].kind == kSeedCandidate; ++i) {
             if (finishActive(set.c[i], candidate)) consider(candidate, best, have, true);
             else ++n.failures;
+        }
+        if (direct) {  // no stable point among the table's: the cell is searched
+            *deferred = !have;
+            return have;
         }
         if (!have && q[c] > 0 && restartRange()) {
             if (!(set.flags & kRestartsSearched)) {

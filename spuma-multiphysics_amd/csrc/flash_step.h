@@ -63,38 +63,67 @@ __device__ inline const HemModel<NS>& workgroupModel(const HemModel<NS>* __restr
 #endif
 }
 
-// Loads cell c into a flash: species masses, e = rhoE - |rho u|^2 / (2 rho)
-// (ReactiveFoam.C:727-728, in FP64) and the step-start seed.
-template <class F>
-__device__ inline void loadCell(F& f, const double* __restrict__ q, size_t stride, const ThermoOut& g, uint32_t c,
-                                int ns) {
-    using R = decltype(f.energy);
-    double rho = 0, mass[4];
-    for (int k = 0; k < ns; ++k) {
-        mass[k] = q[size_t(k) * stride + c];
-        f.q[k] = R(mass[k]);
-        rho += mass[k];
+// The inputs of a flash batch, by cell.  The resident step's: conserved SoA
+// q[k stride + c], e = rhoE - |rho u|^2 / (2 rho) (ReactiveFoam.C:727-728, in
+// FP64) and the step-start seeds.  A HEM batch's (energy non-null): species
+// masses q[c ns + k] and the given internal energies.
+struct FlashCells {
+    const double* q;
+    size_t stride;
+    const double* energy;
+    const ThermoOut* seeds;
+    const double* gate;   // the step's dt: nothing is flashed unless positive (null: always)
+    const uint32_t* rep;  // exact reuse: only cells that represent themselves (null: all)
+    __device__ inline bool flashed(uint32_t c) const { return !(gate && !(*gate > 0)) && !(rep && rep[c] != c); }
+    template <int NS, class F>
+    __device__ inline void load(F& f, uint32_t c) const {
+        using R = decltype(f.energy);
+        if (energy) {
+            for (int k = 0; k < NS; ++k) f.q[k] = R(q[size_t(c) * NS + k]);
+            f.energy = R(energy[c]);
+        } else {
+            double rho = 0;
+            for (int k = 0; k < NS; ++k) {
+                const double mass = q[size_t(k) * stride + c];
+                f.q[k] = R(mass);
+                rho += mass;
+            }
+            const double m0 = q[size_t(NS) * stride + c], m1 = q[size_t(NS + 1) * stride + c];
+            const double m2 = q[size_t(NS + 2) * stride + c], E = q[size_t(NS + 3) * stride + c];
+            f.energy = R(E - .5 * (m0 * m0 + m1 * m1 + m2 * m2) / rho);
+        }
+        const ThermoOut& g = seeds[c];
+        f.guessP = R(g.p);
+        f.guessT = R(g.T);
+        f.guessLiquid = R(g.liquidMass[0]);
     }
-    const double m0 = q[size_t(ns) * stride + c], m1 = q[size_t(ns + 1) * stride + c];
-    const double m2 = q[size_t(ns + 2) * stride + c], E = q[size_t(ns + 3) * stride + c];
-    f.energy = R(E - .5 * (m0 * m0 + m1 * m1 + m2 * m2) / rho);
-    f.guessP = R(g.p);
-    f.guessT = R(g.T);
-    f.guessLiquid = R(g.liquidMass[0]);
+    // Inputs a single-precision search takes up, with some of the condensable.
+    template <int NS>
+    __device__ inline bool valid(uint32_t c, int condensable) const;
+};
+template <int NS, class R = double>
+struct FlashInput {
+    R q[NS], energy, guessP, guessT, guessLiquid;
+};
+template <int NS>
+__device__ inline bool FlashCells::valid(uint32_t c, int condensable) const {
+    FlashInput<NS, float> f;
+    load<NS>(f, c);
+    float rho = 0;
+    bool ok = fin(f.energy);
+    for (int k = 0; k < NS; ++k) {
+        rho += f.q[k];
+        ok = ok && fin(f.q[k]) && f.q[k] >= 0;
+    }
+    return ok && rho > 0 && f.q[condensable] > 0;
 }
-
-// Loads cell c of a HEM batch into a flash: species masses q[c * NS + k], the
-// given internal energy and the seed.
-template <int NS, class F>
-__device__ inline void loadHemCell(F& f, const double* __restrict__ q, const double* __restrict__ energy,
-                                   const ThermoOut& g, uint32_t c) {
-    using R = decltype(f.energy);
-    for (int k = 0; k < NS; ++k) f.q[k] = R(q[size_t(c) * NS + k]);
-    f.energy = R(energy[c]);
-    f.guessP = R(g.p);
-    f.guessT = R(g.T);
-    f.guessLiquid = R(g.liquidMass[0]);
-}
+// Cells of a launch: `count` of them, or as many as *counted says.
+struct CellList {
+    const uint32_t* cells;
+    uint32_t count;
+    const unsigned* counted;
+    __device__ inline uint32_t size() const { return counted ? *counted : count; }
+};
 
 // Commits a flash result, or keeps the step-start state of a failed cell
 // (the reference commits nothing for it); p, c_frozen and rho go to the SoA
@@ -124,17 +153,46 @@ __device__ inline void countFlash(uint32_t failed, uint32_t phases, unsigned lon
     }
 }
 
-// Single-precision candidate search of the mixed flash (search.hip): one
-// launch over the cells in `order` in workgroups of `block` lanes (64, 128 or
-// 256), candidate sets and FP32 costs by cell; with rep (may be null), only
-// the cells that represent themselves (rep[c] == c) are searched.
-void launchSearch(int ns, int nl, const void* model, const double* q, size_t stride, const ThermoOut* seeds,
-                  const uint32_t* order, uint32_t count, const double* dtDev, CandidateSet* sets, uint16_t* cost,
-                  unsigned long long* phases, hipStream_t stream, unsigned block, const uint32_t* rep);
-// The same search over a HEM batch (loadHemCell's layout), 64-lane workgroups.
-void launchHemSearch(int ns, int nl, const void* model, const double* q, const double* energy,
-                     const ThermoOut* guess, const uint32_t* order, uint32_t count, CandidateSet* sets,
-                     unsigned long long* phases, hipStream_t stream);
+// ---- candidates of the mixed flash (search.hip) ---------------------------
+// One start's outcome: the point, kStart* bits and the evaluations above them.
+struct StartRecord {
+    float x[3];
+    uint32_t bits;
+};
+// Scratch of the search: kStarts records per listed cell (record s of list
+// position i at s stride + i) and the cells to restart.
+struct SearchScratch {
+    StartRecord* records;
+    uint32_t* restarts;
+    unsigned* restartCount;
+};
+// Saturated liquid and vapour at evenly spaced temperatures: specific volumes
+// and energies, ln p.  Interpolated between 2,048 rows over N2O's 161 K they
+// lie within 1e-6 of the curve except next to the critical point, inside the
+// refinement's one or two Newton steps.
+constexpr int kSaturationRows = 2048;
+struct SaturationRow {
+    double vl, vv, el, ev, lnp;
+};
+struct SaturationTable {
+    int count, pad;
+    double T0, dT;
+    SaturationRow row[kSaturationRows];
+};
+// The table of a one-species model with its liquid.
+void launchSaturation(const void* model, SaturationTable* table, hipStream_t stream);
+// The directed search of every cell in `order`: sets of one candidate or none, flagged kDirect.
+void launchDirect(const void* model, const SaturationTable* table, const FlashCells& cells, const uint32_t* order,
+                  uint32_t count, CandidateSet* sets, uint16_t* cost, unsigned long long* phases, hipStream_t stream);
+// Single-precision search, one cell per lane in workgroups of `block` lanes
+// (64, 128 or 256); candidate sets and evaluation counts by cell.
+void launchSearch(int ns, int nl, const void* model, const FlashCells& cells, const uint32_t* order, uint32_t count,
+                  CandidateSet* sets, uint16_t* cost, unsigned long long* phases, hipStream_t stream, unsigned block);
+// The same search, one start per lane, for models without stable-gas pruning;
+// stride: the list's largest length.  *scratch.restartCount is zero on entry.
+void launchSearchStarts(int ns, int nl, const void* model, const FlashCells& cells, const CellList& list, size_t stride,
+                        const SearchScratch& scratch, CandidateSet* sets, uint16_t* cost,
+                        unsigned long long* phases, hipStream_t stream);
 
 }  // namespace ramd
 #endif

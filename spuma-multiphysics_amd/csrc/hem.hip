@@ -136,35 +136,37 @@ __global__ __launch_bounds__(64, RAMD_FLASH_MIN_WAVES) void hemFlashKernel(const
     }
 }
 
-// Mixed arithmetic, second half (after hemSearchKernel): FP64 refinement,
-// stability and selection of each cell's FP32 candidates; cells the
-// refinement defers (a full FP64 search or FP64 restarts) go to the queue.
+// Mixed arithmetic, second half: FP64 refinement, stability and selection of
+// the listed cells' candidates; deferred cells go to the queue, or, where the
+// candidates came from the saturation table, to the list of cells to search.
 template <int NS, int NL>
 __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineKernel(const HemModel<NS>* __restrict__ globalModel,
-                                                     const double* __restrict__ q, const double* __restrict__ energy,
-                                                     const ThermoOut* __restrict__ guess,
-                                                     const uint32_t* __restrict__ order, uint32_t count,
+                                                     FlashCells cells, CellList list,
                                                      const CandidateSet* __restrict__ sets,
                                                      HemOutputDev* __restrict__ out,
                                                      unsigned long long* __restrict__ totals,
-                                                     uint32_t* __restrict__ queue, unsigned* __restrict__ queueCount) {
+                                                     uint32_t* __restrict__ queue, unsigned* __restrict__ queueCount,
+                                                     uint32_t* __restrict__ search,
+                                                     unsigned* __restrict__ searchCount) {
+    const uint32_t count = list.size();
+    if (blockIdx.x * 64u >= count) return;  // uniform per workgroup
     const HemModel<NS>& model = workgroupModel(globalModel);
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     Counts n = {0, 0, 0, 0, 0, 0, 0};
     uint32_t succeeded = 0;
-    if (i < count) {
-        const uint32_t c = order[i];
+    for (uint32_t i = blockIdx.x * 64u + threadIdx.x; i < count; i += gridDim.x * 64u) {
+        const uint32_t c = list.cells[i];
         Flash<NS, NL, double, true, false, false, kModelLds> f(model, n);
-        loadHemCell<NS>(f, q, energy, guess[c], c);
+        cells.load<NS>(f, c);
         EvalT<double, true> result;
         zeroEval(result);
         bool deferred = false;
         const bool ok = f.refine(sets[c], result, &deferred);
         if (deferred) {
-            queue[atomicAdd(queueCount, 1u)] = c;
+            if (sets[c].flags & kDirect) search[atomicAdd(searchCount, 1u)] = c;
+            else queue[atomicAdd(queueCount, 1u)] = c;
         } else {
             storeHemCell(ok, result, out[c]);
-            succeeded = ok ? 1u : 0u;
+            succeeded += ok ? 1u : 0u;
         }
     }
     addTotals(n, succeeded, totals);
@@ -176,13 +178,12 @@ __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineKernel(con
 // short, one cell per lane for a long queue (RAMD_WAVE_QUEUE_CELLS; the count
 // is read on the device).
 template <int NS, int NL, bool WAVE>
-__device__ inline void hemRefineQueued(const HemModel<NS>& model, const double* __restrict__ q,
-                                       const double* __restrict__ energy, const ThermoOut* __restrict__ guess,
-                                       uint32_t c, const CandidateSet& set, bool lead,
-                                       HemOutputDev* __restrict__ out, unsigned long long* __restrict__ totals) {
+__device__ inline void hemRefineQueued(const HemModel<NS>& model, const FlashCells& cells, uint32_t c,
+                                       const CandidateSet& set, bool lead, HemOutputDev* __restrict__ out,
+                                       unsigned long long* __restrict__ totals) {
     Counts n = {0, 0, 0, 0, 0, 0, 0};
     Flash<NS, NL, double, true, false, false, kModelLds, WAVE> f(model, n);
-    loadHemCell<NS>(f, q, energy, guess[c], c);
+    cells.load<NS>(f, c);
     EvalT<double, true> result;
     zeroEval(result);
     const bool ok = f.refine(set, result);
@@ -192,22 +193,21 @@ __device__ inline void hemRefineQueued(const HemModel<NS>& model, const double* 
 }
 template <int NS, int NL>
 __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineQueueKernel(
-    const HemModel<NS>* __restrict__ globalModel, const double* __restrict__ q, const double* __restrict__ energy,
-    const ThermoOut* __restrict__ guess, const uint32_t* __restrict__ queue, const unsigned* __restrict__ queueCount,
-    const CandidateSet* __restrict__ sets, HemOutputDev* __restrict__ out, unsigned long long* __restrict__ totals) {
+    const HemModel<NS>* __restrict__ globalModel, FlashCells cells, const uint32_t* __restrict__ queue,
+    const unsigned* __restrict__ queueCount, const CandidateSet* __restrict__ sets, HemOutputDev* __restrict__ out,
+    unsigned long long* __restrict__ totals) {
     const unsigned count = *queueCount;
     const bool perWave = count <= RAMD_WAVE_QUEUE_CELLS;  // uniform
     if (blockIdx.x * (perWave ? 1u : 64u) >= count) return;  // uniform per workgroup
     const HemModel<NS>& model = workgroupModel(globalModel);
     if (perWave) {
         for (unsigned i = blockIdx.x; i < count; i += gridDim.x)  // uniform per workgroup
-            hemRefineQueued<NS, NL, true>(model, q, energy, guess, queue[i], sets[queue[i]], threadIdx.x == 0, out,
-                                          totals);
+            hemRefineQueued<NS, NL, true>(model, cells, queue[i], sets[queue[i]], threadIdx.x == 0, out, totals);
     } else {
         for (unsigned base = blockIdx.x * 64u; base < count; base += gridDim.x * 64u) {  // uniform per workgroup
             const unsigned i = base + threadIdx.x;
             if (i < count) {
-                hemRefineQueued<NS, NL, false>(model, q, energy, guess, queue[i], sets[queue[i]], true, out, totals);
+                hemRefineQueued<NS, NL, false>(model, cells, queue[i], sets[queue[i]], true, out, totals);
             } else {
                 const Counts none = {0, 0, 0, 0, 0, 0, 0};
                 addTotals(none, 0u, totals);
@@ -216,8 +216,9 @@ __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineQueueKerne
     }
 }
 
-__global__ void clearCountKernel(unsigned* __restrict__ count) {
-    if (threadIdx.x == 0) *count = 0;
+// deferred cells, cells to search, cells to restart
+__global__ void clearCountsKernel(unsigned* __restrict__ counts) {
+    if (threadIdx.x < 3) counts[threadIdx.x] = 0;
 }
 
 // totals[k] = sum over b < blocks of partials[b * width + k], k < width: one
@@ -312,20 +313,40 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
                             size_t count, HemOutputDev* out, hipStream_t s) {
     if (!count) return;
     if (!sets) {
-        sets = static_cast<CandidateSet*>(allocate(capacity * sizeof(CandidateSet)));
         queue = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
-        queueCount = static_cast<unsigned*>(allocate(sizeof(unsigned)));
+        queueCount = static_cast<unsigned*>(allocate(3 * sizeof(unsigned)));
+        if (!prune) {
+            scratch.records = static_cast<StartRecord*>(allocate(kStarts * capacity * sizeof(StartRecord)));
+            scratch.restarts = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
+            scratch.restartCount = queueCount + 2;
+        }
+        if (pure()) {
+            searchList = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
+            saturation = static_cast<SaturationTable*>(allocate(sizeof(SaturationTable)));
+            launchSaturation(model, saturation, s);
+        }
+        sets = static_cast<CandidateSet*>(allocate(capacity * sizeof(CandidateSet)));
     }
     const unsigned blocks = unsigned((count + 63) / 64);
+    const FlashCells cells = {q, 0, e, g, nullptr, nullptr};
+    const CellList whole = {order, uint32_t(count), nullptr}, left = {searchList, 0, queueCount + 1};
     hipLaunchKernelGGL(zeroTotalsKernel, dim3(1), dim3(64), 0, s, totals, 10);
-    launchHemSearch(ns, nl, model, q, e, g, order, uint32_t(count), sets, totals + 8, s);
-    hipLaunchKernelGGL(clearCountKernel, dim3(1), dim3(64), 0, s, queueCount);
+    hipLaunchKernelGGL(clearCountsKernel, dim3(1), dim3(64), 0, s, queueCount);
+    if (saturation) launchDirect(model, saturation, cells, order, uint32_t(count), sets, nullptr, totals + 8, s);
+    else if (prune) launchSearch(ns, nl, model, cells, order, uint32_t(count), sets, nullptr, totals + 8, s, 64);
+    else launchSearchStarts(ns, nl, model, cells, whole, count, scratch, sets, nullptr, totals + 8, s);
 #define RAMD_HEM_MIXED(NS_, NL_)                                                                                  \
     hipLaunchKernelGGL((hemRefineKernel<NS_, NL_>), dim3(blocks), dim3(64), 0, s,                                   \
-                       static_cast<const HemModel<NS_>*>(model), q, e, g, order, uint32_t(count), sets, out, totals, \
-                       queue, queueCount);                                                                          \
+                       static_cast<const HemModel<NS_>*>(model), cells, whole, sets, out, totals, queue,          \
+                       queueCount, searchList, queueCount + 1);                                                   \
+    if (saturation) {                                                                                             \
+        launchSearchStarts(ns, nl, model, cells, left, count, scratch, sets, nullptr, totals + 8, s);             \
+        hipLaunchKernelGGL((hemRefineKernel<NS_, NL_>), dim3(std::min(2048u, blocks)), dim3(64), 0, s,              \
+                           static_cast<const HemModel<NS_>*>(model), cells, left, sets, out, totals, queue,       \
+                           queueCount, searchList, queueCount + 1);                                               \
+    }                                                                                                             \
     hipLaunchKernelGGL((hemRefineQueueKernel<NS_, NL_>), dim3(kQueueBlocks), dim3(64), 0, s,                        \
-                       static_cast<const HemModel<NS_>*>(model), q, e, g, queue, queueCount, sets, out, totals)
+                       static_cast<const HemModel<NS_>*>(model), cells, queue, queueCount, sets, out, totals)
     if (ns == 1 && nl == 0) { RAMD_HEM_MIXED(1, 0); }
     else if (ns == 1) { RAMD_HEM_MIXED(1, 1); }
     else if (nl == 0) { RAMD_HEM_MIXED(2, 0); }
@@ -363,6 +384,7 @@ HemHandle* createHem(const void* raw, size_t bytes, size_t capacity, bool hostPa
     h->nl = m.nl;
     h->analytic = m.analyticJacobian != 0;
     h->boundary = m.boundaryRecovery != 0;
+    h->prune = m.stableGasPrune != 0;
     h->arithmetic = defaultArithmetic();
     h->capacity = capacity;
     h->device = currentDevice();

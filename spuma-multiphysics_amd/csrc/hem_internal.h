@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <vector>
 #include "flash_device.h"
+#include "flash_step.h"
 
 namespace ramd {
 
@@ -27,6 +28,9 @@ struct HemHandle {
     int ns = 0, nl = 0, device = 0;
     bool analytic = false;  // the model's analytic-Jacobian mode (FP64 flash)
     bool boundary = false;  // the model's boundary search (boundaryRecovery = 1)
+    bool prune = false;     // the model's stable-gas pruning (stableGasPrune = 1)
+    // one species with its liquid: the mixed flash looks its candidates up in the saturation table
+    bool pure() const { return ns == 1 && nl == 1 && !prune; }
     int arithmetic = 0;     // equilibrium flash of host batches: REACTIVE_AMD_FLASH_FP64 or _MIXED
     size_t capacity = 0, deviceBytes = 0, modelBytes = 0;
     void* model = nullptr;  // HemModel<ns> in device memory
@@ -38,7 +42,10 @@ struct HemHandle {
     // evaluations and deferred cells
     CandidateSet* sets = nullptr;
     uint32_t* queue = nullptr;
-    unsigned* queueCount = nullptr;
+    unsigned* queueCount = nullptr;  // deferred cells, cells to search, cells to restart
+    SaturationTable* saturation = nullptr;
+    uint32_t* searchList = nullptr;
+    SearchScratch scratch = {};
     uint64_t lastSinglePhases = 0, lastQueued = 0;
     // host-path staging (allocated on the first host batch)
     bool hostReady = false;

@@ -1,14 +1,16 @@
 // SPDX-License-Identifier: GPL-3.0-or-later
-// Single-precision candidate search of the mixed flash.  This file alone is
-// compiled with -freciprocal-math -fapprox-func (build.sh): the FP32 search
-// only chooses and seeds candidates, every accepted result is recomputed by
-// the FP64 refinement, so it may use the hardware reciprocal and
-// transcendental approximations.  Non-finite values keep their IEEE meaning
-// (no finite-math assumption), so the search's NaN and range checks hold.
+// Candidates of the mixed flash: the single-precision search and, for a pure
+// fluid, the saturation table that directs it.  This file alone is
+// compiled with -freciprocal-math -fapprox-func (build.sh): it only chooses
+// and seeds candidates, every accepted result is recomputed by the FP64
+// refinement, so it may use the hardware reciprocal and transcendental
+// approximations.  Non-finite values keep their IEEE meaning (no finite-math
+// assumption), so the search's NaN and range checks hold.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include "flash_step.h"
 
-// Minimum waves per SIMD the register allocation of the search kernel targets
+// Minimum waves per SIMD the register allocation of the search kernels targets
 // (5: 96 VGPRs; at 160^3 3-4 % faster than 4, 6 and 8 slower: more stack).
 #ifndef RAMD_SEARCH_MIN_WAVES
 #define RAMD_SEARCH_MIN_WAVES 5
@@ -16,24 +18,20 @@
 
 namespace ramd {
 
-// Mixed precision, first half: the candidate search in FP32, recording the
-// converged candidates of every cell.
+// ---- the whole search of a cell on one lane: models with stable-gas
+// pruning, whose seeds run only where the gas solve says so.
 template <int NS, int NL>
-__global__ __launch_bounds__(256, RAMD_SEARCH_MIN_WAVES) void stepSearchKernel(const HemModel<NS>* __restrict__ globalModel,
-                                                       const double* __restrict__ q, size_t stride,
-                                                       const ThermoOut* __restrict__ seeds,
-                                                       const uint32_t* __restrict__ order, uint32_t count,
-                                                       const double* __restrict__ dtDev,
-                                                       CandidateSet* __restrict__ sets, uint16_t* __restrict__ cost,
-                                                       unsigned long long* __restrict__ phases,
-                                                       const uint32_t* __restrict__ rep) {
+__global__ __launch_bounds__(256, RAMD_SEARCH_MIN_WAVES) void searchKernel(
+    const HemModel<NS>* __restrict__ globalModel, FlashCells cells, const uint32_t* __restrict__ order,
+    uint32_t count, CandidateSet* __restrict__ sets, uint16_t* __restrict__ cost,
+    unsigned long long* __restrict__ phases) {
     const HemModel<NS>& model = workgroupModel(globalModel);
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    Counts n = {0, 0, 0, 0, 0, 0};
-    if (i < count && *dtDev > 0 && !(rep && rep[order[i]] != order[i])) {
+    Counts n = {0, 0, 0, 0, 0, 0, 0};
+    if (i < count && cells.flashed(order[i])) {
         const uint32_t c = order[i];
         Flash<NS, NL, float, true, false, false, kModelLds> f(model, n);
-        loadCell(f, q, stride, seeds[c], c, NS);
+        cells.load<NS>(f, c);
         CandidateSet set;
         f.searchRecord(set);
         sets[c] = set;
@@ -43,61 +41,381 @@ __global__ __launch_bounds__(256, RAMD_SEARCH_MIN_WAVES) void stepSearchKernel(c
     if ((threadIdx.x & 63) == 0) atomicAdd(phases, (unsigned long long)sum);
 }
 
-// The same search for a HEM batch (reactive_gpu_hem_run_v1 with the mixed
-// arithmetic): species masses q[c * NS + k], internal energy energy[c] and the
-// seed guess[c] by cell, cells in `order`.
+// ---- the search, one start per lane.  A cell's all-gas, all-liquid and
+// five seed solves are independent, so they run side by side: wave (block, s)
+// runs start s of 64 cells, and a wave is as long as the longest of its 64
+// solves rather than the longest sum of seven (and of the twenty restarts,
+// which now run only for the cells that need them, see below).  Bound by the
+// latency of the few solves that crawl, not by arithmetic: a 12^3 box's
+// search took 18 ms sequentially.
 template <int NS, int NL>
-__global__ __launch_bounds__(256, RAMD_SEARCH_MIN_WAVES) void hemSearchKernel(const HemModel<NS>* __restrict__ globalModel,
-                                                      const double* __restrict__ q,
-                                                      const double* __restrict__ energy,
-                                                      const ThermoOut* __restrict__ guess,
-                                                      const uint32_t* __restrict__ order, uint32_t count,
-                                                      CandidateSet* __restrict__ sets,
-                                                      unsigned long long* __restrict__ phases) {
+__global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchStartsKernel(
+    const HemModel<NS>* __restrict__ globalModel, FlashCells cells, CellList list, size_t stride,
+    StartRecord* __restrict__ records, unsigned long long* __restrict__ phases) {
+    const uint32_t count = list.size();
+    if (blockIdx.x * 64u >= count) return;  // uniform per workgroup
     const HemModel<NS>& model = workgroupModel(globalModel);
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    Counts n = {0, 0, 0, 0, 0, 0, 0};
-    if (i < count) {
-        const uint32_t c = order[i];
-        Flash<NS, NL, float, true, false, false, kModelLds> f(model, n);
-        loadHemCell<NS>(f, q, energy, guess[c], c);
-        CandidateSet set;
-        f.searchRecord(set);
-        sets[c] = set;
+    uint32_t total = 0;
+    for (uint32_t base = blockIdx.x * 64u; base < count; base += gridDim.x * 64u) {
+        const uint32_t i = base + threadIdx.x;
+        if (i < count && cells.flashed(list.cells[i])) {
+            Counts n = {0, 0, 0, 0, 0, 0, 0};
+            Flash<NS, NL, float, true, false, false, kModelLds> f(model, n);
+            cells.load<NS>(f, list.cells[i]);
+            StartRecord r;
+            r.bits = f.searchStart(int(blockIdx.y), r.x);
+            r.bits |= n.phases << 2;
+            records[size_t(blockIdx.y) * stride + i] = r;
+            total += n.phases;
+        }
     }
-    const uint32_t sum = waveSum(n.phases);
-    if ((threadIdx.x & 63) == 0) atomicAdd(phases, (unsigned long long)sum);
+    const uint32_t sum = waveSum(total);
+    if (threadIdx.x == 0) atomicAdd(phases, (unsigned long long)sum);
 }
 
-void launchHemSearch(int ns, int nl, const void* model, const double* q, const double* energy,
-                     const ThermoOut* guess, const uint32_t* order, uint32_t count, CandidateSet* sets,
-                     unsigned long long* phases, hipStream_t stream) {
-    const unsigned blocks = unsigned((size_t(count) + 63) / 64);
-#define RAMD_HEM_SEARCH(NS_, NL_)                                                                                 \
-    hipLaunchKernelGGL((hemSearchKernel<NS_, NL_>), dim3(blocks), dim3(64), 0, stream,                             \
-                       static_cast<const HemModel<NS_>*>(model), q, energy, guess, order, count, sets, phases)
-    if (ns == 1 && nl == 0) { RAMD_HEM_SEARCH(1, 0); }
-    else if (ns == 1) { RAMD_HEM_SEARCH(1, 1); }
-    else if (nl == 0) { RAMD_HEM_SEARCH(2, 0); }
-    else { RAMD_HEM_SEARCH(2, 1); }
-#undef RAMD_HEM_SEARCH
+// The seven records of a cell in search order into its candidate set; cells
+// without a stable one go to the restart list.
+template <int NS>
+__global__ __launch_bounds__(256) void searchMergeKernel(const HemModel<NS>* __restrict__ model, FlashCells cells,
+                                                         CellList list, size_t stride,
+                                                         const StartRecord* __restrict__ records,
+                                                         CandidateSet* __restrict__ sets,
+                                                         uint16_t* __restrict__ cost,
+                                                         uint32_t* __restrict__ restarts,
+                                                         unsigned* __restrict__ restartCount) {
+    const uint32_t count = list.size();
+    const double top = lo(model->Tmax, model->liquidTc * (1 - 1e-10)), bottom = hi(model->Tmin, model->liquidTmin);
+    const bool restartable = model->nl && top > bottom;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < count; i += gridDim.x * 256u) {
+        const uint32_t c = list.cells[i];
+        if (!cells.flashed(c)) continue;
+        CandidateSet set;
+        set.count = set.flags = 0;
+        bool have = false;
+        uint32_t evaluations = 0;
+        for (int s = 0; s < kStarts; ++s) {
+            const StartRecord r = records[size_t(s) * stride + i];
+            evaluations += r.bits >> 2;
+            have = have || (r.bits & kStartStable);
+            if (r.bits & kStartFound)
+                noteCandidate(set, s == 0 ? kGasCandidate : s == 1 ? kLiquidCandidate : kSeedCandidate,
+                              int16_t(s < 2 ? 0 : s - 2), r.x, s >= 2);
+        }
+        // (a cell whose inputs no solve accepts has no candidates and no restarts)
+        if (!have && restartable && cells.valid<NS>(c, model->condensable)) {
+            set.flags |= kRestartsSearched;
+            restarts[atomicAdd(restartCount, 1u)] = c;
+        }
+        sets[c] = set;
+        if (cost) cost[c] = uint16_t(evaluations < 65535u ? evaluations : 65535u);
+    }
+}
+
+// The twenty restarts of the listed cells, three cells per wave and one
+// restart per lane, appended to the cells' sets in search order.
+template <int NS, int NL>
+__global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchRestartsKernel(
+    const HemModel<NS>* __restrict__ globalModel, FlashCells cells, CellList list, CandidateSet* __restrict__ sets,
+    uint16_t* __restrict__ cost, unsigned long long* __restrict__ phases) {
+    const uint32_t count = list.size();
+    if (blockIdx.x * 3u >= count) return;  // uniform per workgroup
+    const HemModel<NS>& model = workgroupModel(globalModel);
+    __shared__ StartRecord found[64];
+    uint32_t total = 0;
+    const uint32_t cell = threadIdx.x / kRestarts, s = threadIdx.x % kRestarts;
+    for (uint32_t base = blockIdx.x * 3u; base < count; base += gridDim.x * 3u) {  // uniform per workgroup
+        const uint32_t i = base + cell;
+        const bool active = cell < 3 && i < count;
+        if (active) {
+            Counts n = {0, 0, 0, 0, 0, 0, 0};
+            Flash<NS, NL, float, true, false, false, kModelLds> f(model, n);
+            cells.load<NS>(f, list.cells[i]);
+            StartRecord r;
+            r.bits = f.searchStart(kStarts + int(s), r.x);
+            r.bits |= n.phases << 2;
+            found[threadIdx.x] = r;
+            total += n.phases;
+        }
+        __syncthreads();
+        if (active && s == 0) {
+            const uint32_t c = list.cells[i];
+            CandidateSet set = sets[c];
+            uint32_t evaluations = 0;
+            for (int k = 0; k < kRestarts; ++k) {
+                const StartRecord r = found[threadIdx.x + k];
+                evaluations += r.bits >> 2;
+                if (r.bits & kStartFound) noteCandidate(set, kRestartCandidate, int16_t(k), r.x, true);
+            }
+            sets[c] = set;
+            if (cost) {
+                evaluations += cost[c];
+                cost[c] = uint16_t(evaluations < 65535u ? evaluations : 65535u);
+            }
+        }
+        __syncthreads();
+    }
+    const uint32_t sum = waveSum(total);
+    if (threadIdx.x == 0) atomicAdd(phases, (unsigned long long)sum);
+}
+
+// ---- a pure fluid's search, directed by its saturation curve --------------
+//
+// At a given (rho, e) a pure fluid has one equilibrium: two phases where some
+// saturation temperature T has v_l(T) < 1/rho < v_v(T) and the lever rule's
+// energy equal to e, one phase elsewhere.  Which it is, and where, is looked
+// up: T by bisection in a table of the saturation curve, or, outside the
+// dome, by Newton's method on e(T) at fixed rho.  Of the search's seven
+// solves only one can then lead there; it alone is run (for two phases, from
+// the seed nearest the known liquid fraction), since the reference accepts a
+// cell only where one of its solves arrives.  The refinement then confirms
+// the point with the FP64 solver and stability test, as it does a searched
+// candidate.  A cell whose solve does not arrive or whose point is not
+// confirmed (and every cell the table says too little about: colder than the
+// table, near the critical point or the dome's edge, outside the model's
+// range) runs the whole search.
+__global__ void saturationInitKernel(SaturationTable* __restrict__ table) {
+    if (threadIdx.x == 0) table->count = kSaturationRows;
+}
+// One node per thread: ln p by Newton on mu_l = mu_v (d(mu / RT) / d ln p = z),
+// kept between the pressures known to be too low (no liquid) and too high
+// (no vapour).  The first node without a solution ends the table.
+template <int NS>
+__global__ __launch_bounds__(64) void saturationKernel(const HemModel<NS>* __restrict__ globalModel,
+                                                       SaturationTable* __restrict__ table) {
+    const HemModel<NS>& model = workgroupModel(globalModel);
+    const int i = int(blockIdx.x * 64 + threadIdx.x);
+    if (i >= kSaturationRows) return;
+    const double T0 = hi(model.Tmin, model.liquidTmin);
+    const double dT = (lo(model.Tmax, model.liquidTc) - T0) / kSaturationRows, T = T0 + i * dT;
+    if (i == 0) {
+        table->T0 = T0;
+        table->dT = dT;
+    }
+    Counts n = {0, 0, 0, 0, 0, 0, 0};
+    Flash<NS, 1, double, false, false, false, kModelLds> f(model, n);
+    const double Tc = model.liquid.Tc[0], pc = kOmegaB * kR * Tc / model.liquid.b[0];
+    double low = ::log(model.pmin) - 20, high = ::log(pc);
+    double x = clamp(high + 5.373 * (1 + (model.liquid.kappa[0] - .37464) / 1.54226) * (1 - Tc / T), low, high);
+    bool found = false;
+    PRState g, l;
+    for (int it = 0; it < 60 && !found; ++it) {
+        const double p = ::exp(x);
+        const double Y[NS] = {1};
+        double muG[NS], muL[1];
+        if (f.gasTP(T, p, Y, g, muG) != kOk) high = x;
+        else if (f.liquidTP(T, p, l, muL) != kOk) low = x;
+        else {
+            const double RT = kR * T, difference = (muL[0] - muG[0]) / RT, slope = p * (l.V - g.V) / RT;
+            if (difference > 0) low = x;
+            else high = x;
+            const double next = x - difference / slope;
+            found = ::fabs(next - x) < 1e-11;
+            x = next > low && next < high ? next : .5 * (low + high);
+            continue;
+        }
+        x = .5 * (low + high);
+    }
+    if (!found || !(g.rho < l.rho)) {
+        atomicMin(&table->count, i);
+        return;
+    }
+    table->row[i] = {1 / l.rho, 1 / g.rho, l.e, g.e, x};
+}
+
+// Newton's method on e(T) = u at fixed density (single precision).
+template <int NS>
+__device__ inline bool temperatureAt(const Table<NS>& t, float V, float u, float low, float high, float& T,
+                                     uint32_t& evaluations) {
+    const float b = float(t.b[0]), W = float(t.W[0]), Rg = float(kR), sq2 = float(kSqrt2);
+    const float L = m_log((V + (1 + sq2) * b) / (V + (1 - sq2) * b)) / (2 * sq2 * b);
+    const float one[1] = {1};
+    for (int it = 0; it < 20; ++it) {
+        MixT<float> mx;
+        float cpR, hRT, sR;
+        ++evaluations;
+        if (mixing(t, T, one, mx) != kOk) return false;
+        nasa(region(t, 0, T), T, cpR, hRT, sR);
+        const float F = Rg * T * (hRT - 1) + L * (T * mx.da - mx.aa) - u * W;
+        const float cv = Rg * (cpR - 1) + L * T * mx.d2a;
+        const float step = F / cv;
+        if (!(cv > 0) || !fin(step)) return false;
+        const float next = clamp(T - step, low, high);
+        const bool done = ab(next - T) <= 3e-6f * T;
+        T = next;
+        if (done) return T > low && T < high;
+    }
+    return false;
+}
+
+// Where a saturated state's energy passes the cell's, or the dome ends: both
+// are crossed once as T rises at fixed v.
+__device__ inline bool saturationPast(const SaturationRow& r, double v, double u, bool& outside) {
+    outside = v <= r.vl || v >= r.vv;
+    const double x = (v - r.vl) / (r.vv - r.vl);
+    return outside || r.el + x * (r.ev - r.el) > u;
+}
+// Liquid fractions (and energies, in units of the vaporisation energy) this
+// close to the dome's edge are left to the search, whose candidates on both
+// sides of the edge the refinement compares.
+constexpr double kDomeEdge = 1e-3;
+
+// The cell's equilibrium point into its set (count 0: not known).
+template <int NS>
+__device__ inline void directCandidate(const HemModel<NS>& m, const SaturationTable& table, double rho, double energy,
+                                        double guessT, CandidateSet& set, uint32_t& evaluations) {
+    set.count = 0;
+    set.flags = kDirect;
+    if (!fin(energy) || !(rho > 0) || !fin(rho)) return;
+    const double v = 1 / rho, u = energy / rho;
+    const int rows = table.count;
+    if (rows < 2) return;
+    int low = -1, high = rows;
+    bool outside = false, highOutside = false;
+    while (high - low > 1) {
+        const int mid = (low + high) >> 1;
+        if (saturationPast(table.row[mid], v, u, outside)) { high = mid; highOutside = outside; }
+        else low = mid;
+    }
+    if (high == rows) return;             // near the critical point, or above it
+    if (low < 0 && !highOutside) return;  // colder than the table
+    if (!highOutside) {  // two phases, between the rows low and low + 1
+        const SaturationRow a = table.row[low], b = table.row[high];
+        const double ea = a.el + (v - a.vl) / (a.vv - a.vl) * (a.ev - a.el);
+        const double eb = b.el + (v - b.vl) / (b.vv - b.vl) * (b.ev - b.el);
+        const double w = clamp((u - ea) / (eb - ea), 0., 1.);
+        const double vl = a.vl + w * (b.vl - a.vl), vv = a.vv * ::exp(w * ::log(b.vv / a.vv));
+        const double liquid = (vv - v) / (vv - vl);
+        if (!(liquid > kDomeEdge && liquid < 1 - kDomeEdge)) return;
+        const float at[3] = {float(a.lnp + w * (b.lnp - a.lnp)), float(::log(table.T0 + (low + w) * table.dT)),
+                             float(liquid)};
+        noteCandidate(set, kSeedCandidate, 0, at, false);
+        return;
+    }
+    if (low >= 0) {
+        // the dome ends between the rows: one phase where its edge lies well below the cell's energy
+        const SaturationRow& r = table.row[high];
+        const bool vapour = v >= r.vv;
+        if (u < (vapour ? r.ev : r.el) + kDomeEdge * (r.ev - r.el)) return;
+    }
+    const SaturationRow& r = table.row[high];
+    const bool vapour = v >= r.vv;
+    float T = float(clamp(guessT, m.Tmin, m.Tmax));
+    const double V = v * m.gas.W[0];
+    if (!(V > m.gas.b[0]) || !temperatureAt(m.gas, float(V), float(u), float(m.Tmin), float(m.Tmax), T, evaluations))
+        return;
+    const double one[1] = {1};
+    Mix mx;
+    if (mixing(m.gas, double(T), one, mx) != kOk) return;
+    const double p = kR * T / (V - mx.b) - mx.aa / (V * V + 2 * V * mx.b - mx.b * mx.b);
+    if (!(p >= m.pmin && p <= m.pmax)) return;
+    const float at[3] = {float(::log(p)), m_log(T), 0.f};
+    noteCandidate(set, vapour || T >= float(m.liquidTc) ? kGasCandidate : kLiquidCandidate, 0, at, false);
+}
+
+template <int NS>
+__global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void directKernel(
+    const HemModel<NS>* __restrict__ globalModel, const SaturationTable* __restrict__ table, FlashCells cells,
+    const uint32_t* __restrict__ order, uint32_t count, CandidateSet* __restrict__ sets, uint16_t* __restrict__ cost,
+    unsigned long long* __restrict__ phases) {
+    const HemModel<NS>& model = workgroupModel(globalModel);
+    const uint32_t i = blockIdx.x * 64u + threadIdx.x;
+    const bool active = i < count && cells.flashed(order[i]);
+    const uint32_t c = active ? order[i] : order[0];
+    Counts n = {0, 0, 0, 0, 0, 0, 0};
+    CandidateSet set;
+    set.count = 0;
+    FlashInput<NS> at;
+    cells.load<NS>(at, c);
+    if (active) directCandidate<NS>(model, *table, at.q[0], at.energy, at.guessT, set, n.phases);
+    int start = -1;
+    if (set.count) {
+        start = set.c[0].kind == kGasCandidate ? 0 : 1;
+        if (set.c[0].kind == kSeedCandidate) {
+            const float seeds[5] = {clamp(float(at.guessLiquid / at.q[0]), 0.f, 1.f), .5f, .95f, .1f, .9999f};
+            int nearest = 0;
+            float least = 2;
+            for (int j = 0; j < 5; ++j) {
+                const float d = ab(seeds[j] - set.c[0].x[2]);
+                if (d < least) { least = d; nearest = j; }
+            }
+            start = 2 + nearest;
+        }
+    }
+    Flash<NS, 1, float, true, false, false, kModelLds> f(model, n);
+    cells.load<NS>(f, c);
+    // one start at a time, for the lanes that take it (searchStart's condition)
+    uint32_t bits = 0;
+    for (unsigned long long pending = __ballot(start >= 0); pending; pending &= ~__ballot(bits & 4u)) {
+        const int s = __shfl(start, __ffsll(pending) - 1, 64);
+        if (start == s) {
+            float x[3];
+            bits = f.searchStart(s, x) | 4u;
+        }
+    }
+    if (!(bits & kStartFound)) set.count = 0;
+    if (active) {
+        sets[c] = set;
+        if (cost) cost[c] = uint16_t(n.phases < 65535u ? n.phases : 65535u);
+    }
+    const uint32_t sum = waveSum(active ? n.phases : 0u);
+    if (threadIdx.x == 0) atomicAdd(phases, (unsigned long long)sum);
+}
+
+// ---- launches --------------------------------------------------------------
+#define RAMD_SPECIES(LAUNCH)                         \
+    if (ns == 1 && nl == 0) { LAUNCH(1, 0); }        \
+    else if (ns == 1) { LAUNCH(1, 1); }              \
+    else if (nl == 0) { LAUNCH(2, 0); }              \
+    else { LAUNCH(2, 1); }
+
+void launchSaturation(const void* model, SaturationTable* table, hipStream_t stream) {
+    hipLaunchKernelGGL(saturationInitKernel, dim3(1), dim3(64), 0, stream, table);
+    hipLaunchKernelGGL((saturationKernel<1>), dim3((kSaturationRows + 63) / 64), dim3(64), 0, stream,
+                       static_cast<const HemModel<1>*>(model), table);
     RAMD_HIP(hipGetLastError());
 }
 
-void launchSearch(int ns, int nl, const void* model, const double* q, size_t stride, const ThermoOut* seeds,
-                  const uint32_t* order, uint32_t count, const double* dtDev, CandidateSet* sets, uint16_t* cost,
-                  unsigned long long* phases, hipStream_t stream, unsigned block, const uint32_t* rep) {
+void launchDirect(const void* model, const SaturationTable* table, const FlashCells& cells, const uint32_t* order,
+                  uint32_t count, CandidateSet* sets, uint16_t* cost, unsigned long long* phases, hipStream_t stream) {
+    hipLaunchKernelGGL((directKernel<1>), dim3(unsigned((size_t(count) + 63) / 64)), dim3(64), 0, stream,
+                       static_cast<const HemModel<1>*>(model), table, cells, order, count, sets, cost, phases);
+    RAMD_HIP(hipGetLastError());
+}
+
+void launchSearch(int ns, int nl, const void* model, const FlashCells& cells, const uint32_t* order, uint32_t count,
+                  CandidateSet* sets, uint16_t* cost, unsigned long long* phases, hipStream_t stream, unsigned block) {
     const unsigned blocks = unsigned((size_t(count) + block - 1) / block);
-#define RAMD_SEARCH(NS_, NL_)                                                                                     \
-    hipLaunchKernelGGL((stepSearchKernel<NS_, NL_>), dim3(blocks), dim3(block), 0, stream,                         \
-                       static_cast<const HemModel<NS_>*>(model), q, stride, seeds, order, count, dtDev, sets, cost, \
-                       phases, rep)
-    if (ns == 1 && nl == 0) { RAMD_SEARCH(1, 0); }
-    else if (ns == 1) { RAMD_SEARCH(1, 1); }
-    else if (nl == 0) { RAMD_SEARCH(2, 0); }
-    else { RAMD_SEARCH(2, 1); }
+#define RAMD_SEARCH(NS_, NL_)                                                                                \
+    hipLaunchKernelGGL((searchKernel<NS_, NL_>), dim3(blocks), dim3(block), 0, stream,                        \
+                       static_cast<const HemModel<NS_>*>(model), cells, order, count, sets, cost, phases)
+    RAMD_SPECIES(RAMD_SEARCH)
 #undef RAMD_SEARCH
     RAMD_HIP(hipGetLastError());
 }
+
+// Waves of a launch over a list counted on the device: enough to fill the
+// chip at the search's five waves per SIMD; a longer list takes more rounds.
+constexpr unsigned kListWaves = 5120;
+
+void launchSearchStarts(int ns, int nl, const void* model, const FlashCells& cells, const CellList& list, size_t stride,
+                        const SearchScratch& scratch, CandidateSet* sets, uint16_t* cost,
+                        unsigned long long* phases, hipStream_t stream) {
+    const unsigned waves = unsigned((stride + 63) / 64);
+    const unsigned blocks = list.counted ? std::min(waves, kListWaves / kStarts) : waves;
+#define RAMD_STARTS(NS_, NL_)                                                                                \
+    hipLaunchKernelGGL((searchStartsKernel<NS_, NL_>), dim3(blocks, kStarts), dim3(64), 0, stream,            \
+                       static_cast<const HemModel<NS_>*>(model), cells, list, stride, scratch.records, phases); \
+    hipLaunchKernelGGL((searchMergeKernel<NS_>), dim3(std::min(2048u, (waves + 3) / 4)), dim3(256), 0, stream, \
+                       static_cast<const HemModel<NS_>*>(model), cells, list, stride, scratch.records, sets, cost, \
+                       scratch.restarts, scratch.restartCount);                                              \
+    hipLaunchKernelGGL((searchRestartsKernel<NS_, NL_>),                                                      \
+                       dim3(std::min(kListWaves, unsigned((stride + 2) / 3))), dim3(64), 0, stream,           \
+                       static_cast<const HemModel<NS_>*>(model), cells,                                       \
+                       CellList{scratch.restarts, 0, scratch.restartCount}, sets, cost, phases)
+    RAMD_SPECIES(RAMD_STARTS)
+#undef RAMD_STARTS
+    RAMD_HIP(hipGetLastError());
+}
+#undef RAMD_SPECIES
 
 }  // namespace ramd

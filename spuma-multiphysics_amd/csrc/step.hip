@@ -36,33 +36,33 @@
 namespace ramd {
 
 // ---------------------------------------------------------------- kernels
+// Counts of the mixed flash's lists: deferred cells, cells to search, cells to restart.
+constexpr int kQueueCounts = 3;
+
 // Plain FP64 flash of the cells in `order`; RJ: the model's
 // analytic-Jacobian mode.
 template <int NS, int NL, bool RJ>
 __global__ __launch_bounds__(256, RAMD_FLASH_MIN_WAVES) void stepFlashKernel(const HemModel<NS>* __restrict__ globalModel,
-                                                      const double* __restrict__ q, size_t stride,
-                                                      const ThermoOut* __restrict__ seeds,
+                                                      FlashCells cells,
                                                       const uint32_t* __restrict__ order, uint32_t count,
-                                                      const double* __restrict__ dtDev, ThermoOut* __restrict__ out,
+                                                      ThermoOut* __restrict__ out,
                                                       double* __restrict__ pOut, double* __restrict__ cOut,
                                                       double* __restrict__ rOut, uint16_t* __restrict__ cost,
                                                       unsigned long long* __restrict__ counters,
-                                                      uint8_t* __restrict__ failMark,
-                                                      const uint32_t* __restrict__ rep) {
+                                                      uint8_t* __restrict__ failMark) {
     const HemModel<NS>& model = workgroupModel(globalModel);
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     Counts n = {0, 0, 0, 0, 0, 0};
     uint32_t failed = 0;
-    if (i < count && *dtDev > 0 && !(rep && rep[order[i]] != order[i])) {
+    if (i < count && cells.flashed(order[i])) {
         const uint32_t c = order[i];
-        const ThermoOut g = seeds[c];
         using F = Flash<NS, NL, double, false, RJ, false, kModelLds>;
         F f(model, n);
-        loadCell(f, q, stride, g, c, NS);
+        cells.load<NS>(f, c);
         typename F::E result;
         zeroEval(result);
         const bool ok = f.run(result);
-        storeCell(ok, result, g, c, out, pOut, cOut, rOut);
+        storeCell(ok, result, cells.seeds[c], c, out, pOut, cOut, rOut);
         if (!ok && failMark) failMark[c] = 1;
         failed = ok ? 0u : 1u;
         if (cost) cost[c] = uint16_t(n.phases < 65535u ? n.phases : 65535u);
@@ -70,61 +70,63 @@ __global__ __launch_bounds__(256, RAMD_FLASH_MIN_WAVES) void stepFlashKernel(con
     countFlash(failed, n.phases, counters);
 }
 
-// Mixed precision, second half: FP64 refinement, stability and selection.
+// Mixed precision, second half: FP64 refinement, stability and selection of
+// the listed cells' candidates.  Deferred cells go to the queue, or, where
+// the candidates came from the saturation table, to the list of cells to
+// search.  A list counted on the device is swept in rounds.
 template <int NS, int NL>
 __global__ __launch_bounds__(256, RAMD_REFINE_MIN_WAVES) void stepRefineKernel(const HemModel<NS>* __restrict__ globalModel,
-                                                       const double* __restrict__ q, size_t stride,
-                                                       const ThermoOut* __restrict__ seeds,
-                                                       const uint32_t* __restrict__ order, uint32_t count,
-                                                       const double* __restrict__ dtDev,
+                                                       FlashCells cells, CellList list,
                                                        const CandidateSet* __restrict__ sets,
                                                        ThermoOut* __restrict__ out, double* __restrict__ pOut,
                                                        double* __restrict__ cOut, double* __restrict__ rOut,
                                                        uint16_t* __restrict__ cost,
                                                        unsigned long long* __restrict__ counters,
                                                        uint32_t* __restrict__ queue, unsigned* __restrict__ queueCount,
-                                                       uint8_t* __restrict__ failMark,
-                                                       const uint32_t* __restrict__ rep) {
+                                                       uint32_t* __restrict__ search, unsigned* __restrict__ searchCount,
+                                                       uint8_t* __restrict__ failMark) {
+    const uint32_t count = list.size();
+    if (blockIdx.x * blockDim.x >= count) return;  // uniform per workgroup
     const HemModel<NS>& model = workgroupModel(globalModel);
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    Counts n = {0, 0, 0, 0, 0, 0};
-    uint32_t failed = 0;
-    if (i < count && *dtDev > 0 && !(rep && rep[order[i]] != order[i])) {
-        const uint32_t c = order[i];
-        const ThermoOut g = seeds[c];
+    uint32_t failed = 0, phases = 0;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
+        const uint32_t c = list.cells[i];
+        if (!cells.flashed(c)) continue;
+        Counts n = {0, 0, 0, 0, 0, 0, 0};
         Flash<NS, NL, double, true, false, false, kModelLds> f(model, n);
-        loadCell(f, q, stride, g, c, NS);
+        cells.load<NS>(f, c);
         EvalT<double, true> result;
         zeroEval(result);
         bool deferred = false;
         const bool ok = f.refine(sets[c], result, queue ? &deferred : nullptr);
         if (deferred) {
-            queue[atomicAdd(queueCount, 1u)] = c;
+            if (sets[c].flags & kDirect) search[atomicAdd(searchCount, 1u)] = c;
+            else queue[atomicAdd(queueCount, 1u)] = c;
         } else {
-            storeCell(ok, result, g, c, out, pOut, cOut, rOut);
+            storeCell(ok, result, cells.seeds[c], c, out, pOut, cOut, rOut);
             if (!ok && failMark) failMark[c] = 1;
-            failed = ok ? 0u : 1u;
+            failed += ok ? 0u : 1u;
             if (cost) cost[c] = uint16_t(n.phases < 65535u ? n.phases : 65535u);
         }
+        phases += n.phases;
     }
-    countFlash(failed, n.phases, counters);
+    countFlash(failed, phases, counters);
 }
 
 // One deferred cell refined without deferral; lead: this lane stores it.
 template <int NS, int NL, bool WAVE>
-__device__ inline void refineQueued(const HemModel<NS>& model, const double* __restrict__ q, size_t stride,
-                                    const ThermoOut* __restrict__ seeds, uint32_t c, const CandidateSet& set,
-                                    bool lead, ThermoOut* __restrict__ out, double* __restrict__ pOut,
-                                    double* __restrict__ cOut, double* __restrict__ rOut, uint16_t* __restrict__ cost,
-                                    uint8_t* __restrict__ failMark, Counts& n, uint32_t& failed) {
-    const ThermoOut g = seeds[c];
+__device__ inline void refineQueued(const HemModel<NS>& model, const FlashCells& cells, uint32_t c,
+                                    const CandidateSet& set, bool lead, ThermoOut* __restrict__ out,
+                                    double* __restrict__ pOut, double* __restrict__ cOut, double* __restrict__ rOut,
+                                    uint16_t* __restrict__ cost, uint8_t* __restrict__ failMark, Counts& n,
+                                    uint32_t& failed) {
     Flash<NS, NL, double, true, false, false, kModelLds, WAVE> f(model, n);
-    loadCell(f, q, stride, g, c, NS);
+    cells.load<NS>(f, c);
     EvalT<double, true> result;
     zeroEval(result);
     const bool ok = f.refine(set, result);
     if (lead) {
-        storeCell(ok, result, g, c, out, pOut, cOut, rOut);
+        storeCell(ok, result, cells.seeds[c], c, out, pOut, cOut, rOut);
         if (!ok && failMark) failMark[c] = 1;
         if (cost) cost[c] = uint16_t(n.phases < 65535u ? n.phases : 65535u);
         failed = ok ? 0u : 1u;
@@ -141,9 +143,8 @@ __device__ inline void refineQueued(const HemModel<NS>& model, const double* __r
 // launch does not depend on it).
 template <int NS, int NL>
 __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void stepRefineQueueKernel(
-    const HemModel<NS>* __restrict__ globalModel, const double* __restrict__ q, size_t stride,
-    const ThermoOut* __restrict__ seeds, const uint32_t* __restrict__ queue, const unsigned* __restrict__ queueCount,
-    const double* __restrict__ dtDev, const CandidateSet* __restrict__ sets, ThermoOut* __restrict__ out,
+    const HemModel<NS>* __restrict__ globalModel, FlashCells cells, const uint32_t* __restrict__ queue,
+    const unsigned* __restrict__ queueCount, const CandidateSet* __restrict__ sets, ThermoOut* __restrict__ out,
     double* __restrict__ pOut, double* __restrict__ cOut, double* __restrict__ rOut, uint16_t* __restrict__ cost,
     unsigned long long* __restrict__ counters, uint8_t* __restrict__ failMark) {
     const unsigned count = *queueCount;
@@ -155,9 +156,9 @@ __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void stepRefineQueueKern
         for (unsigned i = blockIdx.x; i < count; i += gridDim.x) {  // uniform per workgroup
             Counts n = {0, 0, 0, 0, 0, 0, 0};
             uint32_t failed = 0;
-            if (*dtDev > 0)
-                refineQueued<NS, NL, true>(model, q, stride, seeds, queue[i], sets[queue[i]], lead, out, pOut, cOut,
-                                           rOut, cost, failMark, n, failed);
+            if (!cells.gate || *cells.gate > 0)
+                refineQueued<NS, NL, true>(model, cells, queue[i], sets[queue[i]], lead, out, pOut, cOut, rOut, cost,
+                                           failMark, n, failed);
             countFlash(failed, lead ? n.phases : 0u, counters);
         }
     } else {
@@ -165,15 +166,15 @@ __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void stepRefineQueueKern
             const unsigned i = base + threadIdx.x;
             Counts n = {0, 0, 0, 0, 0, 0, 0};
             uint32_t failed = 0;
-            if (i < count && *dtDev > 0)
-                refineQueued<NS, NL, false>(model, q, stride, seeds, queue[i], sets[queue[i]], true, out, pOut, cOut,
-                                            rOut, cost, failMark, n, failed);
+            if (i < count && (!cells.gate || *cells.gate > 0))
+                refineQueued<NS, NL, false>(model, cells, queue[i], sets[queue[i]], true, out, pOut, cOut, rOut, cost,
+                                            failMark, n, failed);
             countFlash(failed, n.phases, counters);
         }
     }
 }
-__global__ void clearQueueKernel(unsigned* __restrict__ count) {
-    if (threadIdx.x == 0) *count = 0;
+__global__ void clearQueueKernel(unsigned* __restrict__ counts) {
+    if (threadIdx.x < kQueueCounts) counts[threadIdx.x] = 0;
 }
 __global__ void queueTotalKernel(const unsigned* __restrict__ count, unsigned long long* __restrict__ total) {
     if (threadIdx.x == 0) atomicAdd(total, (unsigned long long)*count);
@@ -643,6 +644,13 @@ inline unsigned blocksFor(size_t n, unsigned b) { return unsigned((n + b - 1) / 
 #define RAMD_REFINE_QUEUE 1
 #endif
 constexpr unsigned kQueueBlocks = RAMD_QUEUE_BLOCKS;
+// Waves of the refinement over the searched remainder (two fit a SIMD).
+constexpr unsigned kListBlocks = 2048;
+#define RAMD_STEP_SPECIES(LAUNCH)                     \
+    if (h->ns == 1 && h->nl == 0) { LAUNCH(1, 0); }   \
+    else if (h->ns == 1) { LAUNCH(1, 1); }            \
+    else if (h->nl == 0) { LAUNCH(2, 0); }            \
+    else { LAUNCH(2, 1); }
 constexpr int kMarks = 11;  // events per step
 
 // ---------------------------------------------------------------- handle
@@ -698,8 +706,13 @@ struct Step {
     uint16_t* costSearch = nullptr;
     bool haveCostSearch = false;
     CandidateSet* sets = nullptr;
-    uint32_t* queue = nullptr;  // cells the refinement deferred, and their count
-    unsigned* queueCount = nullptr;
+    uint32_t* queue = nullptr;  // cells the refinement deferred
+    unsigned* queueCount = nullptr;  // kQueueCounts counts
+    // a pure fluid's saturation table and the cells it left to the search; the
+    // search's records and restart list
+    SaturationTable* saturation = nullptr;
+    uint32_t* searchList = nullptr;
+    SearchScratch scratch = {};
     int mode = REACTIVE_AMD_FLASH_FP64;
     unsigned *bucketCount = nullptr, *bucketOffset = nullptr;
     // state order: bin keys, bin counts (kept zero between uses) and offsets, range
@@ -766,32 +779,51 @@ struct Step {
             hipLaunchKernelGGL(reuseResolveKernel, dim3(blocksFor(cells, 256)), dim3(256), 0, stream, reuseTable,
                                reuseSlot, cells, rep);
         }
+        const FlashCells batch = {q, all, nullptr, sA, gate(), rep};
         if (mode == REACTIVE_AMD_FLASH_MIXED) {
-#define RAMD_STEP_MIXED(NS_, NL_)                                                                                  \
-    launchSearch(NS_, NL_, h->model, q, all, sA, orderSearch, uint32_t(cells), gate(), sets,                      \
-                 costOut ? costSearch : nullptr, counters + 6, stream, flashBlock, rep);                           \
-    if (split) RAMD_HIP(hipEventRecord(split, stream));                                                            \
-    if (RAMD_REFINE_QUEUE) hipLaunchKernelGGL(clearQueueKernel, dim3(1), dim3(64), 0, stream, queueCount);          \
-    hipLaunchKernelGGL((stepRefineKernel<NS_, NL_>), dim3(blocks), dim3(flashBlock), 0, stream,                     \
-                       static_cast<const HemModel<NS_>*>(h->model), q, all, sA, order, uint32_t(cells), gate(),    \
-                       sets, out, pOut, cOut, rOut, costOut, counter, RAMD_REFINE_QUEUE ? queue : nullptr,         \
-                       queueCount, failMark, rep);                                                                 \
-    if (RAMD_REFINE_QUEUE) {                                                                                       \
-        hipLaunchKernelGGL((stepRefineQueueKernel<NS_, NL_>), dim3(kQueueBlocks), dim3(64), 0, stream,              \
-                           static_cast<const HemModel<NS_>*>(h->model), q, all, sA, queue, queueCount, gate(),      \
-                           sets, out, pOut, cOut, rOut, costOut, counter, failMark);                                \
-        hipLaunchKernelGGL(queueTotalKernel, dim3(1), dim3(64), 0, stream, queueCount, counters + 7);             \
-    }
-            if (h->ns == 1 && h->nl == 0) { RAMD_STEP_MIXED(1, 0); }
-            else if (h->ns == 1) { RAMD_STEP_MIXED(1, 1); }
-            else if (h->nl == 0) { RAMD_STEP_MIXED(2, 0); }
-            else { RAMD_STEP_MIXED(2, 1); }
-#undef RAMD_STEP_MIXED
+            const CellList whole = {order, uint32_t(cells), nullptr};
+            const CellList left = {searchList, 0, queueCount + 1};
+            uint16_t* searchCost = costOut ? costSearch : nullptr;
+            hipLaunchKernelGGL(clearQueueKernel, dim3(1), dim3(64), 0, stream, queueCount);
+            if (saturation)
+                launchDirect(h->model, saturation, batch, orderSearch, uint32_t(cells), sets, searchCost, counters + 6,
+                             stream);
+            else if (h->prune)
+                launchSearch(ns, h->nl, h->model, batch, orderSearch, uint32_t(cells), sets, searchCost, counters + 6,
+                             stream, flashBlock);
+            else
+                launchSearchStarts(ns, h->nl, h->model, batch, {orderSearch, uint32_t(cells), nullptr}, cells, scratch,
+                                   sets, searchCost, counters + 6, stream);
+            if (split) RAMD_HIP(hipEventRecord(split, stream));
+            const auto refine = [&](const CellList& list, unsigned grid, unsigned block) {
+#define RAMD_STEP_REFINE(NS_, NL_)                                                                                 \
+    hipLaunchKernelGGL((stepRefineKernel<NS_, NL_>), dim3(grid), dim3(block), 0, stream,                            \
+                       static_cast<const HemModel<NS_>*>(h->model), batch, list, sets, out, pOut, cOut, rOut,      \
+                       costOut, counter, RAMD_REFINE_QUEUE ? queue : nullptr, queueCount, searchList,              \
+                       queueCount + 1, failMark)
+                RAMD_STEP_SPECIES(RAMD_STEP_REFINE)
+#undef RAMD_STEP_REFINE
+            };
+            refine(whole, blocks, flashBlock);
+            if (saturation) {  // the cells whose table candidates were not confirmed
+                launchSearchStarts(ns, h->nl, h->model, batch, left, cells, scratch, sets, searchCost, counters + 6,
+                                   stream);
+                refine(left, std::min(kListBlocks, blocksFor(cells, 64)), 64);
+            }
+            if (RAMD_REFINE_QUEUE) {
+#define RAMD_STEP_QUEUE(NS_, NL_)                                                                                  \
+    hipLaunchKernelGGL((stepRefineQueueKernel<NS_, NL_>), dim3(kQueueBlocks), dim3(64), 0, stream,                  \
+                       static_cast<const HemModel<NS_>*>(h->model), batch, queue, queueCount, sets, out, pOut,     \
+                       cOut, rOut, costOut, counter, failMark)
+                RAMD_STEP_SPECIES(RAMD_STEP_QUEUE)
+#undef RAMD_STEP_QUEUE
+                hipLaunchKernelGGL(queueTotalKernel, dim3(1), dim3(64), 0, stream, queueCount, counters + 7);
+            }
         } else {
 #define RAMD_STEP_FLASH(NS_, NL_, RJ_)                                                                            \
     hipLaunchKernelGGL((stepFlashKernel<NS_, NL_, RJ_>), dim3(blocks), dim3(flashBlock), 0, stream,                \
-                       static_cast<const HemModel<NS_>*>(h->model), q, all, sA, order, uint32_t(cells), gate(), out, \
-                       pOut, cOut, rOut, costOut, counter, failMark, rep)
+                       static_cast<const HemModel<NS_>*>(h->model), batch, order, uint32_t(cells), out, pOut,      \
+                       cOut, rOut, costOut, counter, failMark)
             if (h->ns == 1 && h->nl == 0) { RAMD_STEP_FLASH(1, 0, false); }
             else if (h->ns == 1 && !h->analytic) { RAMD_STEP_FLASH(1, 1, false); }
             else if (h->ns == 1) { RAMD_STEP_FLASH(1, 1, true); }
@@ -1301,7 +1333,18 @@ int reactive_amd_step_run(void* step, double cfl, double maximum, int steps, int
         if (flashMode == REACTIVE_AMD_FLASH_MIXED && !s.sets) {
             s.sets = s.alloc<CandidateSet>(s.cells);
             s.queue = s.alloc<uint32_t>(s.cells);
-            s.queueCount = s.alloc<unsigned>(1);
+            s.queueCount = s.alloc<unsigned>(kQueueCounts);
+            if (!s.h->prune) {
+                // one record per start and cell; a pure fluid searches only the cells its table leaves
+                s.scratch.records = s.alloc<StartRecord>(kStarts * s.cells);
+                s.scratch.restarts = s.alloc<uint32_t>(s.cells);
+                s.scratch.restartCount = s.queueCount + 2;
+            }
+            if (s.h->pure()) {
+                s.searchList = s.alloc<uint32_t>(s.cells);
+                s.saturation = s.alloc<SaturationTable>(1);
+                launchSaturation(s.h->model, s.saturation, s.stream);
+            }
         }
         s.mode = flashMode;
         if (reuse && !s.reuseTable) {
