@@ -202,6 +202,8 @@ enum CandidateFlags : uint32_t {
     kOverflow = 2u,          // more distinct candidates than the set holds
     kSeedsPruned = 4u,       // the stable-gas pruning skipped the seeds
     kDirect = 8u,            // the directed search's (saturation table): one candidate or none
+    kNotGas = 16u,           // with kDirect: the all-gas solve cannot lead to the equilibrium
+    kNotLiquid = 32u,        // with kDirect: nor can the all-liquid one
 };
 enum StartBits : uint32_t {
     kStartFound = 1u,   // converged, or stalled near convergence
@@ -1492,45 +1494,45 @@ struct Flash : FlashCap<CAP, R> {
         const float at[3] = {float(x[0]), float(x[1]), float(x[2])};
         noteCandidate(*record, kind, index, at, dedupe);
     }
-    // One start of the search on its own (searchStartsKernel): 0 the all-gas
-    // solve, 1 the all-liquid one, 2 + j seed j, 7 + 5 t + j seed j from restart
-    // temperature t, in searchRecord's order.  Every start begins at the
-    // cell's own inputs, so running them apart finds what the sequence finds.
-    // x: the point reached; returns kStart* bits (0: no such start, or no candidate).
-    // `start` is the same in every lane that calls: where lanes take both
-    // sides of a branch around calls, the compiler may keep a call's saved
-    // scalar registers, written for the whole wave, in the stack slot of a
-    // value that the lanes of the other side still need.
-    RAMD_NOINLINE uint32_t searchStart(int start, R* x) {
-        if (!fin(energy) || !(density() > 0)) return 0;
-        for (int k = 0; k < NS; ++k)
-            if (!fin(q[k]) || q[k] < 0) return 0;
-        E candidate;
-        bool ok;
-        if (start < 2) {
-            if (start == 1) {
-                if (!NL) return 0;
-                R other = 0;
-                for (int k = 0; k < NS; ++k)
-                    if (k != mod().condensable) other += q[k];
-                if (other != 0) return 0;
-            }
-            ok = frozen(start == 0 ? R(0) : q[mod().condensable], candidate, 0);
-            if (!ok && !stalled) return 0;
-            x[0] = m_log(candidate.p);
-            x[1] = m_log(candidate.T);
-            x[2] = 0;
-        } else {
-            if (!NL || !(q[mod().condensable] > 0)) return 0;
-            const bool restart = start >= 7;
-            const int j = restart ? (start - 7) % 5 : start - 2;
-            const R seed = j == 0 ? R(-1) : j == 1 ? R(.5) : j == 2 ? R(.95) : j == 3 ? R(.1) : R(.9999);
-            R scale;
-            ++n.candidates;
-            activeStart(seed, restart, restart ? restartTemperature((start - 7) / 5) : R(0), x, scale);
-            ok = activeNewton(x, scale, candidate, 0);
-            if (!ok && !stalled) return 0;
+    // One start of the search on its own: 0 the all-gas solve, 1 the
+    // all-liquid one (searchFrozen), 2 + j seed j, 7 + 5 t + j seed j from
+    // restart temperature t (searchSeed), in searchRecord's order.  Every
+    // start begins at the cell's own inputs, so running them apart finds what
+    // the sequence finds.  x: the point reached; returns kStart* bits (0: no
+    // such start, or no candidate).
+    RD bool searchable() const {
+        bool ok = fin(energy) && density() > 0;
+        for (int k = 0; k < NS; ++k) ok = ok && fin(q[k]) && q[k] >= 0;
+        return ok;
+    }
+    RAMD_NOINLINE uint32_t searchFrozen(bool liquid, R* x) {
+        if (!searchable()) return 0;
+        if (liquid) {
+            if (!NL) return 0;
+            R other = 0;
+            for (int k = 0; k < NS; ++k)
+                if (k != mod().condensable) other += q[k];
+            if (other != 0) return 0;
         }
+        E candidate;
+        const bool ok = frozen(liquid ? q[mod().condensable] : R(0), candidate, 0);
+        if (!ok && !stalled) return 0;
+        x[0] = m_log(candidate.p);
+        x[1] = m_log(candidate.T);
+        x[2] = 0;
+        return kStartFound | (ok && stable(candidate) ? kStartStable : 0u);
+    }
+    RAMD_NOINLINE uint32_t searchSeed(int start, R* x) {
+        if (!searchable() || !NL || !(q[mod().condensable] > 0)) return 0;
+        const bool restart = start >= 7;
+        const int j = restart ? (start - 7) % 5 : start - 2;
+        const R seed = j == 0 ? R(-1) : j == 1 ? R(.5) : j == 2 ? R(.95) : j == 3 ? R(.1) : R(.9999);
+        E candidate;
+        R scale;
+        ++n.candidates;
+        activeStart(seed, restart, restart ? restartTemperature((start - 7) / 5) : R(0), x, scale);
+        const bool ok = activeNewton(x, scale, candidate, 0);
+        if (!ok && !stalled) return 0;
         return kStartFound | (ok && stable(candidate) ? kStartStable : 0u);
     }
     RAMD_NOINLINE void searchRecord(CandidateSet& set) {

@@ -160,11 +160,12 @@ struct StartRecord {
     uint32_t bits;
 };
 // Scratch of the search: kStarts records per listed cell (record s of list
-// position i at s stride + i) and the cells to restart.
+// position i at s stride + i), the cells to restart, and the directed
+// search's cells to try again; the counts are zero on entry.
 struct SearchScratch {
     StartRecord* records;
-    uint32_t* restarts;
-    unsigned* restartCount;
+    uint32_t *restarts, *again;
+    unsigned *restartCount, *againCount;
 };
 // Saturated liquid and vapour at evenly spaced temperatures: specific volumes
 // and energies, ln p.  Interpolated between 2,048 rows over N2O's 161 K they
@@ -183,15 +184,17 @@ struct SaturationTable {
 void launchSaturation(const void* model, SaturationTable* table, hipStream_t stream);
 // The directed search of every cell in `order`: sets of one candidate or none, flagged kDirect.
 void launchDirect(const void* model, const SaturationTable* table, const FlashCells& cells, const uint32_t* order,
-                  uint32_t count, CandidateSet* sets, uint16_t* cost, unsigned long long* phases, hipStream_t stream);
+                  uint32_t count, const SearchScratch& scratch, CandidateSet* sets, uint16_t* cost,
+                  unsigned long long* phases, hipStream_t stream);
 // Single-precision search, one cell per lane in workgroups of `block` lanes
 // (64, 128 or 256); candidate sets and evaluation counts by cell.
 void launchSearch(int ns, int nl, const void* model, const FlashCells& cells, const uint32_t* order, uint32_t count,
                   CandidateSet* sets, uint16_t* cost, unsigned long long* phases, hipStream_t stream, unsigned block);
 // The same search, one start per lane, for models without stable-gas pruning;
-// stride: the list's largest length.  *scratch.restartCount is zero on entry.
+// stride: the list's largest length; directed: the sets are the directed
+// search's, whose flags leave out some of the frozen solves.
 void launchSearchStarts(int ns, int nl, const void* model, const FlashCells& cells, const CellList& list, size_t stride,
-                        const SearchScratch& scratch, CandidateSet* sets, uint16_t* cost,
+                        const SearchScratch& scratch, bool directed, CandidateSet* sets, uint16_t* cost,
                         unsigned long long* phases, hipStream_t stream);
 
 }  // namespace ramd

@@ -216,9 +216,9 @@ __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineQueueKerne
     }
 }
 
-// deferred cells, cells to search, cells to restart
+// deferred cells, cells to search, cells to restart, cells the directed search tries again
 __global__ void clearCountsKernel(unsigned* __restrict__ counts) {
-    if (threadIdx.x < 3) counts[threadIdx.x] = 0;
+    if (threadIdx.x < 4) counts[threadIdx.x] = 0;
 }
 
 // totals[k] = sum over b < blocks of partials[b * width + k], k < width: one
@@ -314,7 +314,7 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
     if (!count) return;
     if (!sets) {
         queue = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
-        queueCount = static_cast<unsigned*>(allocate(3 * sizeof(unsigned)));
+        queueCount = static_cast<unsigned*>(allocate(4 * sizeof(unsigned)));
         if (!prune) {
             scratch.records = static_cast<StartRecord*>(allocate(kStarts * capacity * sizeof(StartRecord)));
             scratch.restarts = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
@@ -322,6 +322,8 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
         }
         if (pure()) {
             searchList = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
+            scratch.again = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
+            scratch.againCount = queueCount + 3;
             saturation = static_cast<SaturationTable*>(allocate(sizeof(SaturationTable)));
             launchSaturation(model, saturation, s);
         }
@@ -332,15 +334,15 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
     const CellList whole = {order, uint32_t(count), nullptr}, left = {searchList, 0, queueCount + 1};
     hipLaunchKernelGGL(zeroTotalsKernel, dim3(1), dim3(64), 0, s, totals, 10);
     hipLaunchKernelGGL(clearCountsKernel, dim3(1), dim3(64), 0, s, queueCount);
-    if (saturation) launchDirect(model, saturation, cells, order, uint32_t(count), sets, nullptr, totals + 8, s);
+    if (saturation) launchDirect(model, saturation, cells, order, uint32_t(count), scratch, sets, nullptr, totals + 8, s);
     else if (prune) launchSearch(ns, nl, model, cells, order, uint32_t(count), sets, nullptr, totals + 8, s, 64);
-    else launchSearchStarts(ns, nl, model, cells, whole, count, scratch, sets, nullptr, totals + 8, s);
+    else launchSearchStarts(ns, nl, model, cells, whole, count, scratch, false, sets, nullptr, totals + 8, s);
 #define RAMD_HEM_MIXED(NS_, NL_)                                                                                  \
     hipLaunchKernelGGL((hemRefineKernel<NS_, NL_>), dim3(blocks), dim3(64), 0, s,                                   \
                        static_cast<const HemModel<NS_>*>(model), cells, whole, sets, out, totals, queue,          \
                        queueCount, searchList, queueCount + 1);                                                   \
     if (saturation) {                                                                                             \
-        launchSearchStarts(ns, nl, model, cells, left, count, scratch, sets, nullptr, totals + 8, s);             \
+        launchSearchStarts(ns, nl, model, cells, left, count, scratch, true, sets, nullptr, totals + 8, s);       \
         hipLaunchKernelGGL((hemRefineKernel<NS_, NL_>), dim3(std::min(2048u, blocks)), dim3(64), 0, s,              \
                            static_cast<const HemModel<NS_>*>(model), cells, left, sets, out, totals, queue,       \
                            queueCount, searchList, queueCount + 1);                                               \

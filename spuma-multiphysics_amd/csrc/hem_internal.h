@@ -42,7 +42,7 @@ struct HemHandle {
     // evaluations and deferred cells
     CandidateSet* sets = nullptr;
     uint32_t* queue = nullptr;
-    unsigned* queueCount = nullptr;  // deferred cells, cells to search, cells to restart
+    unsigned* queueCount = nullptr;  // deferred cells; to search, to restart, to try again
     SaturationTable* saturation = nullptr;
     uint32_t* searchList = nullptr;
     SearchScratch scratch = {};

@@ -51,7 +51,8 @@ __global__ __launch_bounds__(256, RAMD_SEARCH_MIN_WAVES) void searchKernel(
 template <int NS, int NL>
 __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchStartsKernel(
     const HemModel<NS>* __restrict__ globalModel, FlashCells cells, CellList list, size_t stride,
-    StartRecord* __restrict__ records, unsigned long long* __restrict__ phases) {
+    const CandidateSet* __restrict__ directed, StartRecord* __restrict__ records,
+    unsigned long long* __restrict__ phases) {
     const uint32_t count = list.size();
     if (blockIdx.x * 64u >= count) return;  // uniform per workgroup
     const HemModel<NS>& model = workgroupModel(globalModel);
@@ -63,7 +64,9 @@ __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchStartsKernel(
             Flash<NS, NL, float, true, false, false, kModelLds> f(model, n);
             cells.load<NS>(f, list.cells[i]);
             StartRecord r;
-            r.bits = f.searchStart(int(blockIdx.y), r.x);
+            if (blockIdx.y >= 2) r.bits = f.searchSeed(int(blockIdx.y), r.x);
+            else if (directed && (directed[list.cells[i]].flags & (blockIdx.y ? kNotLiquid : kNotGas))) r.bits = 0;
+            else r.bits = f.searchFrozen(blockIdx.y == 1, r.x);
             r.bits |= n.phases << 2;
             records[size_t(blockIdx.y) * stride + i] = r;
             total += n.phases;
@@ -131,7 +134,7 @@ __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchRestartsKerne
             Flash<NS, NL, float, true, false, false, kModelLds> f(model, n);
             cells.load<NS>(f, list.cells[i]);
             StartRecord r;
-            r.bits = f.searchStart(kStarts + int(s), r.x);
+            r.bits = f.searchSeed(kStarts + int(s), r.x);
             r.bits |= n.phases << 2;
             found[threadIdx.x] = r;
             total += n.phases;
@@ -164,15 +167,20 @@ __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchRestartsKerne
 // saturation temperature T has v_l(T) < 1/rho < v_v(T) and the lever rule's
 // energy equal to e, one phase elsewhere.  Which it is, and where, is looked
 // up: T by bisection in a table of the saturation curve, or, outside the
-// dome, by Newton's method on e(T) at fixed rho.  Of the search's seven
-// solves only one can then lead there; it alone is run (for two phases, from
-// the seed nearest the known liquid fraction), since the reference accepts a
-// cell only where one of its solves arrives.  The refinement then confirms
-// the point with the FP64 solver and stability test, as it does a searched
-// candidate.  A cell whose solve does not arrive or whose point is not
-// confirmed (and every cell the table says too little about: colder than the
-// table, near the critical point or the dome's edge, outside the model's
-// range) runs the whole search.
+// dome, by Newton's method on e(T) at fixed rho.  The reference accepts a
+// cell only where one of its solves arrives, so one has to be seen to: for
+// one phase its own solve, for two any seed (of the step-start temperature,
+// or of a restart temperature: those run only if no other start finds a
+// stable point, and here none could).  The seed nearest the known liquid
+// fraction arrives in about 90 % of the two-phase cells of a seeded box, and
+// of the rest the restart nearest the known point in as many as all twenty
+// restarts together; the second try runs over a compacted list.  The
+// refinement then confirms the point with the FP64 solver and stability
+// test, as it does a searched candidate.  A cell whose solves do not arrive
+// or whose point is not confirmed (and every cell the table says too little
+// about: colder than the table, near the critical point or the dome's edge,
+// outside the model's range) runs the whole search, but for the frozen
+// solves that cannot lead to the known point.
 __global__ void saturationInitKernel(SaturationTable* __restrict__ table) {
     if (threadIdx.x == 0) table->count = kSaturationRows;
 }
@@ -285,6 +293,8 @@ __device__ inline void directCandidate(const HemModel<NS>& m, const SaturationTa
         const double w = clamp((u - ea) / (eb - ea), 0., 1.);
         const double vl = a.vl + w * (b.vl - a.vl), vv = a.vv * ::exp(w * ::log(b.vv / a.vv));
         const double liquid = (vv - v) / (vv - vl);
+        if (liquid > kDomeEdge) set.flags |= kNotGas;
+        if (liquid < 1 - kDomeEdge) set.flags |= kNotLiquid;
         if (!(liquid > kDomeEdge && liquid < 1 - kDomeEdge)) return;
         const float at[3] = {float(a.lnp + w * (b.lnp - a.lnp)), float(::log(table.T0 + (low + w) * table.dT)),
                              float(liquid)};
@@ -295,7 +305,10 @@ __device__ inline void directCandidate(const HemModel<NS>& m, const SaturationTa
         // the dome ends between the rows: one phase where its edge lies well below the cell's energy
         const SaturationRow& r = table.row[high];
         const bool vapour = v >= r.vv;
-        if (u < (vapour ? r.ev : r.el) + kDomeEdge * (r.ev - r.el)) return;
+        if (u < (vapour ? r.ev : r.el) + kDomeEdge * (r.ev - r.el)) {
+            set.flags |= vapour ? kNotLiquid : kNotGas;
+            return;
+        }
     }
     const SaturationRow& r = table.row[high];
     const bool vapour = v >= r.vv;
@@ -312,11 +325,24 @@ __device__ inline void directCandidate(const HemModel<NS>& m, const SaturationTa
     noteCandidate(set, vapour || T >= float(m.liquidTc) ? kGasCandidate : kLiquidCandidate, 0, at, false);
 }
 
+// The liquid fraction of seed j for a flash input.
+template <int NS>
+__device__ inline float seedFraction(const FlashInput<NS>& at, int j) {
+    return j == 0 ? clamp(float(at.guessLiquid / at.q[0]), 0.f, 1.f) : j == 1 ? .5f : j == 2 ? .95f : j == 3 ? .1f : .9999f;
+}
+template <int NS>
+__device__ inline int nearestSeed(const FlashInput<NS>& at, float liquid, int first) {
+    int nearest = first;
+    for (int j = first + 1; j < 5; ++j)
+        if (ab(seedFraction(at, j) - liquid) < ab(seedFraction(at, nearest) - liquid)) nearest = j;
+    return nearest;
+}
+
 template <int NS>
 __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void directKernel(
     const HemModel<NS>* __restrict__ globalModel, const SaturationTable* __restrict__ table, FlashCells cells,
     const uint32_t* __restrict__ order, uint32_t count, CandidateSet* __restrict__ sets, uint16_t* __restrict__ cost,
-    unsigned long long* __restrict__ phases) {
+    unsigned long long* __restrict__ phases, uint32_t* __restrict__ again, unsigned* __restrict__ againCount) {
     const HemModel<NS>& model = workgroupModel(globalModel);
     const uint32_t i = blockIdx.x * 64u + threadIdx.x;
     const bool active = i < count && cells.flashed(order[i]);
@@ -328,36 +354,68 @@ __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void directKernel(
     cells.load<NS>(at, c);
     if (active) directCandidate<NS>(model, *table, at.q[0], at.energy, at.guessT, set, n.phases);
     int start = -1;
-    if (set.count) {
-        start = set.c[0].kind == kGasCandidate ? 0 : 1;
-        if (set.c[0].kind == kSeedCandidate) {
-            const float seeds[5] = {clamp(float(at.guessLiquid / at.q[0]), 0.f, 1.f), .5f, .95f, .1f, .9999f};
-            int nearest = 0;
-            float least = 2;
-            for (int j = 0; j < 5; ++j) {
-                const float d = ab(seeds[j] - set.c[0].x[2]);
-                if (d < least) { least = d; nearest = j; }
-            }
-            start = 2 + nearest;
-        }
-    }
+    if (set.count)
+        start = set.c[0].kind == kGasCandidate      ? 0
+                : set.c[0].kind == kLiquidCandidate ? 1
+                                                    : 2 + nearestSeed(at, set.c[0].x[2], 0);
     Flash<NS, 1, float, true, false, false, kModelLds> f(model, n);
     cells.load<NS>(f, c);
-    // one start at a time, for the lanes that take it (searchStart's condition)
     uint32_t bits = 0;
-    for (unsigned long long pending = __ballot(start >= 0); pending; pending &= ~__ballot(bits & 4u)) {
-        const int s = __shfl(start, __ffsll(pending) - 1, 64);
-        if (start == s) {
-            float x[3];
-            bits = f.searchStart(s, x) | 4u;
-        }
+    float x[3];
+    if (start >= 2) bits = f.searchSeed(start, x);
+    // The two kinds of start are separate passes of the whole wave: as the
+    // two sides of one branch, the compiler may keep scalar registers that a
+    // call on one side saves (a store of all 64 lanes) in the stack slot of a
+    // value that only the other side's lanes still need.
+    asm volatile("" : "+v"(start), "+v"(bits));
+    if (start == 0 || start == 1) bits = f.searchFrozen(start == 1, x);
+    if (!(bits & kStartFound)) {
+        set.count = 0;
+        if (start >= 2) again[atomicAdd(againCount, 1u)] = c;
     }
-    if (!(bits & kStartFound)) set.count = 0;
     if (active) {
         sets[c] = set;
         if (cost) cost[c] = uint16_t(n.phases < 65535u ? n.phases : 65535u);
     }
     const uint32_t sum = waveSum(active ? n.phases : 0u);
+    if (threadIdx.x == 0) atomicAdd(phases, (unsigned long long)sum);
+}
+
+// The second try of the listed two-phase cells: the restart nearest the known
+// point in temperature and liquid fraction.  Their sets hold the point with a
+// count of zero.
+template <int NS>
+__global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void directAgainKernel(
+    const HemModel<NS>* __restrict__ globalModel, FlashCells cells, CellList list, CandidateSet* __restrict__ sets,
+    uint16_t* __restrict__ cost, unsigned long long* __restrict__ phases) {
+    const uint32_t count = list.size();
+    if (blockIdx.x * 64u >= count) return;  // uniform per workgroup
+    const HemModel<NS>& model = workgroupModel(globalModel);
+    uint32_t total = 0;
+    for (uint32_t base = blockIdx.x * 64u; base < count; base += gridDim.x * 64u) {
+        const uint32_t i = base + threadIdx.x;
+        if (i < count) {
+            const uint32_t c = list.cells[i];
+            Counts n = {0, 0, 0, 0, 0, 0, 0};
+            FlashInput<NS> at;
+            cells.load<NS>(at, c);
+            Flash<NS, 1, float, true, false, false, kModelLds> f(model, n);
+            cells.load<NS>(f, c);
+            const float T = m_exp(sets[c].c[0].x[1]);
+            int t = 0;
+            for (int k = 1; k < 4; ++k)
+                if (ab(f.restartTemperature(k) - T) < ab(f.restartTemperature(t) - T)) t = k;
+            float x[3];
+            if (f.searchSeed(kStarts + 5 * t + nearestSeed(at, sets[c].c[0].x[2], 1), x) & kStartFound)
+                sets[c].count = 1;
+            total += n.phases;
+            if (cost) {
+                const uint32_t evaluations = n.phases + cost[c];
+                cost[c] = uint16_t(evaluations < 65535u ? evaluations : 65535u);
+            }
+        }
+    }
+    const uint32_t sum = waveSum(total);
     if (threadIdx.x == 0) atomicAdd(phases, (unsigned long long)sum);
 }
 
@@ -372,13 +430,6 @@ void launchSaturation(const void* model, SaturationTable* table, hipStream_t str
     hipLaunchKernelGGL(saturationInitKernel, dim3(1), dim3(64), 0, stream, table);
     hipLaunchKernelGGL((saturationKernel<1>), dim3((kSaturationRows + 63) / 64), dim3(64), 0, stream,
                        static_cast<const HemModel<1>*>(model), table);
-    RAMD_HIP(hipGetLastError());
-}
-
-void launchDirect(const void* model, const SaturationTable* table, const FlashCells& cells, const uint32_t* order,
-                  uint32_t count, CandidateSet* sets, uint16_t* cost, unsigned long long* phases, hipStream_t stream) {
-    hipLaunchKernelGGL((directKernel<1>), dim3(unsigned((size_t(count) + 63) / 64)), dim3(64), 0, stream,
-                       static_cast<const HemModel<1>*>(model), table, cells, order, count, sets, cost, phases);
     RAMD_HIP(hipGetLastError());
 }
 
@@ -397,14 +448,27 @@ void launchSearch(int ns, int nl, const void* model, const FlashCells& cells, co
 // chip at the search's five waves per SIMD; a longer list takes more rounds.
 constexpr unsigned kListWaves = 5120;
 
+void launchDirect(const void* model, const SaturationTable* table, const FlashCells& cells, const uint32_t* order,
+                  uint32_t count, const SearchScratch& scratch, CandidateSet* sets, uint16_t* cost,
+                  unsigned long long* phases, hipStream_t stream) {
+    const unsigned waves = unsigned((size_t(count) + 63) / 64);
+    hipLaunchKernelGGL((directKernel<1>), dim3(waves), dim3(64), 0, stream, static_cast<const HemModel<1>*>(model),
+                       table, cells, order, count, sets, cost, phases, scratch.again, scratch.againCount);
+    hipLaunchKernelGGL((directAgainKernel<1>), dim3(std::min(kListWaves, waves)), dim3(64), 0, stream,
+                       static_cast<const HemModel<1>*>(model), cells,
+                       CellList{scratch.again, 0, scratch.againCount}, sets, cost, phases);
+    RAMD_HIP(hipGetLastError());
+}
+
 void launchSearchStarts(int ns, int nl, const void* model, const FlashCells& cells, const CellList& list, size_t stride,
-                        const SearchScratch& scratch, CandidateSet* sets, uint16_t* cost,
+                        const SearchScratch& scratch, bool directed, CandidateSet* sets, uint16_t* cost,
                         unsigned long long* phases, hipStream_t stream) {
     const unsigned waves = unsigned((stride + 63) / 64);
     const unsigned blocks = list.counted ? std::min(waves, kListWaves / kStarts) : waves;
 #define RAMD_STARTS(NS_, NL_)                                                                                \
     hipLaunchKernelGGL((searchStartsKernel<NS_, NL_>), dim3(blocks, kStarts), dim3(64), 0, stream,            \
-                       static_cast<const HemModel<NS_>*>(model), cells, list, stride, scratch.records, phases); \
+                       static_cast<const HemModel<NS_>*>(model), cells, list, stride,                                   \
+                       directed ? sets : nullptr, scratch.records, phases);                                   \
     hipLaunchKernelGGL((searchMergeKernel<NS_>), dim3(std::min(2048u, (waves + 3) / 4)), dim3(256), 0, stream, \
                        static_cast<const HemModel<NS_>*>(model), cells, list, stride, scratch.records, sets, cost, \
                        scratch.restarts, scratch.restartCount);                                              \

@@ -36,8 +36,9 @@
 namespace ramd {
 
 // ---------------------------------------------------------------- kernels
-// Counts of the mixed flash's lists: deferred cells, cells to search, cells to restart.
-constexpr int kQueueCounts = 3;
+// Counts of the mixed flash's lists: deferred cells, cells to search, cells to restart,
+// cells the directed search tries again.
+constexpr int kQueueCounts = 4;
 
 // Plain FP64 flash of the cells in `order`; RJ: the model's
 // analytic-Jacobian mode.
@@ -786,14 +787,14 @@ struct Step {
             uint16_t* searchCost = costOut ? costSearch : nullptr;
             hipLaunchKernelGGL(clearQueueKernel, dim3(1), dim3(64), 0, stream, queueCount);
             if (saturation)
-                launchDirect(h->model, saturation, batch, orderSearch, uint32_t(cells), sets, searchCost, counters + 6,
-                             stream);
+                launchDirect(h->model, saturation, batch, orderSearch, uint32_t(cells), scratch, sets, searchCost,
+                             counters + 6, stream);
             else if (h->prune)
                 launchSearch(ns, h->nl, h->model, batch, orderSearch, uint32_t(cells), sets, searchCost, counters + 6,
                              stream, flashBlock);
             else
                 launchSearchStarts(ns, h->nl, h->model, batch, {orderSearch, uint32_t(cells), nullptr}, cells, scratch,
-                                   sets, searchCost, counters + 6, stream);
+                                   false, sets, searchCost, counters + 6, stream);
             if (split) RAMD_HIP(hipEventRecord(split, stream));
             const auto refine = [&](const CellList& list, unsigned grid, unsigned block) {
 #define RAMD_STEP_REFINE(NS_, NL_)                                                                                 \
@@ -806,8 +807,8 @@ struct Step {
             };
             refine(whole, blocks, flashBlock);
             if (saturation) {  // the cells whose table candidates were not confirmed
-                launchSearchStarts(ns, h->nl, h->model, batch, left, cells, scratch, sets, searchCost, counters + 6,
-                                   stream);
+                launchSearchStarts(ns, h->nl, h->model, batch, left, cells, scratch, true, sets, searchCost,
+                                   counters + 6, stream);
                 refine(left, std::min(kListBlocks, blocksFor(cells, 64)), 64);
             }
             if (RAMD_REFINE_QUEUE) {
@@ -1342,6 +1343,8 @@ int reactive_amd_step_run(void* step, double cfl, double maximum, int steps, int
             }
             if (s.h->pure()) {
                 s.searchList = s.alloc<uint32_t>(s.cells);
+                s.scratch.again = s.alloc<uint32_t>(s.cells);
+                s.scratch.againCount = s.queueCount + 3;
                 s.saturation = s.alloc<SaturationTable>(1);
                 launchSaturation(s.h->model, s.saturation, s.stream);
             }
