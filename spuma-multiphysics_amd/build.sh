@@ -2,12 +2,16 @@
 # Builds lib/libreactiveTransport.so (HIP, gfx950) from csrc/.
 # Rounding policy: IEEE FP64, no contraction (-ffp-contract=off), no fast-math;
 # search.hip (the FP32 candidate search only) adds -freciprocal-math -fapprox-func.
+# Stack slots are not shared: where the lanes of a wave take both sides of a
+# branch around calls, the compiler keeps the scalar registers that one side
+# saves (stores of all 64 lanes) in slots that lanes of the other side still use.
 set -euo pipefail
 here="$(cd -- "$(dirname -- "${BASH_SOURCE[0]}")" && pwd)"
 hipcc="${HIPCC:-/opt/rocm/bin/hipcc}"
 mkdir -p "$here/lib" "$here/_build"
 flags=(--offload-arch=gfx950 -O3 -std=c++17 -fPIC -ffp-contract=off -fno-fast-math
        -Xclang -target-feature -Xclang -packed-fp32-ops
+       -mllvm -no-stack-slot-sharing
        -I"$here/../include" -Wall -Wno-unused-result)
 objs=()
 pids=()

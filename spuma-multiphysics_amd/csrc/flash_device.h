@@ -360,25 +360,24 @@ __device__ inline HemModel<NS>& sharedModel() {
 
 // LDS: the model is the workgroup's LDS copy (sharedModel); otherwise the
 // reference given to the constructor.
-// WAVE: every lane of a wave runs this flash on the same cell (so its
-// control flow is the wave's), and the Newton line searches evaluate their
-// fractions on the wave's lanes at once, lane j the j-th fraction of the
-// loop; the first accepted fraction in loop order is taken, which is the
-// loop's choice, so the results are those of the one-lane flash bit for bit
-// (the rejected evaluations it adds change nothing: the flash's only memo,
-// an unavailable liquid at (p, T), repeats what recomputing gives).  For the
-// few long refinements: a frozen solve that crawls halves each of its seventy
-// Newton steps many times.  Every lane makes the active set's residual call
-// (the lanes past the loop's end repeat its last fraction): with the call
-// made by only some lanes, the results depended on what earlier work had
-// left on the device.
+// GROUP: 1, or the number of neighbouring lanes (8) that run each solve of
+// this flash together, all on the same cell and start, so that their control
+// flow is one.  A Newton line search evaluates GROUP of its fractions at
+// once, lane j the j-th, and takes the first accepted one in loop order, the
+// loop's own choice; a finite-difference Jacobian evaluates its six residuals
+// at once.  The results are those of the one-lane flash bit for bit, and so
+// are the counts (the evaluations past the loop's end are not counted; the
+// flash's only memo, an unavailable liquid at (p, T), repeats what
+// recomputing gives).  searchGroups runs a cell's starts on the eight groups
+// of a wave.  Every lane of a group makes every call (lanes past a loop's end
+// repeat its last point).
 template <int NS, int NL, class R = double, bool A = FlashPrecision<R>::single, bool RJ = false, bool CAP = false,
-          bool LDS = false, bool WAVE = false>
+          bool LDS = false, int GROUP = 1>
 struct Flash : FlashCap<CAP, R> {
     static_assert(NL == 0 || NL == 1, "one pure liquid at most");
     static_assert(!RJ || (!A && !FlashPrecision<R>::single), "the reference's analytic mode is an FP64 flash");
     static_assert(!CAP || (!A && !FlashPrecision<R>::single), "the capillary flash is an FP64 flash");
-    static_assert(!WAVE || !FlashPrecision<R>::single, "wave-shared line searches are an FP64 refinement");
+    static_assert(GROUP == 1 || (GROUP == 8 && !FlashPrecision<R>::single), "groups of eight lanes, FP64 only");
     using P = FlashPrecision<R>;
     using E = EvalT<R, A, RJ, CAP>;
     using S = PRStateT<R>;
@@ -416,19 +415,52 @@ struct Flash : FlashCap<CAP, R> {
         record = nullptr;
         stalled = false;
     }
-    // WAVE: after a line search shared by the wave, the counts the one-lane
-    // loop makes (the trials up to lane `last`, the winner or all), the same
-    // in every lane.
-    RD void waveCounts(const Counts& before, int last) {
-        const int lane = int(threadIdx.x & 63u);
-        uint32_t phases = lane <= last ? n.phases - before.phases : 0u;
-        uint32_t residuals = lane <= last ? n.residuals - before.residuals : 0u;
-        for (int o = 32; o > 0; o >>= 1) {
-            phases += uint32_t(__shfl_xor(int(phases), o, 64));
-            residuals += uint32_t(__shfl_xor(int(residuals), o, 64));
-        }
+    // GROUP: this lane's place in its group, the group's first lane, a ballot
+    // over the group and a group lane's value.
+    static RD int groupLane() { return int(threadIdx.x) & (GROUP - 1); }
+    static RD int groupBase() { return int(threadIdx.x & 63u) & ~(GROUP - 1); }
+    static RD unsigned groupBallot(bool v) {
+        return unsigned(__ballot(v) >> groupBase()) & ((1u << GROUP) - 1u);
+    }
+    template <class T>
+    static RD T groupValue(const T& v, int lane) {
+        return waveBroadcast(v, groupBase() + lane);
+    }
+    static RD uint32_t groupSum(uint32_t v) {
+        for (int o = GROUP / 2; o > 0; o >>= 1) v += uint32_t(__shfl_xor(int(v), o, 64));
+        return v;
+    }
+    // The flash's memo (the last unavailable liquid's point).
+    struct Memo {
+        R p, T;
+        int status, virtualLiquids;
+    };
+    RD Memo memoNow() const { return {cacheP, cacheT, cacheStatus, int(cacheVirtual)}; }
+    RD void memoSet(const Memo& v) {
+        cacheP = v.p;
+        cacheT = v.T;
+        cacheStatus = v.status;
+        cacheVirtual = v.virtualLiquids != 0;
+    }
+    // After evaluations at (p, T) shared by the group, lane j the j-th of the
+    // sequence and every lane with the memo `entry` before it: the counts of
+    // the lanes up to `last` (of those `counted`) and the memo as the sequence
+    // leaves them, the same in every lane.  An evaluation that repeats the
+    // unavailable point before it is one the memo spares the sequence.
+    RD void groupCounts(const Counts& before, const Memo& entry, R p, R T, bool counted, int last) {
+        const bool took = counted && groupLane() <= last;
+        const bool missed = took && cacheStatus >= 0 && cacheP == p && cacheT == T;
+        const unsigned misses = groupBallot(missed);
+        const int previous = hi(groupLane() - 1, 0);
+        const R beforeP = __shfl(p, groupBase() + previous, 64), beforeT = __shfl(T, groupBase() + previous, 64);
+        const bool spared = groupLane() > 0 && (misses >> previous & 1u) && missed && beforeP == p && beforeT == T;
+        const uint32_t phases = groupSum(took && !spared ? n.phases - before.phases : 0u);
+        const uint32_t residuals = groupSum(took ? n.residuals - before.residuals : 0u);
         n.phases = before.phases + phases;
         n.residuals = before.residuals + residuals;
+        const Memo mine = memoNow();
+        const Memo left = groupValue(mine, misses ? 31 - __builtin_clz(misses) : 0);
+        memoSet(misses ? left : entry);
     }
     // Phase pressures of a curved interface (reactiveDeviceFlash.h:152-153).
     RD R gasPressure(R p) const {
@@ -880,32 +912,30 @@ struct Flash : FlashCap<CAP, R> {
             step[0] /= limit; step[1] /= limit;
             const R previous = hi(ab(rv), ab(re));
             bool accepted = false;
-            if constexpr (WAVE) {
-                // lane j tries fraction 2^-j, the loop's j-th (fractions above 1e-9: j < 30)
-                const int lane = int(threadIdx.x & 63u);
-                const R fraction = R(::ldexp(1.0, -lane));
-                const Counts before = n;
-                E trial;
-                zeroEval(trial);
-                R pp = 0, tt = 0;
-                bool ok = false;
-                if (fraction > R(1e-9)) {
-                    pp = p * m_exp(fraction * step[0]);
-                    tt = T * m_exp(fraction * step[1]);
-                    if (evaluate(mass0, pp, tt, trial, false)) {
-                        const R next = hi(ab(trial.volume - R(1)), ab(trial.energy - energy) / scale);
-                        ok = next < previous * (R(1) - R(1e-4) * fraction) || next < lo(vtol, etol);
+            if constexpr (GROUP > 1) {
+                // fractions above 1e-9: 2^0 ... 2^-29, GROUP at a time
+                for (int first = 0; first < 30 && !accepted; first += GROUP) {
+                    const int index = lo(first + groupLane(), 29);
+                    const bool counted = first + groupLane() < 30;
+                    const R fraction = R(::ldexp(1.0, -index));
+                    const Counts before = n;
+                    const Memo entry = memoNow();
+                    E trial;
+                    zeroEval(trial);
+                    const R pp = p * m_exp(fraction * step[0]), tt = T * m_exp(fraction * step[1]);
+                    bool ok = evaluate(mass0, pp, tt, trial, false);
+                    const R next = hi(ab(trial.volume - R(1)), ab(trial.energy - energy) / scale);
+                    ok = ok && counted && (next < previous * (R(1) - R(1e-4) * fraction) || next < lo(vtol, etol));
+                    const unsigned won = groupBallot(ok);
+                    const int w = won ? __builtin_ctz(won) : GROUP - 1;
+                    groupCounts(before, entry, pp, tt, counted, w);
+                    if (won) {
+                        value = groupValue(trial, w);
+                        p = groupValue(pp, w);
+                        T = groupValue(tt, w);
+                        accepted = true;
+                        stalls = R(::ldexp(1.0, -(first + w))) < R(1) / R(32) ? stalls + 1 : 0;
                     }
-                }
-                const unsigned long long won = __ballot(ok);
-                waveCounts(before, won ? __ffsll(won) - 1 : 63);
-                if (won) {
-                    const int w = __ffsll(won) - 1;
-                    value = waveBroadcast(trial, w);
-                    p = waveBroadcast(pp, w);
-                    T = waveBroadcast(tt, w);
-                    accepted = true;
-                    stalls = R(::ldexp(1.0, -w)) < R(1) / R(32) ? stalls + 1 : 0;
                 }
             } else
             for (R fraction = 1; fraction > R(1e-9); fraction *= R(.5)) {
@@ -968,6 +998,7 @@ struct Flash : FlashCap<CAP, R> {
     // Central finite differences with step halving (reactiveDeviceFlash.h:338-373).
     RAMD_NOINLINE bool jacobian(const R* x, R scale, const R* f, R (&jac)[3][3]) {
         ++n.fd;
+        if constexpr (GROUP > 1) return jacobianGroup(x, scale, f, jac);
         for (int j = 0; j < 3; ++j) {
             R h = j < 2 ? R(P::hLog) : R(P::hFraction);
             bool success = false;
@@ -1010,6 +1041,86 @@ struct Flash : FlashCap<CAP, R> {
             if (!success) return false;
         }
         return true;
+    }
+    // The same differences with the six residuals of an attempt at once: lane
+    // 2 j + s evaluates column j's point at x_j + h (s = 0) or x_j - h.  A
+    // column that fails halves its step for the next attempt; the columns
+    // after one that fails for good are not counted, as the loop above does
+    // not reach them.
+    RD bool jacobianGroup(const R* x, R scale, const R* f, R (&jac)[3][3]) {
+        const int column = lo(groupLane() >> 1, 2);
+        const bool minusSide = groupLane() & 1;
+        bool done[3] = {false, false, false};
+        uint32_t phases[3] = {0, 0, 0}, residuals[3] = {0, 0, 0};
+        const Counts before = n;
+        R h[3] = {R(P::hLog), R(P::hLog), R(P::hFraction)};
+        for (int attempt = 0; attempt < 12 && !(done[0] && done[1] && done[2]); ++attempt) {
+            R xs[3], fs[3] = {};
+            for (int i = 0; i < 3; ++i) {
+                xs[i] = x[i];
+                if (i == column) {
+                    xs[i] = minusSide ? x[i] - h[i] : x[i] + h[i];
+                    if constexpr (CAP) {
+                        if (this->adaptive && xs[i] == x[i])  // a step lost to rounding moves by one ulp instead
+                            xs[i] = ::nextafter(x[i], minusSide ? -double(HUGE_VAL) : double(HUGE_VAL));
+                    }
+                }
+            }
+            const Counts start = n;
+            const Memo entry = memoNow();
+            const bool ok = residual(xs, scale, fs, nullptr);
+            const unsigned found = groupBallot(ok);
+            const unsigned misses = groupBallot(groupLane() < 6 && cacheStatus >= 0 && cacheP == m_exp(xs[0]) &&
+                                                cacheT == m_exp(xs[1]));
+            const Memo mine = memoNow();
+            const Memo left = groupValue(mine, misses ? 31 - __builtin_clz(misses) : 0);
+            memoSet(misses ? left : entry);
+            for (int j = 0; j < 3; ++j) {
+                const uint32_t p2 = groupSum(groupLane() >> 1 == j ? n.phases - start.phases : 0u);
+                const uint32_t r2 = groupSum(groupLane() >> 1 == j ? n.residuals - start.residuals : 0u);
+                const bool plus = found >> (2 * j) & 1u, minus = found >> (2 * j + 1) & 1u;
+                const R xp = groupValue(xs[j], 2 * j), xm = groupValue(xs[j], 2 * j + 1);
+                R fp[3], fm[3];
+                for (int i = 0; i < 3; ++i) {
+                    fp[i] = groupValue(fs[i], 2 * j);
+                    fm[i] = groupValue(fs[i], 2 * j + 1);
+                }
+                if (done[j]) continue;
+                phases[j] += p2;
+                residuals[j] += r2;
+                if (plus || minus) {
+                    bool success = true, weighted = false;
+                    if constexpr (CAP) weighted = this->adaptive;
+                    R maximum = 0;
+                    const R hp = xp - x[j], hm = x[j] - xm;
+                    for (int i = 0; i < 3; ++i) {
+                        R v;
+                        if (weighted)
+                            v = plus && minus ? (hm / (hp + hm)) * ((fp[i] - f[i]) / hp) +
+                                                    (hp / (hp + hm)) * ((f[i] - fm[i]) / hm)
+                                : plus ? (fp[i] - f[i]) / hp : (f[i] - fm[i]) / hm;
+                        else
+                            v = plus && minus ? (fp[i] - fm[i]) / (R(2) * h[j])
+                                : plus ? (fp[i] - f[i]) / h[j] : (f[i] - fm[i]) / h[j];
+                        jac[i][j] = v;
+                        maximum = hi(maximum, ab(v));
+                        success = success && fin(v);
+                    }
+                    done[j] = success && (!weighted || maximum > 0);
+                }
+                h[j] *= R(.5);
+            }
+        }
+        n = before;
+        bool reached = true;
+        for (int j = 0; j < 3; ++j) {
+            if (reached) {
+                n.phases += phases[j];
+                n.residuals += residuals[j];
+            }
+            reached = reached && done[j];
+        }
+        return reached;
     }
     // The reference's analytic Jacobian at a residual point
     // (reactiveDeviceFlash.h:338-352): from the point's own properties
@@ -1248,15 +1359,13 @@ struct Flash : FlashCap<CAP, R> {
             for (int j = 0; j < 3; ++j) step[j] /= limiter;
             bool accepted = false;
             const R previous = hi(hi(hi(R(0), ab(f[0])), ab(f[1])), ab(f[2]));
-            if constexpr (WAVE) {
+            if constexpr (GROUP > 1) {
                 const auto outsideAt = [vapourCoordinates](R y) {
                     return vapourCoordinates ? (!fin(y) || y > 0) : !(y >= 0 && y < 1);
                 };
-                // the loop evaluates the indices from `first` on: 0, or the
-                // end of the rejected prefix of the partition coordinate
-                // (bisected as below); lane j tries index first + j, and
-                // every lane evaluates (lanes past the loop's end repeat its
-                // last index and are not counted)
+                // the loop evaluates the indices from 0 on, or from the end
+                // of the rejected prefix of the partition coordinate
+                // (bisected as below)
                 int first = 0;
                 if (outsideAt(x[2] + step[2])) {
                     int lower = 0, upper = 30;
@@ -1268,28 +1377,28 @@ struct Flash : FlashCap<CAP, R> {
                     n.residuals += uint32_t(upper);
                     first = upper;
                 }
-                if (first < 30) {
-                    const int lane = int(threadIdx.x & 63u);
-                    const int index = first + lane < 30 ? first + lane : 29;
-                    const R fraction = R(::ldexp(1.0, -index));
+                for (; first < 30 && !accepted; first += GROUP) {
+                    const bool counted = first + groupLane() < 30;
+                    const R fraction = R(::ldexp(1.0, -lo(first + groupLane(), 29)));
                     const Counts before = n;
-                    R tx[3], tf[3];
+                    const Memo entry = memoNow();
+                    R tx[3], tf[3] = {};
                     for (int j = 0; j < 3; ++j) tx[j] = x[j] + fraction * step[j];
                     E trial;
                     zeroEval(trial);
                     const bool evaluated = residual(tx, scale, tf, &trial);
-                    const bool ok = first + lane < 30 && evaluated &&
+                    const bool ok = counted && evaluated &&
                                     hi(hi(hi(R(0), ab(tf[0])), ab(tf[1])), ab(tf[2])) <
                                         previous * (R(1) - R(1e-4) * fraction);
-                    const unsigned long long won = __ballot(ok);
-                    waveCounts(before, won ? __ffsll(won) - 1 : 29 - first);
+                    const unsigned won = groupBallot(ok);
+                    const int w = won ? __builtin_ctz(won) : GROUP - 1;
+                    groupCounts(before, entry, m_exp(tx[0]), m_exp(tx[1]), counted, w);
                     if (won) {
-                        const int w = __ffsll(won) - 1;
                         for (int j = 0; j < 3; ++j) {
-                            x[j] = waveBroadcast(tx[j], w);
-                            f[j] = waveBroadcast(tf[j], w);
+                            x[j] = groupValue(tx[j], w);
+                            f[j] = groupValue(tf[j], w);
                         }
-                        value = waveBroadcast(trial, w);
+                        value = groupValue(trial, w);
                         accepted = true;
                     }
                 }
@@ -1449,6 +1558,110 @@ struct Flash : FlashCap<CAP, R> {
             }
         return have;
     }
+    // The same search with the cell's starts on the eight groups of the wave
+    // (the gas and liquid solves on groups 0 and 1, the seeds on 2 to 6, the
+    // trace-vapour start on 7; then the restarts, eight at a time), selected
+    // and counted in the sequence's order.  Every lane of the wave calls it
+    // on the same cell and gets the result.
+    // firstRound 1: the restarts alone.
+    RAMD_NOINLINE bool searchGroups(E& best, int firstRound = 0) {
+        const int group = int(threadIdx.x & 63u) >> 3;
+        bool vapourCoordinates = false;
+        if constexpr (CAP) vapourCoordinates = this->adaptive;
+        const bool prunable = mod().stableGasPrune != 0 && !vapourCoordinates;
+        const int c = NL ? mod().condensable : 0;
+        R other = 0;
+        for (int k = 0; k < NS; ++k)
+            if (!NL || k != c) other += q[k];
+        const bool seeded = NL && q[c] > 0, frozenLiquid = NL && other == 0;
+        const Counts none = {0, 0, 0, 0, 0, 0, 0};
+        Counts total = n;
+        bool have = false, prune = false;
+        // The sequence's memo: a start whose first point it holds (the seeds
+        // all begin at one (p, T)) is spared its evaluation, and fails.
+        Memo memo = memoNow();
+        const auto seedAt = [](int j) { return j == 0 ? R(-1) : j == 1 ? R(.5) : j == 2 ? R(.95) : j == 3 ? R(.1) : R(.9999); };
+        for (int round = firstRound; round < 4; ++round) {
+            if (round == 1 && (have || !seeded || !restartRange())) break;
+            E candidate;
+            zeroEval(candidate);
+            bool ok = false;
+            n = none;
+            cacheStatus = -1;
+            const int start = round == 0 ? group : 8 * (round - 1) + group;  // restart index in the later rounds
+            const bool seedStart = round == 0 ? seeded && group >= 2 && (group < 7 || vapourCoordinates) : start < 20;
+            const bool frozenStart = round == 0 && (group == 0 || (group == 1 && frozenLiquid));
+            if (seedStart)
+                ok = activeFlash(round > 0 ? seedAt(start % 5) : group < 7 ? seedAt(group - 2) : R(-3), candidate, round > 0,
+                                 round > 0 ? restartTemperature(start / 5) : R(0));
+            R first[3] = {};
+            if (seedStart) {
+                R scale;
+                activeStart(R(.5), round > 0, round > 0 ? restartTemperature(start / 5) : R(0), first, scale);
+                first[0] = m_exp(first[0]);
+                first[1] = m_exp(first[1]);
+            } else {
+                first[0] = clamp(guessP, pmin, pmax);
+                first[1] = clamp(guessT, Tmin, Tmax);
+            }
+            if (frozenStart) ok = frozen(group == 0 ? R(0) : q[c], candidate, group == 0 && prunable ? 4 : 0);
+            const bool gas = candidate.gasMass > 0;
+            bool good = false;
+            if (ok) good = stable(candidate);
+            const bool took = seedStart || frozenStart;
+            const Memo mine = memoNow();
+            int winner = -1;
+            R entropy = have ? best.entropyDensity : R(0);
+            for (int g = 0; g < 8; ++g) {  // in the sequence's order
+                const Counts m = waveBroadcast(n, 8 * g);
+                const uint32_t bits = uint32_t(__shfl(int(uint32_t(took) | uint32_t(ok) << 1 | uint32_t(good) << 2 |
+                                                          uint32_t(seedStart) << 3 | uint32_t(gas) << 4), 8 * g, 64));
+                const Memo after = waveBroadcast(mine, 8 * g);
+                const R p0 = waveBroadcast(first[0], 8 * g), T0 = waveBroadcast(first[1], 8 * g);
+                const R s = waveBroadcast(candidate.entropyDensity, 8 * g);
+                if (!(bits & 1u) || (prune && g >= 2)) continue;
+                const bool seedG = (bits & 8u) != 0;
+                const bool spared = memo.status >= 0 && memo.p == p0 && memo.T == T0 &&
+                                    (memo.virtualLiquids != 0) == seedG && (seedG || g == 1);
+                total.phases += spared ? 0u : m.phases;
+                total.residuals += m.residuals;
+                total.candidates += m.candidates;
+                total.fd += m.fd;
+                total.analytic += m.analytic;
+                if (!spared && after.status >= 0) memo = after;
+                if ((bits & 6u) == 6u) {
+                    ++total.stable;
+                    if (!have || s > entropy) { have = true; entropy = s; winner = g; }
+                } else {
+                    ++total.failures;
+                }
+                if (g == 0 && round == 0) prune = prunable && (bits & 6u) == 6u && (bits & 16u);
+            }
+            if (winner >= 0) best = waveBroadcast(candidate, 8 * winner);
+        }
+        n = total;
+        memoSet(memo);
+        return have;
+    }
+    RD bool searchRestarts(E& best) {
+        if constexpr (GROUP > 1) {
+            return searchGroups(best, 1);
+        } else {
+            const R seeds[5] = {R(-1), R(.5), R(.95), R(.1), R(.9999)};
+            bool have = false;
+            E candidate;
+            for (int t = 0; t < 4; ++t)
+                for (int j = 0; j < 5; ++j) {
+                    if (activeFlash(seeds[j], candidate, true, restartTemperature(t))) consider(candidate, best, have);
+                    else ++n.failures;
+                }
+            return have;
+        }
+    }
+    RD bool searchAny(E& best) {
+        if constexpr (GROUP > 1) return searchGroups(best);
+        else return search(best);
+    }
     // :544-560.  CAP: with boundaryRecovery, or for a capillary equilibrium
     // cell (capillaryBoundary), a result whose liquid holds nearly all of the
     // condensable with gas present, or no result, runs the search again in
@@ -1458,11 +1671,11 @@ struct Flash : FlashCap<CAP, R> {
         for (int k = 0; k < NS; ++k)
             if (!fin(q[k]) || q[k] < 0) return false;
         if constexpr (!CAP) {
-            return search(result);
+            return searchAny(result);
         } else {
             E reference;
             zeroEval(reference);
-            const bool have = search(reference);
+            const bool have = searchAny(reference);
             if (!mod().boundaryRecovery && !capillaryBoundary) {
                 if (have) result = reference;
                 return have;
@@ -1478,7 +1691,7 @@ struct Flash : FlashCap<CAP, R> {
             this->adaptive = true;
             E recovered;
             zeroEval(recovered);
-            const bool found = search(recovered);
+            const bool found = searchAny(recovered);
             this->adaptive = false;
             if (!found && !have) return false;
             result = have && (!found || reference.entropyDensity >= recovered.entropyDensity) ? reference : recovered;
@@ -1701,7 +1914,7 @@ struct Flash : FlashCap<CAP, R> {
         if (ok && value.active == best.active) best = value;
     }
     RAMD_NOINLINE bool searchPolished(E& best) {
-        if (!search(best)) return false;
+        if (!searchAny(best)) return false;
         polishBest(best);
         return true;
     }
@@ -1777,13 +1990,7 @@ struct Flash : FlashCap<CAP, R> {
                 if (deferred) { *deferred = true; return false; }
                 // the single-precision search found a stable candidate that FP64
                 // rejects: search the restart temperatures in FP64
-                const R seeds[5] = {R(-1), R(.5), R(.95), R(.1), R(.9999)};
-                for (int t = 0; t < 4; ++t)
-                    for (int j = 0; j < 5; ++j) {
-                        if (activeFlash(seeds[j], candidate, true, restartTemperature(t)))
-                            consider(candidate, best, have);
-                        else ++n.failures;
-                    }
+                have = searchRestarts(best);
                 if (have) polishBest(best);
             } else {
                 for (; i < set.count; ++i) {

@@ -4,6 +4,7 @@
 #ifndef REACTIVE_AMD_FLASH_STEP_H
 #define REACTIVE_AMD_FLASH_STEP_H
 #include <hip/hip_runtime.h>
+#include <cstring>
 #include "hip_common.h"
 #include "flash_device.h"
 
@@ -20,24 +21,18 @@
 #ifndef RAMD_REFINE_MIN_WAVES
 #define RAMD_REFINE_MIN_WAVES 2
 #endif
-// Persistent grid of the queue kernels (the step's and the HEM ABI's mixed
-// flash): 4096 single-wave workgroups (sixteen
-// per CU, more than stay resident, so a wave that finishes its cell is
-// replaced at once) take up to 4096 deferred cells per round one cell per
-// wave, or 262,144 one cell per lane; workgroups beyond the queue leave at
-// once.  Against 1024: 160^3 pure N2O step 135.8 -> 132.5 ms (2,537 deferred
-// cells per flash), binary N2O/N2 96^3 2242 -> 1788 ms, bit for bit the same.
+// Persistent grid of the deferred queue, in single-wave workgroups that take
+// one cell at a time: sixteen per CU, more than stay resident, so that a wave
+// that finishes its cell is replaced at once.  (Against 1024: 160^3 pure N2O
+// step 135.8 -> 132.5 ms with 2,537 deferred cells per flash, binary N2O/N2
+// 96^3 2242 -> 1788 ms, when a flash deferred that many.)
 #ifndef RAMD_QUEUE_BLOCKS
 #define RAMD_QUEUE_BLOCKS 4096
 #endif
-// Deferred refinements up to this many per flash run one cell per wave with
-// the Newton line searches spread over its lanes (the flash's WAVE mode);
-// more run one cell per lane.  Measured on the step's 4096-wave queue grid:
-// one cell per wave takes a binary N2O/N2 160^3 step (75k deferred cells per
-// flash) from 6.51 to 4.85 s; on a 1024-wave grid it had been slower there
-// (6.74 -> 7.18 s) and faster at 96^3 (16k cells, 4.55 -> 2.23 s).
-#ifndef RAMD_WAVE_QUEUE_CELLS
-#define RAMD_WAVE_QUEUE_CELLS 131072
+// FP64 batches of up to this many cells run one cell per wave, its starts on
+// groups of eight lanes (group.hip); larger ones one cell per lane.
+#ifndef RAMD_GROUP_CELLS
+#define RAMD_GROUP_CELLS 65536
 #endif
 
 namespace ramd {
@@ -128,8 +123,8 @@ struct CellList {
 // Commits a flash result, or keeps the step-start state of a failed cell
 // (the reference commits nothing for it); p, c_frozen and rho go to the SoA
 // arrays the next transport stage reads.
-template <bool A, bool RJ>
-__device__ inline void storeCell(bool ok, const EvalT<double, A, RJ>& result, const ThermoOut& g, uint32_t c,
+template <bool A, bool RJ, bool C>
+__device__ inline void storeCell(bool ok, const EvalT<double, A, RJ, C>& result, const ThermoOut& g, uint32_t c,
                                  ThermoOut* __restrict__ out, double* __restrict__ pOut, double* __restrict__ cOut,
                                  double* __restrict__ rOut) {
     if (ok) {
@@ -145,6 +140,65 @@ __device__ inline void storeCell(bool ok, const EvalT<double, A, RJ>& result, co
     }
 }
 
+// Flash output record, byte-compatible with ReactiveGpuHemOutputV1 (184 B).
+struct HemOutputDev {
+    ThermoOut state;
+    int success, reserved;
+};
+// Per-cell capillary input, byte-compatible with ReactiveGpuHemCapillaryInputV2
+// (24 B): the interface's color and pressure jump, and equilibrium 1 for the
+// UV equilibrium with the boundary search, 0 for the frozen inventory.
+struct HemCapillaryDev {
+    double color, pressureJump;
+    int equilibrium, pad;
+};
+// A flash result into the batch's output record (zero state where it failed).
+template <class E>
+__device__ inline void storeHemCell(bool ok, const E& result, HemOutputDev& o) {
+    if (ok) writeOut(result, o.state);
+    else std::memset(&o.state, 0, sizeof(o.state));
+    o.success = ok ? 1 : 0;
+    o.reserved = 0;
+}
+// Adds one wavefront's work counters (phases, residuals, candidates, stable,
+// failures, fd Jacobians, successes, analytic Jacobians) to totals: one
+// 64-bit atomic per counter per wavefront.
+__device__ inline void addTotals(const Counts& n, uint32_t succeeded, unsigned long long* __restrict__ totals) {
+    const uint32_t s0 = waveSum(n.phases), s1 = waveSum(n.residuals), s2 = waveSum(n.candidates);
+    const uint32_t s3 = waveSum(n.stable), s4 = waveSum(n.failures), s5 = waveSum(n.fd);
+    const uint32_t s6 = waveSum(succeeded), s7 = waveSum(n.analytic);
+    if ((threadIdx.x & 63) == 0) {
+        atomicAdd(&totals[0], (unsigned long long)s0);
+        atomicAdd(&totals[1], (unsigned long long)s1);
+        atomicAdd(&totals[2], (unsigned long long)s2);
+        atomicAdd(&totals[3], (unsigned long long)s3);
+        atomicAdd(&totals[4], (unsigned long long)s4);
+        atomicAdd(&totals[5], (unsigned long long)s5);
+        atomicAdd(&totals[6], (unsigned long long)s6);
+        atomicAdd(&totals[7], (unsigned long long)s7);
+    }
+}
+// One cell of a HEM batch by flash f (g: its seed, x: its capillary input or
+// null).  Without capillary input the equilibrium UV flash (recover,
+// reactiveDeviceFlash.h:564-567).  With it (recoverCapillary, :572-590) the
+// cell's interface (color, pressure jump) held during the solve, then the UV
+// equilibrium with the boundary search (equilibrium = 1) or the frozen
+// inventory at the seed's liquid masses (0); a cell whose color or jump the
+// reference rejects (its status 2) fails.
+template <bool CAP, int NL, class F>
+__device__ inline bool runHemCell(F& f, const ThermoOut& g, const HemCapillaryDev* x, typename F::E& result) {
+    if (!x) return f.run(result);
+    if constexpr (CAP) {
+        if (!fin(x->color) || x->color < 0 || x->color > 1 || !fin(x->pressureJump) ||
+            (x->pressureJump != 0 && NL != 1))
+            return false;
+        f.color = x->color;
+        f.jump = x->pressureJump;
+        if (x->equilibrium != 0) return f.run(result, true);
+    }
+    return f.frozen(NL ? g.liquidMass[0] : 0.0, result, 0, g.liquidMass[1]);
+}
+
 __device__ inline void countFlash(uint32_t failed, uint32_t phases, unsigned long long* __restrict__ counters) {
     const uint32_t sumFailed = waveSum(failed), sumPhases = waveSum(phases);
     if ((threadIdx.x & 63) == 0) {
@@ -152,6 +206,27 @@ __device__ inline void countFlash(uint32_t failed, uint32_t phases, unsigned lon
         atomicAdd(&counters[1], (unsigned long long)sumPhases);
     }
 }
+
+// ---- one cell per wave (group.hip) -----------------------------------------
+// Where a cell's result and counts go: a HEM batch's records and totals (or a
+// slot of eight sums per workgroup in partials), or the step's arrays.
+struct FlashSink {
+    HemOutputDev* hem;
+    unsigned long long *totals, *partials;
+    ThermoOut* out;
+    double *p, *c, *r;
+    uint16_t* cost;
+    unsigned long long* counters;
+    uint8_t* failMark;
+};
+// FP64 flash of the cells in `order` (null: 0 .. count - 1); capillary (may be
+// null) by cell; analytic, boundary: the model's modes.
+void launchGroupFlash(int ns, int nl, bool analytic, bool boundary, const void* model, const FlashCells& cells,
+                      const uint32_t* order, uint32_t count, const HemCapillaryDev* capillary, const FlashSink& sink,
+                      hipStream_t stream);
+// The deferred cells of the mixed flash: refined again without deferral.
+void launchRefineQueue(int ns, int nl, const void* model, const FlashCells& cells, const uint32_t* queue,
+                       const unsigned* queueCount, const CandidateSet* sets, const FlashSink& sink, hipStream_t stream);
 
 // ---- candidates of the mixed flash (search.hip) ---------------------------
 // One start's outcome: the point, kStart* bits and the evaluations above them.

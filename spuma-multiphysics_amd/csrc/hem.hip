@@ -37,51 +37,15 @@ static_assert(sizeof(HemOutputDev) == sizeof(ReactiveGpuHemOutputV1) &&
                   offsetof(HemOutputDev, success) == offsetof(ReactiveGpuHemOutputV1, success),
               "output layout");
 
-// Adds one wavefront's work counters (phases, residuals, candidates, stable,
-// failures, fd Jacobians, successes, analytic Jacobians) to totals: one
-// 64-bit atomic per counter per wavefront.
-__device__ inline void addTotals(const Counts& n, uint32_t succeeded, unsigned long long* __restrict__ totals) {
-    const uint32_t s0 = waveSum(n.phases), s1 = waveSum(n.residuals), s2 = waveSum(n.candidates);
-    const uint32_t s3 = waveSum(n.stable), s4 = waveSum(n.failures), s5 = waveSum(n.fd);
-    const uint32_t s6 = waveSum(succeeded), s7 = waveSum(n.analytic);
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&totals[0], (unsigned long long)s0);
-        atomicAdd(&totals[1], (unsigned long long)s1);
-        atomicAdd(&totals[2], (unsigned long long)s2);
-        atomicAdd(&totals[3], (unsigned long long)s3);
-        atomicAdd(&totals[4], (unsigned long long)s4);
-        atomicAdd(&totals[5], (unsigned long long)s5);
-        atomicAdd(&totals[6], (unsigned long long)s6);
-        atomicAdd(&totals[7], (unsigned long long)s7);
-    }
-}
-
-// A flash result into the batch's output record (zero state where it failed).
-template <class E>
-__device__ inline void storeHemCell(bool ok, const E& result, HemOutputDev& o) {
-    if (ok) writeOut(result, o.state);
-    else std::memset(&o.state, 0, sizeof(o.state));
-    o.success = ok ? 1 : 0;
-    o.reserved = 0;
-}
-
-// Without capillary input: equilibrium UV flash (recover,
-// reactiveDeviceFlash.h:564-567).  With it (recoverCapillary, :572-590): the
-// cell's interface (color, pressure jump) held during the solve, then the
-// UV equilibrium with the boundary search (equilibrium = 1) or the frozen
-// inventory at the seed's liquid masses (0); a cell whose color or jump the
-// reference rejects (its status 2) fails.  RJ: the model's analytic-Jacobian
-// mode (analyticJacobian = 1); CAP: the capillary / boundary-search flash,
-// for capillary input and boundaryRecovery models.
+// One cell per lane (runHemCell).  RJ: the model's analytic-Jacobian mode
+// (analyticJacobian = 1); CAP: the capillary / boundary-search flash, for
+// capillary input and boundaryRecovery models.
 template <int NS, int NL, bool RJ, bool CAP>
 __global__ __launch_bounds__(64, RAMD_FLASH_MIN_WAVES) void hemFlashKernel(const HemModel<NS>* __restrict__ globalModel,
-                                                     const double* __restrict__ q, const double* __restrict__ energy,
-                                                     const ThermoOut* __restrict__ guess,
-                                                     const uint32_t* __restrict__ order, uint32_t count,
+                                                     FlashCells cells, const uint32_t* __restrict__ order, uint32_t count,
                                                      const HemCapillaryDev* __restrict__ capillary,
                                                      HemOutputDev* __restrict__ out,
                                                      unsigned long long* __restrict__ totals,
-                                                     uint32_t* __restrict__ cellPhases,
                                                      unsigned long long* __restrict__ partials) {
     const HemModel<NS>& model = workgroupModel(globalModel);
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -91,36 +55,12 @@ __global__ __launch_bounds__(64, RAMD_FLASH_MIN_WAVES) void hemFlashKernel(const
         const uint32_t c = order ? order[i] : i;
         using F = Flash<NS, NL, double, false, RJ, CAP, kModelLds>;
         F f(model, n);
-        for (int k = 0; k < NS; ++k) f.q[k] = q[size_t(c) * NS + k];
-        f.energy = energy[c];
-        const ThermoOut& g = guess[c];
-        f.guessP = g.p;
-        f.guessT = g.T;
-        f.guessLiquid = g.liquidMass[0];
+        cells.load<NS>(f, c);
         typename F::E result;
         zeroEval(result);
-        bool ok;
-        if (capillary) {
-            const HemCapillaryDev& x = capillary[c];
-            if constexpr (CAP) {
-                if (!fin(x.color) || x.color < 0 || x.color > 1 || !fin(x.pressureJump) ||
-                    (x.pressureJump != 0 && NL != 1)) {
-                    ok = false;
-                } else {
-                    f.color = x.color;
-                    f.jump = x.pressureJump;
-                    ok = x.equilibrium != 0 ? f.run(result, true)
-                                            : f.frozen(NL ? g.liquidMass[0] : 0.0, result, 0, g.liquidMass[1]);
-                }
-            } else {
-                ok = f.frozen(NL ? g.liquidMass[0] : 0.0, result, 0, g.liquidMass[1]);
-            }
-        } else {
-            ok = f.run(result);
-        }
+        const bool ok = runHemCell<CAP, NL>(f, cells.seeds[c], capillary ? capillary + c : nullptr, result);
         storeHemCell(ok, result, out[c]);
         succeeded = ok ? 1u : 0u;
-        if (cellPhases) cellPhases[c] = n.phases;
     }
     if (partials) {  // one 64-lane workgroup: its eight sums go to its own slot
         const uint32_t s0 = waveSum(n.phases), s1 = waveSum(n.residuals), s2 = waveSum(n.candidates);
@@ -172,50 +112,6 @@ __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineKernel(con
     addTotals(n, succeeded, totals);
 }
 
-// The deferred cells, refined without deferral by a persistent grid of
-// single-wave workgroups: one queued cell per wave at a time with its line
-// searches spread over the lanes (the flash's WAVE mode) while the queue is
-// short, one cell per lane for a long queue (RAMD_WAVE_QUEUE_CELLS; the count
-// is read on the device).
-template <int NS, int NL, bool WAVE>
-__device__ inline void hemRefineQueued(const HemModel<NS>& model, const FlashCells& cells, uint32_t c,
-                                       const CandidateSet& set, bool lead, HemOutputDev* __restrict__ out,
-                                       unsigned long long* __restrict__ totals) {
-    Counts n = {0, 0, 0, 0, 0, 0, 0};
-    Flash<NS, NL, double, true, false, false, kModelLds, WAVE> f(model, n);
-    cells.load<NS>(f, c);
-    EvalT<double, true> result;
-    zeroEval(result);
-    const bool ok = f.refine(set, result);
-    if (lead) storeHemCell(ok, result, out[c]);
-    const Counts none = {0, 0, 0, 0, 0, 0, 0};
-    addTotals(lead ? n : none, lead && ok ? 1u : 0u, totals);
-}
-template <int NS, int NL>
-__global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineQueueKernel(
-    const HemModel<NS>* __restrict__ globalModel, FlashCells cells, const uint32_t* __restrict__ queue,
-    const unsigned* __restrict__ queueCount, const CandidateSet* __restrict__ sets, HemOutputDev* __restrict__ out,
-    unsigned long long* __restrict__ totals) {
-    const unsigned count = *queueCount;
-    const bool perWave = count <= RAMD_WAVE_QUEUE_CELLS;  // uniform
-    if (blockIdx.x * (perWave ? 1u : 64u) >= count) return;  // uniform per workgroup
-    const HemModel<NS>& model = workgroupModel(globalModel);
-    if (perWave) {
-        for (unsigned i = blockIdx.x; i < count; i += gridDim.x)  // uniform per workgroup
-            hemRefineQueued<NS, NL, true>(model, cells, queue[i], sets[queue[i]], threadIdx.x == 0, out, totals);
-    } else {
-        for (unsigned base = blockIdx.x * 64u; base < count; base += gridDim.x * 64u) {  // uniform per workgroup
-            const unsigned i = base + threadIdx.x;
-            if (i < count) {
-                hemRefineQueued<NS, NL, false>(model, cells, queue[i], sets[queue[i]], true, out, totals);
-            } else {
-                const Counts none = {0, 0, 0, 0, 0, 0, 0};
-                addTotals(none, 0u, totals);
-            }
-        }
-    }
-}
-
 // deferred cells, cells to search, cells to restart, cells the directed search tries again
 __global__ void clearCountsKernel(unsigned* __restrict__ counts) {
     if (threadIdx.x < 4) counts[threadIdx.x] = 0;
@@ -240,9 +136,6 @@ __global__ void zeroTotalsKernel(unsigned long long* totals, int n) {
 __global__ void queueCountKernel(const unsigned* __restrict__ count, unsigned long long* __restrict__ total) {
     if (threadIdx.x == 0) *total = *count;
 }
-
-// Workgroups of the persistent deferred-refinement grid (64 lanes each).
-constexpr unsigned kQueueBlocks = RAMD_QUEUE_BLOCKS;
 
 // Scheduling key (reactiveHemBucket.h:13-18).
 inline unsigned bucketKey(const double* q, int ns, int activeLiquids) {
@@ -284,16 +177,25 @@ void HemHandle::ensureHostPath() {
     hostReady = true;
 }
 
-void HemHandle::launch(const double* q, const double* e, const ThermoOut* g, const uint32_t* order, size_t count,
-                       const HemCapillaryDev* capillary, HemOutputDev* out, uint32_t* cellPhases, hipStream_t s,
-                       unsigned long long* partials) {
-    if (!count) return;
+unsigned HemHandle::launch(const double* q, const double* e, const ThermoOut* g, const uint32_t* order, size_t count,
+                           const HemCapillaryDev* capillary, HemOutputDev* out, hipStream_t s,
+                           unsigned long long* partials, unsigned slots) {
+    if (!count) return 0;
     const unsigned blocks = unsigned((count + 63) / 64);
     if (!partials) hipLaunchKernelGGL(zeroTotalsKernel, dim3(1), dim3(64), 0, s, totals, 8);
+    const FlashCells cells = {q, 0, e, g, nullptr, nullptr};
+    if (count <= RAMD_GROUP_CELLS && (!partials || count <= slots)) {
+        FlashSink sink = {};
+        sink.hem = out;
+        sink.totals = totals;
+        sink.partials = partials;
+        launchGroupFlash(ns, nl, analytic, boundary, model, cells, order, uint32_t(count), capillary, sink, s);
+        return unsigned(count);
+    }
 #define RAMD_HEM_LAUNCH(NS_, NL_, RJ_, CAP_)                                                                       \
     hipLaunchKernelGGL((hemFlashKernel<NS_, NL_, RJ_, CAP_>), dim3(blocks), dim3(64), 0, s,                        \
-                       static_cast<const HemModel<NS_>*>(model), q, e, g, order, uint32_t(count), capillary, out, totals, \
-                       cellPhases, partials)
+                       static_cast<const HemModel<NS_>*>(model), cells, order, uint32_t(count), capillary, out,    \
+                       totals, partials)
 #define RAMD_HEM_SPECIES(CAP_)                                                                                    \
     if (ns == 1 && nl == 0) RAMD_HEM_LAUNCH(1, 0, false, CAP_);                                                   \
     else if (ns == 1 && !analytic) RAMD_HEM_LAUNCH(1, 1, false, CAP_);                                            \
@@ -307,6 +209,7 @@ void HemHandle::launch(const double* q, const double* e, const ThermoOut* g, con
 #undef RAMD_HEM_SPECIES
 #undef RAMD_HEM_LAUNCH
     RAMD_HIP(hipGetLastError());
+    return blocks;
 }
 
 void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g, const uint32_t* order,
@@ -346,14 +249,16 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
         hipLaunchKernelGGL((hemRefineKernel<NS_, NL_>), dim3(std::min(2048u, blocks)), dim3(64), 0, s,              \
                            static_cast<const HemModel<NS_>*>(model), cells, left, sets, out, totals, queue,       \
                            queueCount, searchList, queueCount + 1);                                               \
-    }                                                                                                             \
-    hipLaunchKernelGGL((hemRefineQueueKernel<NS_, NL_>), dim3(kQueueBlocks), dim3(64), 0, s,                        \
-                       static_cast<const HemModel<NS_>*>(model), cells, queue, queueCount, sets, out, totals)
+    }
     if (ns == 1 && nl == 0) { RAMD_HEM_MIXED(1, 0); }
     else if (ns == 1) { RAMD_HEM_MIXED(1, 1); }
     else if (nl == 0) { RAMD_HEM_MIXED(2, 0); }
     else { RAMD_HEM_MIXED(2, 1); }
 #undef RAMD_HEM_MIXED
+    FlashSink sink = {};
+    sink.hem = out;
+    sink.totals = totals;
+    launchRefineQueue(ns, nl, model, cells, queue, queueCount, sets, sink, s);
     hipLaunchKernelGGL(queueCountKernel, dim3(1), dim3(64), 0, s, queueCount, totals + 9);
     RAMD_HIP(hipGetLastError());
 }
@@ -452,7 +357,7 @@ int runHost(HemHandle* h, const double* q, const double* energy, const ReactiveG
     // the mixed arithmetic runs the equilibrium flash without the boundary search
     const bool mixed = !capillary && !h->boundary && h->arithmetic == REACTIVE_AMD_FLASH_MIXED;
     if (mixed) h->launchMixed(h->dq, h->de, h->dguess, h->dorder, count, h->dout, s);
-    else h->launch(h->dq, h->de, h->dguess, h->dorder, count, capillary ? h->dcap : nullptr, h->dout, nullptr, s);
+    else h->launch(h->dq, h->de, h->dguess, h->dorder, count, capillary ? h->dcap : nullptr, h->dout, s);
     RAMD_HIP(hipEventRecord(h->events[2], s));
     RAMD_HIP(hipMemcpyAsync(h->hostOut.data(), h->dout, count * sizeof(HemOutputDev), hipMemcpyDeviceToHost, s));
     unsigned long long totals[10] = {};
@@ -626,7 +531,7 @@ int reactive_gpu_hem_run_resident_v1(void* raw, const double* q, const double* e
         const auto* cap = reinterpret_cast<const HemCapillaryDev*>(capillary);
         RAMD_HIP(hipEventRecord(h->events[0], s));
         h->launch(q, energy, reinterpret_cast<const ThermoOut*>(seed), order, count, cap,
-                  reinterpret_cast<HemOutputDev*>(output), nullptr, s);
+                  reinterpret_cast<HemOutputDev*>(output), s);
         RAMD_HIP(hipEventRecord(h->events[1], s));
         unsigned long long totals[8] = {};
         RAMD_HIP(hipMemcpyAsync(totals, h->totals, sizeof(totals), hipMemcpyDeviceToHost, s));
@@ -681,11 +586,10 @@ int reactive_gpu_hem_run_resident_noalloc_v1(void* raw, const double* q, const d
         unsigned long long* partials = scratchAddress(h->device);
         unsigned long long* totalsDev = partials + size_t(kNoAllocBlocks) * 8;
         hipStream_t s = h->stream;
-        const unsigned blocks = unsigned((count + 63) / 64);
         const auto* cap = reinterpret_cast<const HemCapillaryDev*>(capillary);
         RAMD_HIP(hipEventRecord(h->events[0], s));
-        h->launch(q, energy, reinterpret_cast<const ThermoOut*>(seed), order, count, cap,
-                  reinterpret_cast<HemOutputDev*>(output), nullptr, s, partials);
+        const unsigned blocks = h->launch(q, energy, reinterpret_cast<const ThermoOut*>(seed), order, count, cap,
+                                          reinterpret_cast<HemOutputDev*>(output), s, partials, kNoAllocBlocks);
         hipLaunchKernelGGL(reducePartialsKernel, dim3(1), dim3(64), 0, s, partials, blocks, 8, totalsDev);
         RAMD_HIP(hipGetLastError());
         RAMD_HIP(hipEventRecord(h->events[1], s));

@@ -10,20 +10,6 @@
 
 namespace ramd {
 
-// Flash output record, byte-compatible with ReactiveGpuHemOutputV1 (184 B).
-struct HemOutputDev {
-    ThermoOut state;
-    int success, reserved;
-};
-
-// Per-cell capillary input, byte-compatible with ReactiveGpuHemCapillaryInputV2
-// (24 B): the interface's color and pressure jump, and equilibrium 1 for the
-// UV equilibrium with the boundary search, 0 for the frozen inventory.
-struct HemCapillaryDev {
-    double color, pressureJump;
-    int equilibrium, pad;
-};
-
 struct HemHandle {
     int ns = 0, nl = 0, device = 0;
     bool analytic = false;  // the model's analytic-Jacobian mode (FP64 flash)
@@ -68,11 +54,12 @@ struct HemHandle {
     // guess, capillary and out are indexed by cell.  Totals: phases,
     // residuals, candidates, stable, failures, fd Jacobians, successes,
     // analytic Jacobians.
-    // With partials (one slot of 8 counters per 64-cell workgroup), the
+    // With partials (slots of 8 counters, at least one per 64 cells), the
     // workgroups write their sums there instead of adding them to totals.
-    void launch(const double* q, const double* e, const ThermoOut* guess, const uint32_t* order, size_t count,
-                const HemCapillaryDev* capillary, HemOutputDev* out, uint32_t* cellPhases, hipStream_t s,
-                unsigned long long* partials = nullptr);
+    // Returns the workgroups launched.
+    unsigned launch(const double* q, const double* e, const ThermoOut* guess, const uint32_t* order, size_t count,
+                    const HemCapillaryDev* capillary, HemOutputDev* out, hipStream_t s,
+                    unsigned long long* partials = nullptr, unsigned slots = 0);
     // The equilibrium flash of the same cells in mixed arithmetic: FP32
     // candidate search, FP64 refinement and the deferred queue; totals as
     // launch's plus totals[8] FP32 phases and totals[9] deferred cells.

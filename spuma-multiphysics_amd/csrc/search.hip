@@ -363,11 +363,6 @@ __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void directKernel(
     uint32_t bits = 0;
     float x[3];
     if (start >= 2) bits = f.searchSeed(start, x);
-    // The two kinds of start are separate passes of the whole wave: as the
-    // two sides of one branch, the compiler may keep scalar registers that a
-    // call on one side saves (a store of all 64 lanes) in the stack slot of a
-    // value that only the other side's lanes still need.
-    asm volatile("" : "+v"(start), "+v"(bits));
     if (start == 0 || start == 1) bits = f.searchFrozen(start == 1, x);
     if (!(bits & kStartFound)) {
         set.count = 0;

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256, RAMD_REFINE_MIN_WAVES) void stepRefineKernel(c
         EvalT<double, true> result;
         zeroEval(result);
         bool deferred = false;
-        const bool ok = f.refine(sets[c], result, queue ? &deferred : nullptr);
+        const bool ok = f.refine(sets[c], result, &deferred);
         if (deferred) {
             if (sets[c].flags & kDirect) search[atomicAdd(searchCount, 1u)] = c;
             else queue[atomicAdd(queueCount, 1u)] = c;
@@ -114,66 +114,6 @@ __global__ __launch_bounds__(256, RAMD_REFINE_MIN_WAVES) void stepRefineKernel(c
     countFlash(failed, phases, counters);
 }
 
-// One deferred cell refined without deferral; lead: this lane stores it.
-template <int NS, int NL, bool WAVE>
-__device__ inline void refineQueued(const HemModel<NS>& model, const FlashCells& cells, uint32_t c,
-                                    const CandidateSet& set, bool lead, ThermoOut* __restrict__ out,
-                                    double* __restrict__ pOut, double* __restrict__ cOut, double* __restrict__ rOut,
-                                    uint16_t* __restrict__ cost, uint8_t* __restrict__ failMark, Counts& n,
-                                    uint32_t& failed) {
-    Flash<NS, NL, double, true, false, false, kModelLds, WAVE> f(model, n);
-    cells.load<NS>(f, c);
-    EvalT<double, true> result;
-    zeroEval(result);
-    const bool ok = f.refine(set, result);
-    if (lead) {
-        storeCell(ok, result, cells.seeds[c], c, out, pOut, cOut, rOut);
-        if (!ok && failMark) failMark[c] = 1;
-        if (cost) cost[c] = uint16_t(n.phases < 65535u ? n.phases : 65535u);
-        failed = ok ? 0u : 1u;
-    }
-}
-
-// The cells the refinement deferred (full FP64 search, FP64 restarts, or a
-// frozen candidate's solve from the cell's guess), refined again without
-// deferral by a persistent grid of single-wave workgroups: one queued cell
-// per wave at a time (every lane on the cell, its line searches spread over
-// the lanes) while the queue is short, so that the few long refinements
-// neither share a wave nor halve their steps one evaluation at a time; one
-// cell per lane for a long queue.  queueCount is read on the device (the
-// launch does not depend on it).
-template <int NS, int NL>
-__global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void stepRefineQueueKernel(
-    const HemModel<NS>* __restrict__ globalModel, FlashCells cells, const uint32_t* __restrict__ queue,
-    const unsigned* __restrict__ queueCount, const CandidateSet* __restrict__ sets, ThermoOut* __restrict__ out,
-    double* __restrict__ pOut, double* __restrict__ cOut, double* __restrict__ rOut, uint16_t* __restrict__ cost,
-    unsigned long long* __restrict__ counters, uint8_t* __restrict__ failMark) {
-    const unsigned count = *queueCount;
-    const bool perWave = count <= RAMD_WAVE_QUEUE_CELLS;  // uniform
-    if (blockIdx.x * (perWave ? 1u : 64u) >= count) return;  // uniform per workgroup: usually every workgroup leaves here
-    const HemModel<NS>& model = workgroupModel(globalModel);
-    if (perWave) {
-        const bool lead = threadIdx.x == 0;
-        for (unsigned i = blockIdx.x; i < count; i += gridDim.x) {  // uniform per workgroup
-            Counts n = {0, 0, 0, 0, 0, 0, 0};
-            uint32_t failed = 0;
-            if (!cells.gate || *cells.gate > 0)
-                refineQueued<NS, NL, true>(model, cells, queue[i], sets[queue[i]], lead, out, pOut, cOut, rOut, cost,
-                                           failMark, n, failed);
-            countFlash(failed, lead ? n.phases : 0u, counters);
-        }
-    } else {
-        for (unsigned base = blockIdx.x * 64u; base < count; base += gridDim.x * 64u) {  // uniform per workgroup
-            const unsigned i = base + threadIdx.x;
-            Counts n = {0, 0, 0, 0, 0, 0, 0};
-            uint32_t failed = 0;
-            if (i < count && (!cells.gate || *cells.gate > 0))
-                refineQueued<NS, NL, false>(model, cells, queue[i], sets[queue[i]], true, out, pOut, cOut, rOut, cost,
-                                            failMark, n, failed);
-            countFlash(failed, n.phases, counters);
-        }
-    }
-}
 __global__ void clearQueueKernel(unsigned* __restrict__ counts) {
     if (threadIdx.x < kQueueCounts) counts[threadIdx.x] = 0;
 }
@@ -640,11 +580,6 @@ __global__ void copyFixedKernel(const double* __restrict__ tq, const ReactiveTra
 }
 
 inline unsigned blocksFor(size_t n, unsigned b) { return unsigned((n + b - 1) / b); }
-// Deferred refinements go through a compacted queue (knob, compile time).
-#ifndef RAMD_REFINE_QUEUE
-#define RAMD_REFINE_QUEUE 1
-#endif
-constexpr unsigned kQueueBlocks = RAMD_QUEUE_BLOCKS;
 // Waves of the refinement over the searched remainder (two fit a SIMD).
 constexpr unsigned kListBlocks = 2048;
 #define RAMD_STEP_SPECIES(LAUNCH)                     \
@@ -781,6 +716,14 @@ struct Step {
                                reuseSlot, cells, rep);
         }
         const FlashCells batch = {q, all, nullptr, sA, gate(), rep};
+        FlashSink sink = {};
+        sink.out = out;
+        sink.p = pOut;
+        sink.c = cOut;
+        sink.r = rOut;
+        sink.cost = costOut;
+        sink.counters = counter;
+        sink.failMark = failMark;
         if (mode == REACTIVE_AMD_FLASH_MIXED) {
             const CellList whole = {order, uint32_t(cells), nullptr};
             const CellList left = {searchList, 0, queueCount + 1};
@@ -800,8 +743,8 @@ struct Step {
 #define RAMD_STEP_REFINE(NS_, NL_)                                                                                 \
     hipLaunchKernelGGL((stepRefineKernel<NS_, NL_>), dim3(grid), dim3(block), 0, stream,                            \
                        static_cast<const HemModel<NS_>*>(h->model), batch, list, sets, out, pOut, cOut, rOut,      \
-                       costOut, counter, RAMD_REFINE_QUEUE ? queue : nullptr, queueCount, searchList,              \
-                       queueCount + 1, failMark)
+                       costOut, counter, queue, queueCount, searchList, queueCount + 1,                     \
+                       failMark)
                 RAMD_STEP_SPECIES(RAMD_STEP_REFINE)
 #undef RAMD_STEP_REFINE
             };
@@ -811,15 +754,11 @@ struct Step {
                                    counters + 6, stream);
                 refine(left, std::min(kListBlocks, blocksFor(cells, 64)), 64);
             }
-            if (RAMD_REFINE_QUEUE) {
-#define RAMD_STEP_QUEUE(NS_, NL_)                                                                                  \
-    hipLaunchKernelGGL((stepRefineQueueKernel<NS_, NL_>), dim3(kQueueBlocks), dim3(64), 0, stream,                  \
-                       static_cast<const HemModel<NS_>*>(h->model), batch, queue, queueCount, sets, out, pOut,     \
-                       cOut, rOut, costOut, counter, failMark)
-                RAMD_STEP_SPECIES(RAMD_STEP_QUEUE)
-#undef RAMD_STEP_QUEUE
-                hipLaunchKernelGGL(queueTotalKernel, dim3(1), dim3(64), 0, stream, queueCount, counters + 7);
-            }
+            launchRefineQueue(ns, h->nl, h->model, batch, queue, queueCount, sets, sink, stream);
+            hipLaunchKernelGGL(queueTotalKernel, dim3(1), dim3(64), 0, stream, queueCount, counters + 7);
+        } else if (cells <= RAMD_GROUP_CELLS) {
+            launchGroupFlash(ns, h->nl, h->analytic, false, h->model, batch, order, uint32_t(cells), nullptr, sink,
+                             stream);
         } else {
 #define RAMD_STEP_FLASH(NS_, NL_, RJ_)                                                                            \
     hipLaunchKernelGGL((stepFlashKernel<NS_, NL_, RJ_>), dim3(blocks), dim3(flashBlock), 0, stream,                \
