@@ -63,6 +63,7 @@ struct HemModel {
     PhaseHeuristic gasFixed;     // composition-independent heuristic when NS == 1
     PhaseHeuristic liquidFixed;  // pure liquid table
     int nl, condensable, scalarRecovery, stableGasPrune, enforceBounds, analyticJacobian, boundaryRecovery;
+    int twin, pad;  // one species whose gas and liquid tables are the same
     double weights[NS];
     double liquidTmin, liquidTc, Tmin, Tmax, pmin, pmax, vtol, etol, mutol;
 };
@@ -495,45 +496,77 @@ struct Flash : FlashCap<CAP, R> {
         return memo;
     }
 
+    // What states at one temperature (and one pressure: the cubic's outer
+    // roots) of one composition share: the gas probe's state at (T, rho) and
+    // its check at (T, p), and, for one species with the same gas and liquid
+    // tables, the two phases of a mixture.
+    struct Shared {
+        M mx;
+        IdealT<NS, R> ideal;
+        RootsT<R> r;
+        bool mixed, rooted;
+    };
     // Gas PR state at (T, p) on the gas root (evaluateTPTrusted, reactiveDevicePR.h:574-609).
-    RAMD_NOINLINE int gasTP(R T, R p, const R* Y, S& s, R* mu) { return gasTPBody(T, p, Y, s, mu); }
-    __device__ __attribute__((always_inline)) inline int gasTPBody(R T, R p, const R* Y, S& s, R* mu) {
+    // sh (may be null): what is known already, and kept for the next state;
+    // both: the cubic's smallest root too.
+    RAMD_NOINLINE int gasTP(R T, R p, const R* Y, S& s, R* mu) { return gasTPBody(T, p, Y, s, mu, nullptr, false); }
+    __device__ __attribute__((always_inline)) inline int gasTPBody(R T, R p, const R* Y, S& s, R* mu, Shared* sh,
+                                                                   bool both) {
         if (!fin(T) || !fin(p) || T <= 0 || p <= 0) return kBadInput;
         R x[NS], W = 0;
         int st = massToMole(mod().gas, Y, x, W);
         if (st != kOk) return st;
-        M mx;
-        st = mixing(mod().gas, T, x, mx);
+        Shared own;
+        Shared& k = sh ? *sh : own;
+        if (!sh || !sh->mixed) {
+            st = mixing(mod().gas, T, x, k.mx);
+            if (st != kOk) return st;
+            if (sh) {
+                idealAt(mod().gas, T, sh->ideal);
+                sh->mixed = true;
+            }
+        }
+        if (both) st = roots<kOuterRoots>(T, p, k.mx.a, k.mx.b, k.mx.aa, k.r);
+        else st = roots<kLargestRoot>(T, p, k.mx.a, k.mx.b, k.mx.aa, k.r);
         if (st != kOk) return st;
-        RootsT<R> r;
-        st = roots(T, p, mx.a, mx.b, mx.aa, r);
+        if (sh) sh->rooted = both;
+        if (!k.r.gas) return kUnavailable;
+        st = stateTrho(mod().gas, T, W / k.r.vLast, x, W, k.mx, s, mu, sh ? &sh->ideal : nullptr);
         if (st != kOk) return st;
-        if (!r.gas) return kUnavailable;
-        st = stateTrho(mod().gas, T, W / r.vLast, x, W, mx, s, mu);
-        if (st != kOk) return st;
-        st = finishState<NS>(gasHeuristic(x, W, mx), T, s, mu);
+        st = finishState<NS>(gasHeuristic(x, W, k.mx), T, s, mu);
         if (st != kOk) return st;
         if (ab(s.p - p) > R(P::rootCheck) * hi(R(1), p)) return kNonFinite;
         s.p = p;
         if (s.phase >= 0) return kUnavailable;
         return kOk;
     }
-    // Pure-liquid PR state at (T, p) on the liquid root.
-    RAMD_NOINLINE int liquidTP(R T, R p, S& s, R* mu) { return liquidTPBody(T, p, s, mu); }
-    __device__ __attribute__((always_inline)) inline int liquidTPBody(R T, R p, S& s, R* mu) {
+    // Pure-liquid PR state at (T, p) on the liquid root; sh: the mixture's gas
+    // at the same point, from the same table.
+    RAMD_NOINLINE int liquidTP(R T, R p, S& s, R* mu) { return liquidTPBody(T, p, s, mu, nullptr); }
+    __device__ __attribute__((always_inline)) inline int liquidTPBody(R T, R p, S& s, R* mu, const Shared* sh) {
         if (!fin(T) || !fin(p) || T <= 0 || p <= 0) return kBadInput;
         const R Y[1] = {R(1)};
         R x[1], W = 0;
         int st = massToMole(mod().liquid, Y, x, W);
         if (st != kOk) return st;
         M mx;
-        st = mixing(mod().liquid, T, x, mx);
-        if (st != kOk) return st;
         RootsT<R> r;
-        st = roots(T, p, mx.a, mx.b, mx.aa, r);
-        if (st != kOk) return st;
+        const IdealT<1, R>* ideal = nullptr;
+        if constexpr (NS == 1) {
+            if (sh) {
+                mx = sh->mx;
+                r = sh->r;
+                ideal = &sh->ideal;
+            }
+        }
+        if (!ideal) {
+            st = mixing(mod().liquid, T, x, mx);
+            if (st != kOk) return st;
+            st = roots<kSmallestRoot>(T, p, mx.a, mx.b, mx.aa, r);
+            if (st != kOk) return st;
+        }
         if (!r.liquid) return kUnavailable;
-        st = stateTrho(mod().liquid, T, W / r.v0, x, W, mx, s, mu);
+        st = stateTrho(mod().liquid, T, W / r.v0, x, W, mx, s, mu, ideal);
         if (st != kOk) return st;
         st = finishState<1>(mod().liquidFixed, T, s, mu);
         if (st != kOk) return st;
@@ -544,7 +577,7 @@ struct Flash : FlashCap<CAP, R> {
     }
 
     // reactiveDeviceFlash.h:157-196 for index -1 (gas) and 0 (liquid).
-    RD int phaseStatus(int index, R p, R T, const R* Y, S& out, R* mu) {
+    RD int phaseStatus(int index, R p, R T, const R* Y, S& out, R* mu, Shared* sh = nullptr, bool both = false) {
         ++n.phases;
         if (!bounds(p, T)) return kBadInput;
         if (index >= 0 && T < liquidTmin) return kBadInput;
@@ -553,8 +586,8 @@ struct Flash : FlashCap<CAP, R> {
             for (int k = 0; k < NS; ++k)
                 if (Y[k] > 0 && (T < R(mod().gas.tlo[k]) || T > R(mod().gas.thi[k]))) return kBadInput;
         if constexpr (P::single ? RAMD_SEARCH_INLINE != 0 : RAMD_FLASH_INLINE != 0) {
-            if (index >= 0) return liquidTPBody(T, p, out, mu);
-            return gasTPBody(T, p, Y, out, mu);
+            if (index >= 0) return liquidTPBody(T, p, out, mu, sh);
+            return gasTPBody(T, p, Y, out, mu, sh, both);
         }
         if (index >= 0) return liquidTP(T, p, out, mu);
         return gasTP(T, p, Y, out, mu);
@@ -705,11 +738,17 @@ struct Flash : FlashCap<CAP, R> {
         for (int k = 0; k < NS; ++k) mg += gas[k];
         v.gasMass = mg;
         const R pg = gasPressure(p), pl = liquidPressure(p);
+        const bool withLiquid = NL && (mass0 > 0 || (virtualLiquids && q[c] > 0));
+        // one species, one table, one pressure: the liquid shares the gas's mixing, ideal part and cubic
+        Shared shared;
+        const bool share = NS == 1 && NL && withLiquid && mod().twin != 0 && pg == pl;
+        shared.mixed = shared.rooted = false;
         if (mg > 0) {
             for (int k = 0; k < NS; ++k) gas[k] /= mg;
             S prop;
             R mu[NS];
-            if (phaseStatus(-1, pg, T, gas, prop, virtualLiquids ? mu : nullptr) != kOk) return false;
+            if (phaseStatus(-1, pg, T, gas, prop, virtualLiquids ? mu : nullptr, share ? &shared : nullptr, share) != kOk)
+                return false;
             if constexpr (RJ) v.ref.gasMolarVolume = prop.V;
             accumulate(v, mg, prop, pg);
             if constexpr (E::kOutputs) {
@@ -724,7 +763,7 @@ struct Flash : FlashCap<CAP, R> {
         }
         if (NL) {
             v.liqMass = mass0;
-            if (mass0 > 0 || (virtualLiquids && q[c] > 0)) {
+            if (withLiquid) {
                 S prop;
                 R mu[1];
                 int st;
@@ -732,7 +771,8 @@ struct Flash : FlashCap<CAP, R> {
                     ++n.phases;
                     st = cacheStatus;
                 } else {
-                    st = phaseStatus(0, pl, T, nullptr, prop, virtualLiquids ? mu : nullptr);
+                    st = phaseStatus(0, pl, T, nullptr, prop, virtualLiquids ? mu : nullptr,
+                                     shared.rooted ? &shared : nullptr);
                     if (unavailable(st) && T >= liquidTmin && T < liquidTc * (R(1) - R(1e-10))) {
                         cacheP = p; cacheT = T; cacheVirtual = virtualLiquids; cacheStatus = st;
                     }
@@ -788,14 +828,17 @@ struct Flash : FlashCap<CAP, R> {
         for (int k = 0; k < NS; ++k) Y[k] = q[k] / rho;
         ++n.phases;
         S prop;
+        Shared shared;
+        shared.mixed = shared.rooted = false;
         {
             if (!fin(T) || !fin(rho) || T <= 0 || rho <= 0) return false;
             R x[NS], W = 0;
             if (massToMole(mod().gas, Y, x, W) != kOk) return false;
-            M mx;
-            if (mixing(mod().gas, T, x, mx) != kOk) return false;
-            if (stateTrho(mod().gas, T, rho, x, W, mx, prop, (R*)nullptr) != kOk) return false;
-            if (finishState<NS>(gasHeuristic(x, W, mx), T, prop, (const R*)nullptr) != kOk) return false;
+            if (mixing(mod().gas, T, x, shared.mx) != kOk) return false;
+            idealAt(mod().gas, T, shared.ideal);
+            shared.mixed = true;
+            if (stateTrho(mod().gas, T, rho, x, W, shared.mx, prop, (R*)nullptr, &shared.ideal) != kOk) return false;
+            if (finishState<NS>(gasHeuristic(x, W, shared.mx), T, prop, (const R*)nullptr) != kOk) return false;
         }
         const R gasP = prop.p;
         if constexpr (CAP) p = gasP + this->color * this->jump;
@@ -803,7 +846,7 @@ struct Flash : FlashCap<CAP, R> {
         if (!bounds(p, T)) return false;
         if (check) {
             S gas;
-            if (phaseStatus(-1, gasP, T, Y, gas, nullptr) != kOk || ab(gas.rho - rho) > R(P::densityCheck) * rho)
+            if (phaseStatus(-1, gasP, T, Y, gas, nullptr, &shared) != kOk || ab(gas.rho - rho) > R(P::densityCheck) * rho)
                 return false;
         }
         F = rho * prop.e - energy;

@@ -136,6 +136,9 @@ inline void buildDeviceModel(const Model& m, HemModel<NS>& d) {
         compactTable<1>(m.phase[1], d.liquid);
         fixedHeuristic<1>(d.liquid, d.liquidFixed);
     }
+    if constexpr (NS == 1)
+        d.twin = m.nl && std::memcmp(&d.gas, &d.liquid, sizeof(d.gas)) == 0 &&
+                 std::memcmp(&d.gasFixed, &d.liquidFixed, sizeof(d.gasFixed)) == 0;
     d.nl = m.nl;
     d.condensable = m.nl ? m.condensable[0] : 0;
     d.scalarRecovery = m.scalarRecovery;

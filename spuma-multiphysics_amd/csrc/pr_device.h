@@ -62,11 +62,13 @@ template <> struct Real<double> {
     static constexpr double big = 1.7976931348623157e308, eps = DBL_EPSILON, tiny = 1e-300;
     static constexpr double polish = 4e-15;    // cubic-root Newton polish (reactiveDevicePR.h:280-307)
     static constexpr double flatness = 1e-14;  // |f'| below which the polish stops
+    static constexpr double separated = 1e-6;  // -disc / h^2 above which three roots are well apart
 };
 template <> struct Real<float> {
     static constexpr float big = 3.4028234663852886e38f, eps = FLT_EPSILON, tiny = 1e-30f;
     static constexpr float polish = 2e-7f;
     static constexpr float flatness = 1e-30f;
+    static constexpr float separated = 1e-2f;
 };
 
 template <class R> RHD bool fin(R x) { return x == x && (x < 0 ? -x : x) <= Real<R>::big; }
@@ -225,14 +227,36 @@ struct CubicTrig<double, false> {
     static RHD double cos(double x) { return elem::cosFast(x); }
 };
 
-template <class R, bool Exact = true> RHD int roots(R T, R p, R a, R b, R aa, RootsT<R>& out);
+// Which of three roots a caller reads: the largest (a gas state), the
+// smallest (a liquid state), both, or all of them sorted.
+enum RootsWanted : int { kAllRoots = 0, kLargestRoot = 1, kSmallestRoot = 2, kOuterRoots = 3 };
+template <int Wanted = kAllRoots, class R, bool Exact = true> RHD int roots(R T, R p, R a, R b, R aa, RootsT<R>& out);
+
+// Newton polish of one root.
+template <class R>
+RHD R polishedRoot(R x, R bn, R cn, R dn) {
+    for (int it = 0; it < 12; ++it) {
+        const R res = cubic(x, bn, cn, dn);
+        const R der = (R(3) * x + R(2) * bn) * x + cn;
+        if (ab(der) <= R(Real<R>::tiny)) break;
+        const R step = res / der;
+        x -= step;
+        if (ab(step) <= R(Real<R>::polish) * hi(R(1), ab(x))) break;
+    }
+    return x;
+}
 
 // Cubic root set at (T, p) from the mixture coefficients
 // (rootsFromMixingCached, reactiveDevicePR.h:701-790).  Only the smallest and
 // largest physical roots are kept: the flash selects nothing else.
 // In single precision the classification of a near-repeated root pair (the
 // discriminant within rounding of zero) is decided in double precision.
-template <class R, bool Exact>
+// Wanted: three roots that are well apart need no sorting, and the cubic is
+// negative at the covolume, -2 b^2 RT / p, so all three lie above it where its
+// local maximum at center - delta does: then only the roots that the caller
+// reads are computed, as the general sequence computes them (bit for bit; a
+// cosine and a polish of some four Newton steps less for each of the others).
+template <int Wanted, class R, bool Exact>
 RHD int roots(R T, R p, R a, R b, R aa, RootsT<R>& out) {
     if (!fin(T) || !fin(p) || !fin(a) || !fin(b) || !fin(aa) || T <= 0 || p <= 0 || a <= 0 || b <= 0 || aa <= 0)
         return kBadInput;
@@ -249,7 +273,7 @@ RHD int roots(R T, R p, R a, R b, R aa, RootsT<R>& out) {
     R disc = q * q - h * h;
     if (sizeof(R) < sizeof(double) && ab(disc) <= R(RAMD_CUBIC_FP64_BAND) * (q * q + h * h)) {
         RootsT<double> d;
-        const int st = roots<double, false>(double(T), double(p), double(a), double(b), double(aa), d);
+        const int st = roots<Wanted, double, false>(double(T), double(p), double(a), double(b), double(aa), d);
         out.v0 = R(d.v0); out.vLast = R(d.vLast);
         out.count = d.count; out.signedCount = d.signedCount; out.gas = d.gas; out.liquid = d.liquid;
         return st;
@@ -276,6 +300,16 @@ RHD int roots(R T, R p, R a, R b, R aa, RootsT<R>& out) {
         arg = hi(R(-1), lo(R(1), arg));
         using Trig = CubicTrig<R, Exact>;
         const R theta = Trig::acos(arg) / R(3);
+        if (Wanted != kAllRoots && -disc > R(Real<R>::separated) * (h * h) && b < center - delta) {
+            if (Wanted & kLargestRoot) out.vLast = polishedRoot(center + R(2) * delta * Trig::cos(theta), bn, cn, dn);
+            if (Wanted & kSmallestRoot)
+                out.v0 = polishedRoot(center + R(2) * delta * Trig::cos(theta + R(2) * R(kPi) / R(3)), bn, cn, dn);
+            out.count = out.signedCount = 3;
+            out.gas = out.liquid = 1;
+            const bool fine = (!(Wanted & kLargestRoot) || (fin(out.vLast) && out.vLast > center)) &&
+                              (!(Wanted & kSmallestRoot) || (out.v0 > b && out.v0 < center));
+            if (fine) return kOk;
+        }
         raw[0] = center + R(2) * delta * Trig::cos(theta);
         raw[1] = center + R(2) * delta * Trig::cos(theta + R(2) * R(kPi) / R(3));
         raw[2] = center + R(2) * delta * Trig::cos(theta + R(4) * R(kPi) / R(3));
@@ -284,15 +318,7 @@ RHD int roots(R T, R p, R a, R b, R aa, RootsT<R>& out) {
         return kNoRoot;
     }
     if (!isolated)
-        for (int i = 0; i < n; ++i)
-            for (int it = 0; it < 12; ++it) {
-                const R res = cubic(raw[i], bn, cn, dn);
-                const R der = (R(3) * raw[i] + R(2) * bn) * raw[i] + cn;
-                if (ab(der) <= R(Real<R>::tiny)) break;
-                const R step = res / der;
-                raw[i] -= step;
-                if (ab(step) <= R(Real<R>::polish) * hi(R(1), ab(raw[i]))) break;
-            }
+        for (int i = 0; i < n; ++i) raw[i] = polishedRoot(raw[i], bn, cn, dn);
     // ascending order, finite roots above the covolume (reactiveDevicePR.h:253-269)
     for (int i = 1; i < n; ++i) {
         const R key = raw[i];
@@ -369,7 +395,7 @@ RHD void phaseHeuristic(const Table<N>& t, const R* x, R W, R mixA, R mixB, Phas
     bool found = false;
     for (int it = 0; it < 100; ++it) {
         RootsT<R> r;
-        st = roots(tmid, pp, mm.a, mm.b, mm.aa, r);
+        st = roots<kSmallestRoot>(tmid, pp, mm.a, mm.b, mm.aa, r);
         if (st != kOk) { h.status = st; return; }
         if (r.signedCount == 1 || r.signedCount == 2) {
             found = pp > pc;
@@ -408,8 +434,16 @@ RHD int reportedPhase(const PhaseHeuristic& h, R T, R rho, int& phase) {
 // is computed for every species when mu != nullptr.
 // The phaseState comparison and the final finiteness checks follow in
 // finishState(), in the reference's order.
+// ideal (may be null): the species' ideal-gas properties at T, already at hand.
 template <int N, class R>
-RHD int stateTrho(const Table<N>& t, R T, R rho, const R* x, R W, const MixT<R>& mx, PRStateT<R>& s, R* mu) {
+struct IdealT { R cpR[N], hRT[N], sR[N]; };
+template <int N, class R>
+RHD void idealAt(const Table<N>& t, R T, IdealT<N, R>& out) {
+    for (int k = 0; k < N; ++k) nasa(region(t, k, T), T, out.cpR[k], out.hRT[k], out.sR[k]);
+}
+template <int N, class R>
+RHD int stateTrho(const Table<N>& t, R T, R rho, const R* x, R W, const MixT<R>& mx, PRStateT<R>& s, R* mu,
+                  const IdealT<N, R>* ideal = nullptr) {
     if (!fin(T) || !fin(rho) || T <= 0 || rho <= 0) return kBadInput;
     const R b = mx.b, aa = mx.aa, da = mx.da, d2a = mx.d2a;
     const R Rg = R(kR), sq2 = R(kSqrt2);
@@ -432,7 +466,11 @@ RHD int stateTrho(const Table<N>& t, R T, R rho, const R* x, R W, const MixT<R>&
     R hRT[N], sR[N];
     for (int k = 0; k < N; ++k) {
         R cpR, hk, sk;
-        nasa(region(t, k, T), T, cpR, hk, sk);
+        if (ideal) {
+            cpR = ideal->cpR[k]; hk = ideal->hRT[k]; sk = ideal->sR[k];
+        } else {
+            nasa(region(t, k, T), T, cpR, hk, sk);
+        }
         hRT[k] = hk; sR[k] = sk;
         cp0 += x[k] * Rg * cpR;
         h0 += x[k] * Rg * T * hk;
