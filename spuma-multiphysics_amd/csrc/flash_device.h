@@ -205,6 +205,7 @@ enum CandidateFlags : uint32_t {
     kDirect = 8u,            // the directed search's (saturation table): one candidate or none
     kNotGas = 16u,           // with kDirect: the all-gas solve cannot lead to the equilibrium
     kNotLiquid = 32u,        // with kDirect: nor can the all-liquid one
+    kSingle = 64u,           // with kDirect: the point has one phase
 };
 enum StartBits : uint32_t {
     kStartFound = 1u,   // converged, or stalled near convergence
@@ -1012,7 +1013,8 @@ struct Flash : FlashCap<CAP, R> {
     // Residual [V-1, (E-e)/scale, mu_l/RT - mu_g/RT] in x = [ln p, ln T, beta]
     // (reactiveDeviceFlash.h:327-337).
     // In vapour coordinates (CAP, this->adaptive) x[2] = ln(vapour fraction) <= 0.
-    RAMD_NOINLINE bool residual(const R* x, R scale, R* f, E* out) {
+    RAMD_NOINLINE bool residual(const R* x, R scale, R* f, E* out) { return residualBody(x, scale, f, out); }
+    __device__ __attribute__((always_inline)) inline bool residualBody(const R* x, R scale, R* f, E* out) {
         ++n.residuals;
         R mass0, vapour = R(-1);
         if constexpr (CAP) {
@@ -1030,7 +1032,7 @@ struct Flash : FlashCap<CAP, R> {
             mass0 = x[2] * q[mod().condensable];
         }
         E v;
-        if (!evaluate(mass0, m_exp(x[0]), m_exp(x[1]), v, true, vapour) || !(v.gasMass > 0)) return false;
+        if (!evaluateBody(mass0, m_exp(x[0]), m_exp(x[1]), v, true, vapour) || !(v.gasMass > 0)) return false;
         f[0] = v.volume - R(1);
         f[1] = (v.energy - energy) / scale;
         f[2] = v.muLiquid - v.muGas;
@@ -1336,6 +1338,9 @@ struct Flash : FlashCap<CAP, R> {
     // Converged point: the equilibrium sound speed from the Jacobian's response
     // to a volume/energy perturbation (reactiveDeviceFlash.h:400-409).
     RAMD_NOINLINE bool activeFinish(const R* x, R scale, const R* f, E& value) {
+        return activeFinishBody(x, scale, f, value);
+    }
+    __device__ __attribute__((always_inline)) inline bool activeFinishBody(const R* x, R scale, const R* f, E& value) {
         const R rho = density();
         R jac[3][3];
         if constexpr (A && NS == 1 && !P::single) {
@@ -1487,6 +1492,119 @@ struct Flash : FlashCap<CAP, R> {
             }
         }
         return polishing && activeFinish(x, scale, f, value);
+    }
+    // activeNewton of a pure fluid with this build's analytic Jacobian, as one
+    // loop around one evaluation, so that all of it inlines and its state
+    // stays in registers: the general solvers keep the flash and its records
+    // on the stack, and a solve waits for the stack (75 % of the cycles of a
+    // 160^3 search, whose stacks do not fit the L2).  Same evaluations, same
+    // steps, same result; the FP64 form gives up (false) at the first step it
+    // would have to shorten, so that it needs one evaluation record only.
+    __device__ __attribute__((always_inline)) inline bool activeLean(R (&x)[3], R scale, E& value, int polish) {
+        static_assert(A && NS == 1 && GROUP == 1 && !CAP, "a pure fluid's analytic Newton");
+        const auto outside = [](R y) { return !(y >= 0 && y < 1); };
+        stalled = false;
+        R tx[3] = {x[0], x[1], x[2]}, f[3] = {}, step[3] = {};
+        R previous = 0, fraction = 1;
+        int index = -1, it = 0;  // index -1: the starting point
+        for (;;) {
+            E trial;
+            E& now = P::single ? trial : value;
+            R tf[3];
+            bool accepted = residualBody(tx, scale, tf, &now);
+            if (index < 0) {
+                if (!accepted) return false;
+            } else {
+                accepted = accepted && hi(hi(hi(R(0), ab(tf[0])), ab(tf[1])), ab(tf[2])) <
+                                           previous * (R(1) - R(1e-4) * fraction);
+            }
+            if (!P::single && !accepted) return false;
+            if (accepted) {
+                for (int j = 0; j < 3; ++j) { x[j] = tx[j]; f[j] = tf[j]; }
+                if constexpr (P::single) value = trial;
+                it += index < 0 ? 0 : 1;
+                if (it >= 90) return false;
+                const R chemical = hi(R(0), ab(f[2]));
+                if (ab(f[0]) <= vtol && ab(f[1]) <= etol && chemical <= mutol) {
+                    if constexpr (E::kOutputs) {
+                        value.volRes = ab(f[0]);
+                        value.enRes = ab(f[1]);
+                        value.chemRes = chemical;
+                        value.iterations = it;
+                    }
+                    if (P::single) return true;
+                    const bool tight = ab(f[0]) <= R(1e-3) * vtol && ab(f[1]) <= R(1e-3) * etol &&
+                                       chemical <= R(1e-3) * mutol;
+                    if (!(polish > 0 && !tight)) return activeFinishBody(x, scale, f, value);
+                    --polish;
+                }
+                R jac[3][3];
+                analyticJacobian(value, scale, jac);
+                R rhs[3] = {-f[0], -f[1], -f[2]};
+                if (!solveN<3>(jac, rhs, step)) return false;
+                R limiter = hi(R(1), hi(ab(step[0]) / R(.7), ab(step[1]) / R(.18)));
+                limiter = hi(limiter, ab(step[2]) / R(.3));
+                for (int j = 0; j < 3; ++j) step[j] /= limiter;
+                previous = hi(hi(hi(R(0), ab(f[0])), ab(f[1])), ab(f[2]));
+                fraction = 1;
+                index = 0;
+            } else {
+                ++index;
+                fraction *= R(.5);
+            }
+            bool exhausted = index >= 30;
+            for (int j = 0; j < 3; ++j) tx[j] = x[j] + fraction * step[j];
+            if (!exhausted && outside(tx[2])) {  // the rejected prefix of the fractions
+                if constexpr (!P::single) return false;
+                int lower = index, upper = 30;
+                while (upper - lower > 1) {
+                    const int mid = (lower + upper) / 2;
+                    if (outside(x[2] + R(::ldexp(1.0, -mid)) * step[2])) lower = mid;
+                    else upper = mid;
+                }
+                n.residuals += uint32_t(upper - index);
+                exhausted = upper == 30;
+                index = upper;
+                fraction = R(::ldexp(1.0, -upper));
+                for (int j = 0; j < 3; ++j) tx[j] = x[j] + fraction * step[j];
+            }
+            if constexpr (P::single) exhausted = exhausted || (tx[0] == x[0] && tx[1] == x[1] && tx[2] == x[2]);
+            if (exhausted) {
+                stalled = P::single && previous <= R(P::handOver);
+                return false;
+            }
+        }
+    }
+    // Seed j (2 + j) or restart (7 + 5 t + j) of a pure fluid's search:
+    // whether it arrives.
+    __device__ __attribute__((always_inline)) inline bool seedArrives(int start) {
+        if (!searchable() || !(q[0] > 0)) return false;
+        const bool restart = start >= 7;
+        const int j = restart ? (start - 7) % 5 : start - 2;
+        const R seed = j == 0 ? R(-1) : j == 1 ? R(.5) : j == 2 ? R(.95) : j == 3 ? R(.1) : R(.9999);
+        E candidate;
+        R x[3], scale;
+        ++n.candidates;
+        activeStart(seed, restart, restart ? restartTemperature((start - 7) / 5) : R(0), x, scale);
+        return activeLean(x, scale, candidate, 0) || stalled;
+    }
+    // refine() of a set that holds one two-phase point of a pure fluid, where
+    // it succeeds without a shortened step; otherwise false, and the counters
+    // are to be dropped.
+    __device__ __attribute__((always_inline)) inline bool refineTwoPhase(const Candidate& c, E& best) {
+        if (!searchable()) return false;
+        ++n.failures;  // the gas candidate refine() counts as not found
+        ++n.candidates;
+        R x[3], scale;
+        activeStart(R(-1), false, R(0), x, scale);
+        x[0] = R(c.x[0]);
+        x[1] = R(c.x[1]);
+        x[2] = R(c.x[2]);
+        if (!activeLean(x, scale, best, 2)) return false;
+        // stable(): the converged point's own chemical potentials
+        const R affinity = best.muLiquid - best.muGas;
+        ++n.stable;
+        return fin(affinity) && !(ab(affinity) > mutol * R(2));
     }
     RAMD_NOINLINE bool activeFlash(R seed, E& value, bool restart, R restartT) {
         ++n.candidates;

@@ -236,12 +236,19 @@ struct StartRecord {
 };
 // Scratch of the search: kStarts records per listed cell (record s of list
 // position i at s stride + i), the cells to restart, and the directed
-// search's cells to try again; the counts are zero on entry.
+// search's two-phase cells to try again and one-phase cells; the counts are
+// zero on entry.
 struct SearchScratch {
     StartRecord* records;
-    uint32_t *restarts, *again;
-    unsigned *restartCount, *againCount;
+    uint32_t *restarts, *again, *single;
+    unsigned *restartCount, *againCount, *singleCount;
 };
+// FP64 refinement of a directed search's two-phase points.  Cells without a
+// point go to the list `search`; one-phase cells, and those whose point takes
+// more than full Newton steps, are left to refine(), in scratch.single.
+void launchRefineTwoPhase(const void* model, const FlashCells& cells, const uint32_t* order, uint32_t count,
+                          const CandidateSet* sets, const FlashSink& sink, const SearchScratch& scratch,
+                          uint32_t* search, unsigned* searchCount, hipStream_t stream);
 // Saturated liquid and vapour at evenly spaced temperatures: specific volumes
 // and energies, ln p.  Interpolated between 2,048 rows over N2O's 161 K they
 // lie within 1e-6 of the curve except next to the critical point, inside the

@@ -112,9 +112,9 @@ __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineKernel(con
     addTotals(n, succeeded, totals);
 }
 
-// deferred cells, cells to search, cells to restart, cells the directed search tries again
+// deferred cells, cells to search, to restart, to try again, one-phase cells
 __global__ void clearCountsKernel(unsigned* __restrict__ counts) {
-    if (threadIdx.x < 4) counts[threadIdx.x] = 0;
+    if (threadIdx.x < 5) counts[threadIdx.x] = 0;
 }
 
 // totals[k] = sum over b < blocks of partials[b * width + k], k < width: one
@@ -217,7 +217,7 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
     if (!count) return;
     if (!sets) {
         queue = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
-        queueCount = static_cast<unsigned*>(allocate(4 * sizeof(unsigned)));
+        queueCount = static_cast<unsigned*>(allocate(5 * sizeof(unsigned)));
         if (!prune) {
             scratch.records = static_cast<StartRecord*>(allocate(kStarts * capacity * sizeof(StartRecord)));
             scratch.restarts = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
@@ -227,6 +227,8 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
             searchList = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
             scratch.again = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
             scratch.againCount = queueCount + 3;
+            scratch.single = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
+            scratch.singleCount = queueCount + 4;
             saturation = static_cast<SaturationTable*>(allocate(sizeof(SaturationTable)));
             launchSaturation(model, saturation, s);
         }
@@ -235,14 +237,21 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
     const unsigned blocks = unsigned((count + 63) / 64);
     const FlashCells cells = {q, 0, e, g, nullptr, nullptr};
     const CellList whole = {order, uint32_t(count), nullptr}, left = {searchList, 0, queueCount + 1};
+    const CellList first = saturation ? CellList{scratch.single, 0, scratch.singleCount} : whole;
+    FlashSink sink = {};
+    sink.hem = out;
+    sink.totals = totals;
     hipLaunchKernelGGL(zeroTotalsKernel, dim3(1), dim3(64), 0, s, totals, 10);
     hipLaunchKernelGGL(clearCountsKernel, dim3(1), dim3(64), 0, s, queueCount);
     if (saturation) launchDirect(model, saturation, cells, order, uint32_t(count), scratch, sets, nullptr, totals + 8, s);
     else if (prune) launchSearch(ns, nl, model, cells, order, uint32_t(count), sets, nullptr, totals + 8, s, 64);
     else launchSearchStarts(ns, nl, model, cells, whole, count, scratch, false, sets, nullptr, totals + 8, s);
+    if (saturation)
+        launchRefineTwoPhase(model, cells, order, uint32_t(count), sets, sink, scratch, searchList,
+                             queueCount + 1, s);
 #define RAMD_HEM_MIXED(NS_, NL_)                                                                                  \
     hipLaunchKernelGGL((hemRefineKernel<NS_, NL_>), dim3(blocks), dim3(64), 0, s,                                   \
-                       static_cast<const HemModel<NS_>*>(model), cells, whole, sets, out, totals, queue,          \
+                       static_cast<const HemModel<NS_>*>(model), cells, first, sets, out, totals, queue,          \
                        queueCount, searchList, queueCount + 1);                                                   \
     if (saturation) {                                                                                             \
         launchSearchStarts(ns, nl, model, cells, left, count, scratch, true, sets, nullptr, totals + 8, s);       \
@@ -255,9 +264,6 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
     else if (nl == 0) { RAMD_HEM_MIXED(2, 0); }
     else { RAMD_HEM_MIXED(2, 1); }
 #undef RAMD_HEM_MIXED
-    FlashSink sink = {};
-    sink.hem = out;
-    sink.totals = totals;
     launchRefineQueue(ns, nl, model, cells, queue, queueCount, sets, sink, s);
     hipLaunchKernelGGL(queueCountKernel, dim3(1), dim3(64), 0, s, queueCount, totals + 9);
     RAMD_HIP(hipGetLastError());

@@ -37,8 +37,8 @@ namespace ramd {
 
 // ---------------------------------------------------------------- kernels
 // Counts of the mixed flash's lists: deferred cells, cells to search, cells to restart,
-// cells the directed search tries again.
-constexpr int kQueueCounts = 4;
+// cells the directed search tries again, one-phase cells.
+constexpr int kQueueCounts = 5;
 
 // Plain FP64 flash of the cells in `order`; RJ: the model's
 // analytic-Jacobian mode.
@@ -788,7 +788,13 @@ struct Step {
                 RAMD_STEP_SPECIES(RAMD_STEP_REFINE)
 #undef RAMD_STEP_REFINE
             };
-            refine(whole, blocks, flashBlock);
+            if (saturation) {
+                launchRefineTwoPhase(h->model, batch, orderSearch, uint32_t(cells), sets, sink, scratch,
+                                     searchList, queueCount + 1, stream);
+                refine({scratch.single, 0, scratch.singleCount}, std::min(kListBlocks, blocksFor(cells, 64)), 64);
+            } else {
+                refine(whole, blocks, flashBlock);
+            }
             if (saturation) {  // the cells whose table candidates were not confirmed
                 launchSearchStarts(ns, h->nl, h->model, batch, left, cells, scratch, true, sets, searchCost,
                                    counters + 6, stream);
@@ -1320,6 +1326,8 @@ int reactive_amd_step_run(void* step, double cfl, double maximum, int steps, int
                 s.searchList = s.alloc<uint32_t>(s.cells);
                 s.scratch.again = s.alloc<uint32_t>(s.cells);
                 s.scratch.againCount = s.queueCount + 3;
+                s.scratch.single = s.alloc<uint32_t>(s.cells);
+                s.scratch.singleCount = s.queueCount + 4;
                 s.saturation = s.alloc<SaturationTable>(1);
                 launchSaturation(s.h->model, s.saturation, s.stream);
             }
