@@ -370,7 +370,8 @@ __device__ inline HemModel<NS>& sharedModel() {
 // at once.  The results are those of the one-lane flash bit for bit, and so
 // are the counts (the evaluations past the loop's end are not counted; the
 // flash's only memo, an unavailable liquid at (p, T), repeats what
-// recomputing gives).  searchGroups runs a cell's starts on the eight groups
+// recomputing gives; in single precision, where the gas heuristic of a close
+// composition is reused, the lanes agree on the last one kept).  searchGroups runs a cell's starts on the eight groups
 // of a wave.  Every lane of a group makes every call (lanes past a loop's end
 // repeat its last point).
 template <int NS, int NL, class R = double, bool A = FlashPrecision<R>::single, bool RJ = false, bool CAP = false,
@@ -379,7 +380,7 @@ struct Flash : FlashCap<CAP, R> {
     static_assert(NL == 0 || NL == 1, "one pure liquid at most");
     static_assert(!RJ || (!A && !FlashPrecision<R>::single), "the reference's analytic mode is an FP64 flash");
     static_assert(!CAP || (!A && !FlashPrecision<R>::single), "the capillary flash is an FP64 flash");
-    static_assert(GROUP == 1 || (GROUP == 8 && !FlashPrecision<R>::single), "groups of eight lanes, FP64 only");
+    static_assert(GROUP == 1 || GROUP == 8, "groups of eight lanes");
     using P = FlashPrecision<R>;
     using E = EvalT<R, A, RJ, CAP>;
     using S = PRStateT<R>;
@@ -403,6 +404,10 @@ struct Flash : FlashCap<CAP, R> {
     // single-precision search: where converged candidates are recorded
     CandidateSet* record;
     bool stalled;  // the last FP32 Newton stopped near convergence (hand-over)
+    // single-precision search of one start: given up past this many phase
+    // evaluations, for a group of lanes to do instead
+    uint32_t phaseLimit;
+    bool overrun;
 
     RD Flash(const HemModel<NS>& model, Counts& counts) : m(model), n(counts) {
         cacheP = cacheT = 0;
@@ -416,6 +421,8 @@ struct Flash : FlashCap<CAP, R> {
         liquidTmin = R(mod().liquidTmin); liquidTc = R(mod().liquidTc);
         record = nullptr;
         stalled = false;
+        phaseLimit = ~0u;
+        overrun = false;
     }
     // GROUP: this lane's place in its group, the group's first lane, a ballot
     // over the group and a group lane's value.
@@ -463,6 +470,14 @@ struct Flash : FlashCap<CAP, R> {
         const Memo mine = memoNow();
         const Memo left = groupValue(mine, misses ? 31 - __builtin_clz(misses) : 0);
         memoSet(misses ? left : entry);
+        if constexpr (P::single && NS > 1) heuristicFrom(last);
+    }
+    // The lanes' gas heuristics after such evaluations are lane `last`'s: in
+    // single precision a close composition's is reused, so they must agree.
+    RD void heuristicFrom(int last) {
+        for (int k = 0; k < NS; ++k) memoKey[k] = groupValue(memoKey[k], last);
+        memo = groupValue(memo, last);
+        memoValid = groupBallot(memoValid) >> last & 1u;
     }
     // Phase pressures of a curved interface (reactiveDeviceFlash.h:152-153).
     RD R gasPressure(R p) const {
@@ -958,15 +973,21 @@ struct Flash : FlashCap<CAP, R> {
             bool accepted = false;
             if constexpr (GROUP > 1) {
                 // fractions above 1e-9: 2^0 ... 2^-29, GROUP at a time
-                for (int first = 0; first < 30 && !accepted; first += GROUP) {
+                bool moved = true;
+                for (int first = 0; first < 30 && !accepted && moved; first += GROUP) {
                     const int index = lo(first + groupLane(), 29);
-                    const bool counted = first + groupLane() < 30;
+                    bool counted = first + groupLane() < 30;
                     const R fraction = R(::ldexp(1.0, -index));
                     const Counts before = n;
                     const Memo entry = memoNow();
                     E trial;
                     zeroEval(trial);
                     const R pp = p * m_exp(fraction * step[0]), tt = T * m_exp(fraction * step[1]);
+                    if constexpr (P::single) {  // no movement now or at any smaller fraction
+                        const bool moves = !(pp == p && tt == T);
+                        counted = counted && moves;
+                        moved = !groupBallot(!moves);
+                    }
                     bool ok = evaluate(mass0, pp, tt, trial, false);
                     const R next = hi(ab(trial.volume - R(1)), ab(trial.energy - energy) / scale);
                     ok = ok && counted && (next < previous * (R(1) - R(1e-4) * fraction) || next < lo(vtol, etol));
@@ -991,6 +1012,10 @@ struct Flash : FlashCap<CAP, R> {
                 // FP64 flashes keep every halving, as the reference counts them
                 if constexpr (P::single)
                     if (pp == p && tt == T) break;
+                if constexpr (P::single) {
+                    overrun = n.phases > phaseLimit;
+                    if (overrun) return false;
+                }
                 if (evaluate(mass0, pp, tt, trial, false)) {
                     const R next = hi(ab(trial.volume - R(1)), ab(trial.energy - energy) / scale);
                     if (next < previous * (R(1) - R(1e-4) * fraction) || next < lo(vtol, etol)) {
@@ -1120,6 +1145,7 @@ struct Flash : FlashCap<CAP, R> {
             const Memo mine = memoNow();
             const Memo left = groupValue(mine, misses ? 31 - __builtin_clz(misses) : 0);
             memoSet(misses ? left : entry);
+            if constexpr (P::single && NS > 1) heuristicFrom(5);
             for (int j = 0; j < 3; ++j) {
                 const uint32_t p2 = groupSum(groupLane() >> 1 == j ? n.phases - start.phases : 0u);
                 const uint32_t r2 = groupSum(groupLane() >> 1 == j ? n.residuals - start.residuals : 0u);
@@ -1425,13 +1451,19 @@ struct Flash : FlashCap<CAP, R> {
                     n.residuals += uint32_t(upper);
                     first = upper;
                 }
-                for (; first < 30 && !accepted; first += GROUP) {
-                    const bool counted = first + groupLane() < 30;
+                bool moved = true;
+                for (; first < 30 && !accepted && moved; first += GROUP) {
+                    bool counted = first + groupLane() < 30;
                     const R fraction = R(::ldexp(1.0, -lo(first + groupLane(), 29)));
                     const Counts before = n;
                     const Memo entry = memoNow();
                     R tx[3], tf[3] = {};
                     for (int j = 0; j < 3; ++j) tx[j] = x[j] + fraction * step[j];
+                    if constexpr (P::single) {  // no movement now or at any smaller fraction
+                        const bool moves = !(tx[0] == x[0] && tx[1] == x[1] && tx[2] == x[2]);
+                        counted = counted && moves;
+                        moved = !groupBallot(!moves);
+                    }
                     E trial;
                     zeroEval(trial);
                     const bool evaluated = residual(tx, scale, tf, &trial);
@@ -1476,6 +1508,10 @@ struct Flash : FlashCap<CAP, R> {
                 }
                 if constexpr (P::single)  // FP32 search: no movement now or at any smaller fraction
                     if (tx[0] == x[0] && tx[1] == x[1] && tx[2] == x[2]) break;
+                if constexpr (P::single) {
+                    overrun = n.phases > phaseLimit;
+                    if (overrun) return false;
+                }
                 E trial;
                 if (residual(tx, scale, tf, &trial) &&
                     hi(hi(hi(R(0), ab(tf[0])), ab(tf[1])), ab(tf[2])) < previous * (R(1) - R(1e-4) * fraction)) {
@@ -1890,7 +1926,7 @@ struct Flash : FlashCap<CAP, R> {
         }
         E candidate;
         const bool ok = frozen(liquid ? q[mod().condensable] : R(0), candidate, 0);
-        if (!ok && !stalled) return 0;
+        if (overrun || (!ok && !stalled)) return 0;
         x[0] = m_log(candidate.p);
         x[1] = m_log(candidate.T);
         x[2] = 0;

@@ -235,13 +235,14 @@ struct StartRecord {
     uint32_t bits;
 };
 // Scratch of the search: kStarts records per listed cell (record s of list
-// position i at s stride + i), the cells to restart, and the directed
-// search's two-phase cells to try again and one-phase cells; the counts are
-// zero on entry.
+// position i at s stride + i), the cells to restart (two species: before that
+// the slow starts, up to kStarts per listed cell), and the directed search's
+// two-phase cells to try again and one-phase cells; the counts are zero on
+// entry.
 struct SearchScratch {
     StartRecord* records;
     uint32_t *restarts, *again, *single;
-    unsigned *restartCount, *againCount, *singleCount;
+    unsigned *restartCount, *againCount, *singleCount, *slowCount;
 };
 // FP64 refinement of a directed search's two-phase points.  Cells without a
 // point go to the list `search`; one-phase cells, and those whose point takes

@@ -112,9 +112,9 @@ __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineKernel(con
     addTotals(n, succeeded, totals);
 }
 
-// deferred cells, cells to search, to restart, to try again, one-phase cells
+// deferred cells, cells to search, to restart, to try again, one-phase cells, slow starts
 __global__ void clearCountsKernel(unsigned* __restrict__ counts) {
-    if (threadIdx.x < 5) counts[threadIdx.x] = 0;
+    if (threadIdx.x < 6) counts[threadIdx.x] = 0;
 }
 
 // totals[k] = sum over b < blocks of partials[b * width + k], k < width: one
@@ -217,11 +217,12 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
     if (!count) return;
     if (!sets) {
         queue = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
-        queueCount = static_cast<unsigned*>(allocate(5 * sizeof(unsigned)));
+        queueCount = static_cast<unsigned*>(allocate(6 * sizeof(unsigned)));
         if (!prune) {
             scratch.records = static_cast<StartRecord*>(allocate(kStarts * capacity * sizeof(StartRecord)));
-            scratch.restarts = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
+            scratch.restarts = static_cast<uint32_t*>(allocate((ns > 1 ? kStarts : 1) * capacity * sizeof(uint32_t)));
             scratch.restartCount = queueCount + 2;
+            scratch.slowCount = queueCount + 5;
         }
         if (pure()) {
             searchList = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));

@@ -19,6 +19,10 @@
 #ifndef RAMD_LEAN_MIN_WAVES
 #define RAMD_LEAN_MIN_WAVES 4
 #endif
+// Phase evaluations after which a start's solve by one lane is given up.
+#ifndef RAMD_SLOW_PHASES
+#define RAMD_SLOW_PHASES 64
+#endif
 
 namespace ramd {
 
@@ -51,12 +55,14 @@ __global__ __launch_bounds__(256, RAMD_SEARCH_MIN_WAVES) void searchKernel(
 // solves rather than the longest sum of seven (and of the twenty restarts,
 // which now run only for the cells that need them, see below).  Bound by the
 // latency of the few solves that crawl, not by arithmetic: a 12^3 box's
-// search took 18 ms sequentially.
+// search took 18 ms sequentially.  With two species, starts that crawl (past
+// RAMD_SLOW_PHASES phase evaluations; one that arrives takes about 25) are
+// given up and listed for searchSlowKernel.
 template <int NS, int NL>
 __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchStartsKernel(
     const HemModel<NS>* __restrict__ globalModel, FlashCells cells, CellList list, size_t stride,
-    const CandidateSet* __restrict__ directed, StartRecord* __restrict__ records,
-    unsigned long long* __restrict__ phases) {
+    const CandidateSet* __restrict__ directed, StartRecord* __restrict__ records, uint32_t* __restrict__ slow,
+    unsigned* __restrict__ slowCount, unsigned long long* __restrict__ phases) {
     const uint32_t count = list.size();
     if (blockIdx.x * 64u >= count) return;  // uniform per workgroup
     const HemModel<NS>& model = workgroupModel(globalModel);
@@ -68,12 +74,54 @@ __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchStartsKernel(
             Flash<NS, NL, float, true, false, false, kModelLds> f(model, n);
             cells.load<NS>(f, list.cells[i]);
             StartRecord r;
+            if (NS > 1 && stride <= size_t(1) << 29) f.phaseLimit = RAMD_SLOW_PHASES;  // (an entry's position)
             if (blockIdx.y >= 2) r.bits = f.searchSeed(int(blockIdx.y), r.x);
             else if (directed && (directed[list.cells[i]].flags & (blockIdx.y ? kNotLiquid : kNotGas))) r.bits = 0;
             else r.bits = f.searchFrozen(blockIdx.y == 1, r.x);
+            if (NS > 1 && f.overrun) {
+                slow[atomicAdd(slowCount, 1u)] = i * 8u + blockIdx.y;
+                continue;
+            }
             r.bits |= n.phases << 2;
             records[size_t(blockIdx.y) * stride + i] = r;
             total += n.phases;
+        }
+    }
+    const uint32_t sum = waveSum(total);
+    if (threadIdx.x == 0) atomicAdd(phases, (unsigned long long)sum);
+}
+
+// The listed (list position, start) pairs, one per group of eight lanes: a
+// line search tries eight fractions at a time and the difference Jacobian its
+// six points, as the solve of one lane would one after the other.  A crawling
+// start's latency (ninety iterations of up to thirty fractions) is what the
+// search of a small or mid-size batch waits for: 40^3 binary cells 55 ms on
+// one lane per start, now 26 with both kernels.  A pure fluid's few starts
+// without a table point (47^3 cells) end as soon on one lane, 3.2 ms against
+// 3.6, and are not listed.
+template <int NS, int NL>
+__global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchSlowKernel(
+    const HemModel<NS>* __restrict__ globalModel, FlashCells cells, CellList list, size_t stride,
+    StartRecord* __restrict__ records, const uint32_t* __restrict__ slow, const unsigned* __restrict__ slowCount,
+    unsigned long long* __restrict__ phases) {
+    const uint32_t count = *slowCount;
+    if (blockIdx.x * 8u >= count) return;  // uniform per workgroup
+    const HemModel<NS>& model = workgroupModel(globalModel);
+    uint32_t total = 0;
+    for (uint32_t base = blockIdx.x * 8u; base < count; base += gridDim.x * 8u) {
+        const uint32_t k = base + threadIdx.x / 8u;
+        if (k < count) {
+            const uint32_t i = slow[k] / 8u, start = slow[k] % 8u;
+            Counts n = {0, 0, 0, 0, 0, 0, 0};
+            Flash<NS, NL, float, true, false, false, kModelLds, 8> f(model, n);
+            cells.load<NS>(f, list.cells[i]);
+            StartRecord r;
+            r.bits = start >= 2 ? f.searchSeed(int(start), r.x) : f.searchFrozen(start == 1, r.x);
+            r.bits |= n.phases << 2;
+            if (threadIdx.x % 8u == 0) {
+                records[size_t(start) * stride + i] = r;
+                total += n.phases;
+            }
         }
     }
     const uint32_t sum = waveSum(total);
@@ -118,38 +166,40 @@ __global__ __launch_bounds__(256) void searchMergeKernel(const HemModel<NS>* __r
     }
 }
 
-// The twenty restarts of the listed cells, three cells per wave and one
-// restart per lane, appended to the cells' sets in search order.
+// The twenty restarts of the listed cells, a cell per workgroup of three
+// waves and a restart per group of eight lanes (as searchSlowKernel), appended
+// to the cells' sets in search order.  40^3 binary cells: 40 ms with a restart
+// per lane, 14.5 so; 47^3 cells of a pure fluid: 0.44 and 0.11 ms.
 template <int NS, int NL>
-__global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchRestartsKernel(
+__global__ __launch_bounds__(192, RAMD_SEARCH_MIN_WAVES) void searchRestartsKernel(
     const HemModel<NS>* __restrict__ globalModel, FlashCells cells, CellList list, CandidateSet* __restrict__ sets,
     uint16_t* __restrict__ cost, unsigned long long* __restrict__ phases) {
     const uint32_t count = list.size();
-    if (blockIdx.x * 3u >= count) return;  // uniform per workgroup
+    if (blockIdx.x >= count) return;  // uniform per workgroup
     const HemModel<NS>& model = workgroupModel(globalModel);
-    __shared__ StartRecord found[64];
+    __shared__ StartRecord found[kRestarts];
     uint32_t total = 0;
-    const uint32_t cell = threadIdx.x / kRestarts, s = threadIdx.x % kRestarts;
-    for (uint32_t base = blockIdx.x * 3u; base < count; base += gridDim.x * 3u) {  // uniform per workgroup
-        const uint32_t i = base + cell;
-        const bool active = cell < 3 && i < count;
-        if (active) {
+    const uint32_t s = threadIdx.x / 8u;
+    for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {  // uniform per workgroup
+        if (s < kRestarts) {
             Counts n = {0, 0, 0, 0, 0, 0, 0};
-            Flash<NS, NL, float, true, false, false, kModelLds> f(model, n);
+            Flash<NS, NL, float, true, false, false, kModelLds, 8> f(model, n);
             cells.load<NS>(f, list.cells[i]);
             StartRecord r;
             r.bits = f.searchSeed(kStarts + int(s), r.x);
             r.bits |= n.phases << 2;
-            found[threadIdx.x] = r;
-            total += n.phases;
+            if (threadIdx.x % 8u == 0) {
+                found[s] = r;
+                total += n.phases;
+            }
         }
         __syncthreads();
-        if (active && s == 0) {
+        if (threadIdx.x == 0) {
             const uint32_t c = list.cells[i];
             CandidateSet set = sets[c];
             uint32_t evaluations = 0;
             for (int k = 0; k < kRestarts; ++k) {
-                const StartRecord r = found[threadIdx.x + k];
+                const StartRecord r = found[k];
                 evaluations += r.bits >> 2;
                 if (r.bits & kStartFound) noteCandidate(set, kRestartCandidate, int16_t(k), r.x, true);
             }
@@ -162,7 +212,7 @@ __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchRestartsKerne
         __syncthreads();
     }
     const uint32_t sum = waveSum(total);
-    if (threadIdx.x == 0) atomicAdd(phases, (unsigned long long)sum);
+    if (threadIdx.x % 64u == 0) atomicAdd(phases, (unsigned long long)sum);
 }
 
 // ---- a pure fluid's search, directed by its saturation curve --------------
@@ -476,12 +526,15 @@ void launchSearchStarts(int ns, int nl, const void* model, const FlashCells& cel
 #define RAMD_STARTS(NS_, NL_)                                                                                \
     hipLaunchKernelGGL((searchStartsKernel<NS_, NL_>), dim3(blocks, kStarts), dim3(64), 0, stream,            \
                        static_cast<const HemModel<NS_>*>(model), cells, list, stride,                                   \
-                       directed ? sets : nullptr, scratch.records, phases);                                   \
+                       directed ? sets : nullptr, scratch.records, scratch.restarts, scratch.slowCount, phases); \
+    if (NS_ > 1) hipLaunchKernelGGL((searchSlowKernel<NS_, NL_>), dim3(unsigned(std::min(size_t(kListWaves), (stride * kStarts + 7) / 8))), dim3(64), 0, \
+                       stream, static_cast<const HemModel<NS_>*>(model), cells, list, stride, scratch.records, \
+                       scratch.restarts, scratch.slowCount, phases);                                          \
     hipLaunchKernelGGL((searchMergeKernel<NS_>), dim3(std::min(2048u, (waves + 3) / 4)), dim3(256), 0, stream, \
                        static_cast<const HemModel<NS_>*>(model), cells, list, stride, scratch.records, sets, cost, \
                        scratch.restarts, scratch.restartCount);                                              \
     hipLaunchKernelGGL((searchRestartsKernel<NS_, NL_>),                                                      \
-                       dim3(std::min(kListWaves, unsigned((stride + 2) / 3))), dim3(64), 0, stream,           \
+                       dim3(unsigned(std::min(size_t(kListWaves), stride))), dim3(192), 0, stream,            \
                        static_cast<const HemModel<NS_>*>(model), cells,                                       \
                        CellList{scratch.restarts, 0, scratch.restartCount}, sets, cost, phases)
     RAMD_SPECIES(RAMD_STARTS)

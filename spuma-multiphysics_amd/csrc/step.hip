@@ -37,8 +37,8 @@ namespace ramd {
 
 // ---------------------------------------------------------------- kernels
 // Counts of the mixed flash's lists: deferred cells, cells to search, cells to restart,
-// cells the directed search tries again, one-phase cells.
-constexpr int kQueueCounts = 5;
+// cells the directed search tries again, one-phase cells, slow starts.
+constexpr int kQueueCounts = 6;
 
 // Plain FP64 flash of the cells in `order`; RJ: the model's
 // analytic-Jacobian mode.
@@ -1319,8 +1319,9 @@ int reactive_amd_step_run(void* step, double cfl, double maximum, int steps, int
             if (!s.h->prune) {
                 // one record per start and cell; a pure fluid searches only the cells its table leaves
                 s.scratch.records = s.alloc<StartRecord>(kStarts * s.cells);
-                s.scratch.restarts = s.alloc<uint32_t>(s.cells);
+                s.scratch.restarts = s.alloc<uint32_t>((s.h->ns > 1 ? kStarts : 1) * s.cells);
                 s.scratch.restartCount = s.queueCount + 2;
+                s.scratch.slowCount = s.queueCount + 5;
             }
             if (s.h->pure()) {
                 s.searchList = s.alloc<uint32_t>(s.cells);
