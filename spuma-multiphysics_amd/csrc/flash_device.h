@@ -408,6 +408,25 @@ struct Flash : FlashCap<CAP, R> {
     // evaluations, for a group of lanes to do instead
     uint32_t phaseLimit;
     bool overrun;
+    // The deferred cells' flash: its restarts on the groups of all waves of a
+    // workgroup, which the first wave calls on through LDS (see searchWide).
+    static constexpr bool kWide = GROUP > 1 && A && !P::single;
+    struct Memo {  // the flash's memo (the last unavailable liquid's point)
+        R p, T;
+        int status, virtualLiquids;
+    };
+    struct WideStart {
+        Counts n;
+        uint32_t bits;
+        Memo memo;
+        R p, T;
+    };
+    struct Wide {
+        int restarts;  // whether the other waves are called on, or the cell is done
+        WideStart start[kRestarts];
+        E candidate[kRestarts];
+    };
+    Wide* wide;
 
     RD Flash(const HemModel<NS>& model, Counts& counts) : m(model), n(counts) {
         cacheP = cacheT = 0;
@@ -423,6 +442,7 @@ struct Flash : FlashCap<CAP, R> {
         stalled = false;
         phaseLimit = ~0u;
         overrun = false;
+        wide = nullptr;
     }
     // GROUP: this lane's place in its group, the group's first lane, a ballot
     // over the group and a group lane's value.
@@ -439,11 +459,6 @@ struct Flash : FlashCap<CAP, R> {
         for (int o = GROUP / 2; o > 0; o >>= 1) v += uint32_t(__shfl_xor(int(v), o, 64));
         return v;
     }
-    // The flash's memo (the last unavailable liquid's point).
-    struct Memo {
-        R p, T;
-        int status, virtualLiquids;
-    };
     RD Memo memoNow() const { return {cacheP, cacheT, cacheStatus, int(cacheVirtual)}; }
     RD void memoSet(const Memo& v) {
         cacheP = v.p;
@@ -1779,7 +1794,15 @@ struct Flash : FlashCap<CAP, R> {
         Memo memo = memoNow();
         const auto seedAt = [](int j) { return j == 0 ? R(-1) : j == 1 ? R(.5) : j == 2 ? R(.95) : j == 3 ? R(.1) : R(.9999); };
         for (int round = firstRound; round < 4; ++round) {
-            if (round == 1 && (have || !seeded || !restartRange())) break;
+            if (round == 1) {
+                const bool stop = have || !seeded || !restartRange();
+                if constexpr (kWide) {  // (a scalar branch around the workgroup's barriers)
+                    if (!__builtin_amdgcn_readfirstlane(int(stop))) have = searchWide(best, total, memo);
+                    break;
+                } else if (stop) {
+                    break;
+                }
+            }
             E candidate;
             zeroEval(candidate);
             bool ok = false;
@@ -1839,6 +1862,73 @@ struct Flash : FlashCap<CAP, R> {
         n = total;
         memoSet(memo);
         return have;
+    }
+    // Restart `restart` of the cell on this lane's group, its outcome in LDS.
+    RAMD_NOINLINE void wideRestart(int restart) {
+        const Counts none = {0, 0, 0, 0, 0, 0, 0};
+        n = none;
+        cacheStatus = -1;
+        if (restart >= kRestarts) return;
+        const int j = restart % 5;
+        E candidate;
+        zeroEval(candidate);
+        const bool ok = activeFlash(j == 0 ? R(-1) : j == 1 ? R(.5) : j == 2 ? R(.95) : j == 3 ? R(.1) : R(.9999),
+                                    candidate, true, restartTemperature(restart / 5));
+        R first[3] = {}, scale;
+        activeStart(R(.5), true, restartTemperature(restart / 5), first, scale);
+        const bool good = ok && stable(candidate);
+        if (groupLane() == 0) {
+            WideStart& o = wide->start[restart];
+            o.n = n;
+            o.bits = good ? 1u : 0u;
+            o.memo = memoNow();
+            o.p = m_exp(first[0]);
+            o.T = m_exp(first[1]);
+            if (good) wide->candidate[restart] = candidate;
+        }
+    }
+    // The twenty restarts at once, on the groups of the workgroup's three
+    // waves, selected and counted in the sequence's order.  The first wave
+    // calls this; the others wait in wideWorker.
+    RD bool searchWide(E& best, Counts& total, Memo& memo) {
+        if (threadIdx.x == 0) wide->restarts = 1;
+        __syncthreads();
+        wideRestart(int(threadIdx.x) / GROUP);
+        __syncthreads();
+        int winner = -1;
+        R entropy = 0;
+        for (int k = 0; k < kRestarts; ++k) {
+            const WideStart& r = wide->start[k];
+            const bool spared = memo.status >= 0 && memo.p == r.p && memo.T == r.T && memo.virtualLiquids != 0;
+            total.phases += spared ? 0u : r.n.phases;
+            total.residuals += r.n.residuals;
+            total.candidates += r.n.candidates;
+            total.fd += r.n.fd;
+            total.analytic += r.n.analytic;
+            if (!spared && r.memo.status >= 0) memo = r.memo;
+            if (r.bits) {
+                ++total.stable;
+                const R s = wide->candidate[k].entropyDensity;
+                if (winner < 0 || s > entropy) { entropy = s; winner = k; }
+            } else {
+                ++total.failures;
+            }
+        }
+        if (winner >= 0) best = wide->candidate[winner];
+        return winner >= 0;
+    }
+    // The other waves' part of a cell, and how the first wave ends it.
+    RD void wideWorker() {
+        for (;;) {
+            __syncthreads();
+            if (!wide->restarts) break;
+            wideRestart(int(threadIdx.x) / GROUP);
+            __syncthreads();
+        }
+    }
+    RD void wideDone() {
+        if (threadIdx.x == 0) wide->restarts = 0;
+        __syncthreads();
     }
     RD bool searchRestarts(E& best) {
         if constexpr (GROUP > 1) {
