@@ -5,6 +5,12 @@
 # Stack slots are not shared: where the lanes of a wave take both sides of a
 # branch around calls, the compiler keeps the scalar registers that one side
 # saves (stores of all 64 lanes) in slots that lanes of the other side still use.
+# lanes.hip: the registers that hold saved scalars are allocated without
+# splitting (-wwm-regalloc=basic).  A split's copy runs for all 64 lanes, and
+# the ordinary allocation puts single lanes' moves and spills inside it (up to
+# 42 instructions in the FP64 flash's frozen solve), which overwrote other
+# lanes' values: a batch of binary cells, one per lane, read a wild pointer.
+# The other files' kernels have no such copy with anything inside it.
 set -euo pipefail
 here="$(cd -- "$(dirname -- "${BASH_SOURCE[0]}")" && pwd)"
 hipcc="${HIPCC:-/opt/rocm/bin/hipcc}"
@@ -21,6 +27,7 @@ for src in "$here"/csrc/*.hip; do
   extra=()
   # the FP32 candidate search may use approximate reciprocals and transcendentals
   if [ "$(basename "$src")" = "search.hip" ]; then extra=(-freciprocal-math -fapprox-func); fi
+  if [ "$(basename "$src")" = "lanes.hip" ]; then extra=(-mllvm -wwm-regalloc=basic); fi
   "$hipcc" "${flags[@]}" "${extra[@]}" -c "$src" -o "$obj" 2> >(grep -v "packed-fp32-ops" >&2) &
   objs+=("$obj")
   pids+=("$!")

@@ -24,6 +24,7 @@
 #include "model_image.h"
 #include "hem_internal.h"
 #include "flash_step.h"
+#include "lane_flash.h"
 #include "reactive_gpu_hem.h"
 #include "reactive_amd.h"
 
@@ -36,45 +37,6 @@ static_assert(sizeof(HemCapillaryDev) == sizeof(ReactiveGpuHemCapillaryInputV2) 
 static_assert(sizeof(HemOutputDev) == sizeof(ReactiveGpuHemOutputV1) &&
                   offsetof(HemOutputDev, success) == offsetof(ReactiveGpuHemOutputV1, success),
               "output layout");
-
-// One cell per lane (runHemCell).  RJ: the model's analytic-Jacobian mode
-// (analyticJacobian = 1); CAP: the capillary / boundary-search flash, for
-// capillary input and boundaryRecovery models.
-template <int NS, int NL, bool RJ, bool CAP>
-__global__ __launch_bounds__(64, RAMD_FLASH_MIN_WAVES) void hemFlashKernel(const HemModel<NS>* __restrict__ globalModel,
-                                                     FlashCells cells, const uint32_t* __restrict__ order, uint32_t count,
-                                                     const HemCapillaryDev* __restrict__ capillary,
-                                                     HemOutputDev* __restrict__ out,
-                                                     unsigned long long* __restrict__ totals,
-                                                     unsigned long long* __restrict__ partials) {
-    const HemModel<NS>& model = workgroupModel(globalModel);
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    Counts n = {0, 0, 0, 0, 0, 0, 0};
-    uint32_t succeeded = 0;
-    if (i < count) {
-        const uint32_t c = order ? order[i] : i;
-        using F = Flash<NS, NL, double, false, RJ, CAP, kModelLds>;
-        F f(model, n);
-        cells.load<NS>(f, c);
-        typename F::E result;
-        zeroEval(result);
-        const bool ok = runHemCell<CAP, NL>(f, cells.seeds[c], capillary ? capillary + c : nullptr, result);
-        storeHemCell(ok, result, out[c]);
-        succeeded = ok ? 1u : 0u;
-    }
-    if (partials) {  // one 64-lane workgroup: its eight sums go to its own slot
-        const uint32_t s0 = waveSum(n.phases), s1 = waveSum(n.residuals), s2 = waveSum(n.candidates);
-        const uint32_t s3 = waveSum(n.stable), s4 = waveSum(n.failures), s5 = waveSum(n.fd);
-        const uint32_t s6 = waveSum(succeeded), s7 = waveSum(n.analytic);
-        if (threadIdx.x == 0) {
-            unsigned long long* slot = partials + size_t(blockIdx.x) * 8;
-            slot[0] = s0; slot[1] = s1; slot[2] = s2; slot[3] = s3;
-            slot[4] = s4; slot[5] = s5; slot[6] = s6; slot[7] = s7;
-        }
-    } else if (totals) {
-        addTotals(n, succeeded, totals);
-    }
-}
 
 // Mixed arithmetic, second half: FP64 refinement, stability and selection of
 // the listed cells' candidates; deferred cells go to the queue, or, where the
@@ -192,21 +154,14 @@ unsigned HemHandle::launch(const double* q, const double* e, const ThermoOut* g,
         launchGroupFlash(ns, nl, analytic, boundary, model, cells, order, uint32_t(count), capillary, sink, s);
         return unsigned(count);
     }
-#define RAMD_HEM_LAUNCH(NS_, NL_, RJ_, CAP_)                                                                       \
-    hipLaunchKernelGGL((hemFlashKernel<NS_, NL_, RJ_, CAP_>), dim3(blocks), dim3(64), 0, s,                        \
+#define RAMD_HEM_LAUNCH(NS_, NL_)                                                                                  \
+    hipLaunchKernelGGL((hemFlashKernel<NS_, NL_, false, false>), dim3(blocks), dim3(64), 0, s,                     \
                        static_cast<const HemModel<NS_>*>(model), cells, order, uint32_t(count), capillary, out,    \
                        totals, partials)
-#define RAMD_HEM_SPECIES(CAP_)                                                                                    \
-    if (ns == 1 && nl == 0) RAMD_HEM_LAUNCH(1, 0, false, CAP_);                                                   \
-    else if (ns == 1 && !analytic) RAMD_HEM_LAUNCH(1, 1, false, CAP_);                                            \
-    else if (ns == 1) RAMD_HEM_LAUNCH(1, 1, true, CAP_);                                                          \
-    else if (nl == 0) RAMD_HEM_LAUNCH(2, 0, false, CAP_);                                                         \
-    else if (!analytic) RAMD_HEM_LAUNCH(2, 1, false, CAP_);                                                       \
-    else RAMD_HEM_LAUNCH(2, 1, true, CAP_);
-    // the capillary / boundary-search flash for interface input and boundaryRecovery models
-    if (capillary || boundary) { RAMD_HEM_SPECIES(true) }
-    else { RAMD_HEM_SPECIES(false) }
-#undef RAMD_HEM_SPECIES
+    if (capillary || boundary || ns != 1 || (nl && analytic))
+        launchLaneHem(ns, nl, analytic, boundary, model, cells, order, uint32_t(count), capillary, out, totals, partials, s);
+    else if (nl == 0) RAMD_HEM_LAUNCH(1, 0);
+    else RAMD_HEM_LAUNCH(1, 1);
 #undef RAMD_HEM_LAUNCH
     RAMD_HIP(hipGetLastError());
     return blocks;

@@ -31,6 +31,7 @@
 #include "transport_internal.h"
 #include "cartesian_kernels.h"
 #include "flash_step.h"
+#include "lane_flash.h"
 #include "reactive_amd.h"
 
 namespace ramd {
@@ -39,37 +40,6 @@ namespace ramd {
 // Counts of the mixed flash's lists: deferred cells, cells to search, cells to restart,
 // cells the directed search tries again, one-phase cells, slow starts.
 constexpr int kQueueCounts = 6;
-
-// Plain FP64 flash of the cells in `order`; RJ: the model's
-// analytic-Jacobian mode.
-template <int NS, int NL, bool RJ>
-__global__ __launch_bounds__(256, RAMD_FLASH_MIN_WAVES) void stepFlashKernel(const HemModel<NS>* __restrict__ globalModel,
-                                                      FlashCells cells,
-                                                      const uint32_t* __restrict__ order, uint32_t count,
-                                                      ThermoOut* __restrict__ out,
-                                                      double* __restrict__ pOut, double* __restrict__ cOut,
-                                                      double* __restrict__ rOut, uint16_t* __restrict__ cost,
-                                                      unsigned long long* __restrict__ counters,
-                                                      uint8_t* __restrict__ failMark) {
-    const HemModel<NS>& model = workgroupModel(globalModel);
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    Counts n = {0, 0, 0, 0, 0, 0};
-    uint32_t failed = 0;
-    if (i < count && cells.flashed(order[i])) {
-        const uint32_t c = order[i];
-        using F = Flash<NS, NL, double, false, RJ, false, kModelLds>;
-        F f(model, n);
-        cells.load<NS>(f, c);
-        typename F::E result;
-        zeroEval(result);
-        const bool ok = f.run(result);
-        storeCell(ok, result, cells.seeds[c], c, out, pOut, cOut, rOut);
-        if (!ok && failMark) failMark[c] = 1;
-        failed = ok ? 0u : 1u;
-        if (cost) cost[c] = uint16_t(n.phases < 65535u ? n.phases : 65535u);
-    }
-    countFlash(failed, n.phases, counters);
-}
 
 // Mixed precision, second half: FP64 refinement, stability and selection of
 // the listed cells' candidates.  Deferred cells go to the queue, or, where
@@ -812,10 +782,10 @@ struct Step {
                        cOut, rOut, costOut, counter, failMark)
             if (h->ns == 1 && h->nl == 0) { RAMD_STEP_FLASH(1, 0, false); }
             else if (h->ns == 1 && !h->analytic) { RAMD_STEP_FLASH(1, 1, false); }
-            else if (h->ns == 1) { RAMD_STEP_FLASH(1, 1, true); }
-            else if (h->nl == 0) { RAMD_STEP_FLASH(2, 0, false); }
-            else if (!h->analytic) { RAMD_STEP_FLASH(2, 1, false); }
-            else { RAMD_STEP_FLASH(2, 1, true); }
+            else {
+                launchLaneStep(h->ns, h->nl, h->analytic, h->model, batch, order, uint32_t(cells), sink, blocks, flashBlock,
+                               stream);
+            }
 #undef RAMD_STEP_FLASH
         }
         if (rep)
