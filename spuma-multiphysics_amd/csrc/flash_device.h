@@ -375,7 +375,7 @@ __device__ inline HemModel<NS>& sharedModel() {
 // of a wave.  Every lane of a group makes every call (lanes past a loop's end
 // repeat its last point).
 template <int NS, int NL, class R = double, bool A = FlashPrecision<R>::single, bool RJ = false, bool CAP = false,
-          bool LDS = false, int GROUP = 1>
+          bool LDS = false, int GROUP = 1, bool WIDE = false>
 struct Flash : FlashCap<CAP, R> {
     static_assert(NL == 0 || NL == 1, "one pure liquid at most");
     static_assert(!RJ || (!A && !FlashPrecision<R>::single), "the reference's analytic mode is an FP64 flash");
@@ -408,9 +408,8 @@ struct Flash : FlashCap<CAP, R> {
     // evaluations, for a group of lanes to do instead
     uint32_t phaseLimit;
     bool overrun;
-    // The deferred cells' flash: its restarts on the groups of all waves of a
-    // workgroup, which the first wave calls on through LDS (see searchWide).
-    static constexpr bool kWide = GROUP > 1 && A && !P::single;
+    // WIDE: the restarts run on the groups of all waves of a workgroup, which
+    // the first wave calls on through LDS (see searchWide).
     struct Memo {  // the flash's memo (the last unavailable liquid's point)
         R p, T;
         int status, virtualLiquids;
@@ -1796,7 +1795,7 @@ struct Flash : FlashCap<CAP, R> {
         for (int round = firstRound; round < 4; ++round) {
             if (round == 1) {
                 const bool stop = have || !seeded || !restartRange();
-                if constexpr (kWide) {  // (a scalar branch around the workgroup's barriers)
+                if constexpr (WIDE) {  // (a scalar branch around the workgroup's barriers)
                     if (!__builtin_amdgcn_readfirstlane(int(stop))) have = searchWide(best, total, memo);
                     break;
                 } else if (stop) {

@@ -29,6 +29,11 @@
 #ifndef RAMD_QUEUE_BLOCKS
 #define RAMD_QUEUE_BLOCKS 4096
 #endif
+// A queue of up to this many deferred cells gives each a workgroup of three
+// waves for its restarts, a longer one a wave.
+#ifndef RAMD_WIDE_CELLS
+#define RAMD_WIDE_CELLS 4096
+#endif
 // FP64 batches of up to this many cells run one cell per wave, its starts on
 // groups of eight lanes (group.hip); larger ones one cell per lane.
 #ifndef RAMD_GROUP_CELLS

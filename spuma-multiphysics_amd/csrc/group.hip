@@ -69,14 +69,14 @@ __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void groupFlashKernel(
 // in a flash of 40^3 binary cells, now 57.
 constexpr int kQueueThreads = 192;
 static_assert(kQueueThreads / 8 >= kRestarts, "a group per restart");
-template <int NS, int NL>
-__global__ __launch_bounds__(kQueueThreads, RAMD_REFINE_MIN_WAVES) void refineQueueKernel(
+template <int NS, int NL, bool WIDE>
+__global__ __launch_bounds__(WIDE ? kQueueThreads : 64, RAMD_REFINE_MIN_WAVES) void refineQueueKernel(
     const HemModel<NS>* __restrict__ globalModel, FlashCells cells, const uint32_t* __restrict__ queue,
     const unsigned* __restrict__ queueCount, const CandidateSet* __restrict__ sets, FlashSink sink) {
     const unsigned count = *queueCount;
-    if (blockIdx.x >= count) return;  // uniform per workgroup: usually every workgroup leaves here
+    if (blockIdx.x >= count || (NL > 0 && count <= RAMD_WIDE_CELLS) != WIDE) return;  // uniform per workgroup
     const HemModel<NS>& model = workgroupModel(globalModel);
-    using F = Flash<NS, NL, double, true, false, false, kModelLds, 8>;
+    using F = Flash<NS, NL, double, true, false, false, kModelLds, 8, WIDE>;
     __shared__ typename F::Wide wide;
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
     for (unsigned i = blockIdx.x; i < count; i += gridDim.x) {  // uniform per workgroup
@@ -84,17 +84,17 @@ __global__ __launch_bounds__(kQueueThreads, RAMD_REFINE_MIN_WAVES) void refineQu
         Counts n = {0, 0, 0, 0, 0, 0, 0};
         F f(model, n);
         cells.load<NS>(f, c);
-        f.wide = &wide;
-        if (wave == 0) {
+        if (WIDE) f.wide = &wide;
+        if (!WIDE || wave == 0) {
             EvalT<double, true> result;
             zeroEval(result);
             const bool ok = f.refine(sets[c], result);
-            f.wideDone();
+            if (WIDE) f.wideDone();
             storeGroup(sink, ok, result, cells, c, n);
         } else {
             f.wideWorker();
         }
-        __syncthreads();  // before the next cell's first call
+        if (WIDE) __syncthreads();  // before the next cell's first call
     }
 }
 
@@ -121,7 +121,9 @@ void launchGroupFlash(int ns, int nl, bool analytic, bool boundary, const void* 
 void launchRefineQueue(int ns, int nl, const void* model, const FlashCells& cells, const uint32_t* queue,
                        const unsigned* queueCount, const CandidateSet* sets, const FlashSink& sink, hipStream_t stream) {
 #define RAMD_QUEUE(NS_, NL_)                                                                                      \
-    hipLaunchKernelGGL((refineQueueKernel<NS_, NL_>), dim3(RAMD_QUEUE_BLOCKS), dim3(kQueueThreads), 0, stream,     \
+    if (NL_) hipLaunchKernelGGL((refineQueueKernel<NS_, NL_, true>), dim3(RAMD_WIDE_CELLS), dim3(kQueueThreads), 0, \
+                       stream, static_cast<const HemModel<NS_>*>(model), cells, queue, queueCount, sets, sink);   \
+    hipLaunchKernelGGL((refineQueueKernel<NS_, NL_, false>), dim3(RAMD_QUEUE_BLOCKS), dim3(64), 0, stream,         \
                        static_cast<const HemModel<NS_>*>(model), cells, queue, queueCount, sets, sink)
     if (ns == 1 && nl == 0) { RAMD_QUEUE(1, 0); }
     else if (ns == 1) { RAMD_QUEUE(1, 1); }
