@@ -307,12 +307,8 @@ def stage_roofline(rep, cells, steps, n, nv=5):
             "avg_launch_ms": [1e3 * rep.stageSeconds[0] / steps, 1e3 * rep.stageSeconds[1] / steps]}
 
 
-# HBM bytes per launch of the FP32 search at 160^3 pure N2O (the bench's
-# seeded box, mixed step, tuned launch shapes), from rocprofv3 FETCH_SIZE and
-# WRITE_SIZE scaled as below: profiles/stepSearch160_traffic.txt
-SEARCH_TRAFFIC_160 = 135.97e9
-# The source commit the profiles behind SEARCH_TRAFFIC_160, STAGE_TRAFFIC_160
-# and FLOP_PER_PHASE were measured on (reported with the rooflines).
+# The source commit the profiles behind STAGE_TRAFFIC_160 and FLOP_PER_PHASE
+# were measured on (reported with the rooflines).
 PROFILED_COMMIT = "4d905b9"
 
 # HBM bytes per launch of the fused stage kernel at 160^3 pure N2O, stage 0 and
@@ -325,7 +321,9 @@ GRAPH = 0x100  # REACTIVE_AMD_STEP_GRAPH
 # VALU FLOPs per phase evaluation (ADD, MUL, TRANS = 1, FMA = 2), measured with
 # rocprofv3 on divergence-free uniform cells, mean of a two-phase cell and a
 # gas cell: profiles/flash_valu_uniform32.txt.  The flash roofline's achieved
-# rate is phase evaluations x this figure / event-timed kernel time.
+# rate is phase evaluations x this figure / event-timed kernel time.  (An
+# evaluation has become cheaper since, two states sharing what they have in
+# common, so the rates are upper figures.)
 FLOP_PER_PHASE = {"fp64_flash": (1619 + 2115) / 2, "fp32_search": (370 + 523) / 2, "fp64_refine": (2253 + 1596) / 2}
 FP32_PEAK_TFLOPS = 157.3
 
@@ -382,10 +380,10 @@ def flash_roofline(rep, rep64, cells, steps, mixed):
         a32 = rep.singlePhaseEvaluations / flashes * FLOP_PER_PHASE["fp32_search"] / ts / 1e12
         ar = rep.phaseEvaluations / flashes * FLOP_PER_PHASE["fp64_refine"] / tr / 1e12
         out["avg_launch_ms"] = 1e3 * t
-        out["fp32_search"] = {"kernel": "stepSearchKernel", "avg_launch_ms": 1e3 * ts, "achieved": a32,
+        out["fp32_search"] = {"kernel": "FP32 search (directKernel, searchStartsKernel and their lists)", "avg_launch_ms": 1e3 * ts, "achieved": a32,
                               "peak": FP32_PEAK_TFLOPS, "frac": a32 / FP32_PEAK_TFLOPS,
                               "phase_evaluations_per_cell": rep.singlePhaseEvaluations / (cells * flashes)}
-        out["fp64_refine"] = {"kernel": "stepRefineKernel (+ stepRefineQueueKernel)", "avg_launch_ms": 1e3 * tr,
+        out["fp64_refine"] = {"kernel": "refineTwoPhaseKernel, stepRefineKernel, refineQueueKernel", "avg_launch_ms": 1e3 * tr,
                               "achieved": ar, "peak": FP64_PEAK_TFLOPS, "frac": ar / FP64_PEAK_TFLOPS,
                               "phase_evaluations_per_cell": rep.phaseEvaluations / (cells * flashes),
                               "queued_cells_per_flash": rep.queuedCells / flashes}
@@ -397,12 +395,11 @@ def flash_roofline(rep, rep64, cells, steps, mixed):
 
 
 def search_roofline(flash, rep, steps, n, case="n2o"):
-    """The dominant kernel: the FP32 candidate search of the mixed flash."""
+    """The FP32 candidate search of the mixed flash: bound by the latency of its solves."""
     s = flash["fp32_search"]
-    return {"bound": "valu", "kernel": "stepSearchKernel (FP32 candidate search of the mixed flash)",
+    return {"bound": "valu", "kernel": "FP32 candidate search of the mixed flash (directKernel, searchStartsKernel)",
             "achieved": s["achieved"], "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": s["frac"],
-            "traffic": SEARCH_TRAFFIC_160 if n == 160 and case == "n2o" else None,
-            "traffic_source": "profiles/stepSearch160_traffic.txt", "profiled_commit": PROFILED_COMMIT,
+            "traffic": None, "profiled_commit": PROFILED_COMMIT,
             "avg_launch_ms": s["avg_launch_ms"],
             "flop_per_phase_evaluation": FLOP_PER_PHASE["fp32_search"],
             "phase_evaluations_per_cell": s["phase_evaluations_per_cell"],

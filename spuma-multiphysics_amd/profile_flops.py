@@ -20,7 +20,7 @@ def kernels(db):
     per = defaultdict(lambda: defaultdict(lambda: defaultdict(float)))
     dur = defaultdict(dict)
     for did, name, d, counter, value in rows:
-        if "stepFlash" in name or "stepSearch" in name or "stepRefine" in name:
+        if any(k in name for k in ("stepFlash", "direct", "search", "stepRefine", "refineTwoPhase", "refineQueue")):
             key = name.split("<")[0].split("::")[-1]
             per[key][did][counter] += value
             dur[key][did] = d
