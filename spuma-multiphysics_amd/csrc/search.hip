@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256, RAMD_SEARCH_MIN_WAVES) void searchKernel(
 // solves rather than the longest sum of seven (and of the twenty restarts,
 // which now run only for the cells that need them, see below).  Bound by the
 // latency of the few solves that crawl, not by arithmetic: a 12^3 box's
-// search took 18 ms sequentially.  With two species, starts that crawl (past
+// search took 18 ms sequentially.  With two species and a liquid, starts that crawl (past
 // RAMD_SLOW_PHASES phase evaluations; one that arrives takes about 25) are
 // given up and listed for searchSlowKernel.
 template <int NS, int NL>
@@ -74,11 +74,11 @@ __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchStartsKernel(
             Flash<NS, NL, float, true, false, false, kModelLds> f(model, n);
             cells.load<NS>(f, list.cells[i]);
             StartRecord r;
-            if (NS > 1 && stride <= size_t(1) << 29) f.phaseLimit = RAMD_SLOW_PHASES;  // (an entry's position)
+            if (NS > 1 && NL && stride <= size_t(1) << 29) f.phaseLimit = RAMD_SLOW_PHASES;  // (an entry's position)
             if (blockIdx.y >= 2) r.bits = f.searchSeed(int(blockIdx.y), r.x);
             else if (directed && (directed[list.cells[i]].flags & (blockIdx.y ? kNotLiquid : kNotGas))) r.bits = 0;
             else r.bits = f.searchFrozen(blockIdx.y == 1, r.x);
-            if (NS > 1 && f.overrun) {
+            if (NS > 1 && NL && f.overrun) {
                 slow[atomicAdd(slowCount, 1u)] = i * 8u + blockIdx.y;
                 continue;
             }
@@ -169,7 +169,8 @@ __global__ __launch_bounds__(256) void searchMergeKernel(const HemModel<NS>* __r
 // The twenty restarts of the listed cells, a cell per workgroup of three
 // waves and a restart per group of eight lanes (as searchSlowKernel), appended
 // to the cells' sets in search order.  40^3 binary cells: 40 ms with a restart
-// per lane, 14.5 so; 47^3 cells of a pure fluid: 0.44 and 0.11 ms.
+// per lane, 14.5 so; 47^3 cells of a pure fluid: 0.44 and 0.11 ms
+// (160^3: 0.41 and 0.70, of 11 ms a flash).
 template <int NS, int NL>
 __global__ __launch_bounds__(192, RAMD_SEARCH_MIN_WAVES) void searchRestartsKernel(
     const HemModel<NS>* __restrict__ globalModel, FlashCells cells, CellList list, CandidateSet* __restrict__ sets,
@@ -527,7 +528,7 @@ void launchSearchStarts(int ns, int nl, const void* model, const FlashCells& cel
     hipLaunchKernelGGL((searchStartsKernel<NS_, NL_>), dim3(blocks, kStarts), dim3(64), 0, stream,            \
                        static_cast<const HemModel<NS_>*>(model), cells, list, stride,                                   \
                        directed ? sets : nullptr, scratch.records, scratch.restarts, scratch.slowCount, phases); \
-    if (NS_ > 1) hipLaunchKernelGGL((searchSlowKernel<NS_, NL_>), dim3(unsigned(std::min(size_t(kListWaves), (stride * kStarts + 7) / 8))), dim3(64), 0, \
+    if constexpr (NS_ > 1 && NL_ > 0) hipLaunchKernelGGL((searchSlowKernel<NS_, NL_>), dim3(unsigned(std::min(size_t(kListWaves), (stride * kStarts + 7) / 8))), dim3(64), 0, \
                        stream, static_cast<const HemModel<NS_>*>(model), cells, list, stride, scratch.records, \
                        scratch.restarts, scratch.slowCount, phases);                                          \
     hipLaunchKernelGGL((searchMergeKernel<NS_>), dim3(std::min(2048u, (waves + 3) / 4)), dim3(256), 0, stream, \
