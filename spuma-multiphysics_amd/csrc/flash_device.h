@@ -24,6 +24,7 @@
 #define REACTIVE_AMD_FLASH_DEVICE_H
 #include <type_traits>
 #include "pr_device.h"
+#include "mixed_data.h"
 #include "flash_jacobian.h"
 
 // Inlining of the phase evaluation (knobs, per arithmetic: the FP32 search
@@ -189,34 +190,6 @@ RD void writeOut(const EvalT<double, A, RJ, C>& v, ThermoOut& o) {
     o.gasMass = v.gasMass; o.cp = v.cp; o.cv = v.cv;
     o.activeLiquids = v.active; o.iterations = v.iterations;
 }
-
-// Candidates of the single-precision search, in search order.
-enum CandidateKind : int16_t { kGasCandidate = 0, kLiquidCandidate = 1, kSeedCandidate = 2, kRestartCandidate = 3 };
-struct Candidate {
-    float x[3];     // ln p, ln T, liquid fraction (0 for the gas and all-liquid candidates)
-    int16_t kind;   // CandidateKind
-    int16_t index;  // seed j, or 5 t + j for restart temperature t
-};
-constexpr int kMaxCandidates = 6;
-enum CandidateFlags : uint32_t {
-    kRestartsSearched = 1u,  // the search ran the restart temperatures
-    kOverflow = 2u,          // more distinct candidates than the set holds
-    kSeedsPruned = 4u,       // the stable-gas pruning skipped the seeds
-    kDirect = 8u,            // the directed search's (saturation table): one candidate or none
-    kNotGas = 16u,           // with kDirect: the all-gas solve cannot lead to the equilibrium
-    kNotLiquid = 32u,        // with kDirect: nor can the all-liquid one
-    kSingle = 64u,           // with kDirect: the point has one phase
-};
-enum StartBits : uint32_t {
-    kStartFound = 1u,   // converged, or stalled near convergence
-    kStartStable = 2u,  // converged and stable in single precision
-};
-constexpr int kStarts = 7, kRestarts = 20;  // all gas, all liquid, five seeds; the seeds from four temperatures
-struct CandidateSet {
-    uint32_t count, flags;
-    Candidate c[kMaxCandidates];
-};
-static_assert(sizeof(CandidateSet) == 104, "candidate set layout");
 
 // Appends a converged candidate to the set; dedupe: unless one of its kind
 // lies within 1e-4 of it.

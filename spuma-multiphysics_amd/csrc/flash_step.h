@@ -236,40 +236,12 @@ void launchRefineQueue(int ns, int nl, const void* model, const FlashCells& cell
                        const unsigned* queueCount, const CandidateSet* sets, const FlashSink& sink, hipStream_t stream);
 
 // ---- candidates of the mixed flash (search.hip) ---------------------------
-// One start's outcome: the point, kStart* bits and the evaluations above them.
-struct StartRecord {
-    float x[3];
-    uint32_t bits;
-};
-// Scratch of the search: kStarts records per listed cell (record s of list
-// position i at s stride + i), the cells to restart (two species: before that
-// the slow starts, up to kStarts per listed cell), and the directed search's
-// two-phase cells to try again and one-phase cells; the counts are zero on
-// entry.
-struct SearchScratch {
-    StartRecord* records;
-    uint32_t *restarts, *again, *single;
-    unsigned *restartCount, *againCount, *singleCount, *slowCount;
-};
 // FP64 refinement of a directed search's two-phase points.  Cells without a
 // point go to the list `search`; one-phase cells, and those whose point takes
 // more than full Newton steps, are left to refine(), in scratch.single.
 void launchRefineTwoPhase(const void* model, const FlashCells& cells, const uint32_t* order, uint32_t count,
                           const CandidateSet* sets, const FlashSink& sink, const SearchScratch& scratch,
                           uint32_t* search, unsigned* searchCount, hipStream_t stream);
-// Saturated liquid and vapour at evenly spaced temperatures: specific volumes
-// and energies, ln p.  Interpolated between 2,048 rows over N2O's 161 K they
-// lie within 1e-6 of the curve except next to the critical point, inside the
-// refinement's one or two Newton steps.
-constexpr int kSaturationRows = 2048;
-struct SaturationRow {
-    double vl, vv, el, ev, lnp;
-};
-struct SaturationTable {
-    int count, pad;
-    double T0, dT;
-    SaturationRow row[kSaturationRows];
-};
 // The table of a one-species model with its liquid.
 void launchSaturation(const void* model, SaturationTable* table, hipStream_t stream);
 // The directed search of every cell in `order`: sets of one candidate or none, flagged kDirect.

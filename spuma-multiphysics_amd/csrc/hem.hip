@@ -74,9 +74,8 @@ __global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineKernel(con
     addTotals(n, succeeded, totals);
 }
 
-// deferred cells, cells to search, to restart, to try again, one-phase cells, slow starts
 __global__ void clearCountsKernel(unsigned* __restrict__ counts) {
-    if (threadIdx.x < 6) counts[threadIdx.x] = 0;
+    if (threadIdx.x < kListCounts) counts[threadIdx.x] = 0;
 }
 
 // totals[k] = sum over b < blocks of partials[b * width + k], k < width: one
@@ -170,50 +169,41 @@ unsigned HemHandle::launch(const double* q, const double* e, const ThermoOut* g,
 void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g, const uint32_t* order,
                             size_t count, HemOutputDev* out, hipStream_t s) {
     if (!count) return;
-    if (!sets) {
-        queue = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
-        queueCount = static_cast<unsigned*>(allocate(6 * sizeof(unsigned)));
-        if (!prune) {
-            scratch.records = static_cast<StartRecord*>(allocate(kStarts * capacity * sizeof(StartRecord)));
-            scratch.restarts = static_cast<uint32_t*>(allocate((ns > 1 ? kStarts : 1) * capacity * sizeof(uint32_t)));
-            scratch.restartCount = queueCount + 2;
-            scratch.slowCount = queueCount + 5;
-        }
-        if (pure()) {
-            searchList = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
-            scratch.again = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
-            scratch.againCount = queueCount + 3;
-            scratch.single = static_cast<uint32_t*>(allocate(capacity * sizeof(uint32_t)));
-            scratch.singleCount = queueCount + 4;
-            saturation = static_cast<SaturationTable*>(allocate(sizeof(SaturationTable)));
-            launchSaturation(model, saturation, s);
-        }
-        sets = static_cast<CandidateSet*>(allocate(capacity * sizeof(CandidateSet)));
+    mixed.need(ns, prune, pure(), capacity, [this](auto*& p, size_t n) {
+        if (!p) p = static_cast<std::remove_reference_t<decltype(p)>>(allocate(n * sizeof(*p)));
+    });
+    if (mixed.saturation && !mixed.tableMade) {
+        launchSaturation(model, mixed.saturation, s);
+        mixed.tableMade = true;
     }
+    const SearchScratch& scratch = mixed.search;
+    SaturationTable* const saturation = mixed.saturation;
+    CandidateSet* const sets = mixed.sets;
+    uint32_t *const queue = mixed.queue, *const searchList = mixed.searchList;
+    unsigned *const queueCount = mixed.counts + kDeferredCount, *const searchCount = mixed.counts + kSearchCount;
     const unsigned blocks = unsigned((count + 63) / 64);
     const FlashCells cells = {q, 0, e, g, nullptr, nullptr};
-    const CellList whole = {order, uint32_t(count), nullptr}, left = {searchList, 0, queueCount + 1};
+    const CellList whole = {order, uint32_t(count), nullptr}, left = {searchList, 0, searchCount};
     const CellList first = saturation ? CellList{scratch.single, 0, scratch.singleCount} : whole;
     FlashSink sink = {};
     sink.hem = out;
     sink.totals = totals;
     hipLaunchKernelGGL(zeroTotalsKernel, dim3(1), dim3(64), 0, s, totals, 10);
-    hipLaunchKernelGGL(clearCountsKernel, dim3(1), dim3(64), 0, s, queueCount);
+    hipLaunchKernelGGL(clearCountsKernel, dim3(1), dim3(64), 0, s, mixed.counts);
     if (saturation) launchDirect(model, saturation, cells, order, uint32_t(count), scratch, sets, nullptr, totals + 8, s);
     else if (prune) launchSearch(ns, nl, model, cells, order, uint32_t(count), sets, nullptr, totals + 8, s, 64);
     else launchSearchStarts(ns, nl, model, cells, whole, count, scratch, false, sets, nullptr, totals + 8, s);
     if (saturation)
-        launchRefineTwoPhase(model, cells, order, uint32_t(count), sets, sink, scratch, searchList,
-                             queueCount + 1, s);
+        launchRefineTwoPhase(model, cells, order, uint32_t(count), sets, sink, scratch, searchList, searchCount, s);
 #define RAMD_HEM_MIXED(NS_, NL_)                                                                                  \
     hipLaunchKernelGGL((hemRefineKernel<NS_, NL_>), dim3(blocks), dim3(64), 0, s,                                   \
                        static_cast<const HemModel<NS_>*>(model), cells, first, sets, out, totals, queue,          \
-                       queueCount, searchList, queueCount + 1);                                                   \
+                       queueCount, searchList, searchCount);                                                      \
     if (saturation) {                                                                                             \
         launchSearchStarts(ns, nl, model, cells, left, count, scratch, true, sets, nullptr, totals + 8, s);       \
         hipLaunchKernelGGL((hemRefineKernel<NS_, NL_>), dim3(std::min(2048u, blocks)), dim3(64), 0, s,              \
                            static_cast<const HemModel<NS_>*>(model), cells, left, sets, out, totals, queue,       \
-                           queueCount, searchList, queueCount + 1);                                               \
+                           queueCount, searchList, searchCount);                                                  \
     }
     if (ns == 1 && nl == 0) { RAMD_HEM_MIXED(1, 0); }
     else if (ns == 1) { RAMD_HEM_MIXED(1, 1); }

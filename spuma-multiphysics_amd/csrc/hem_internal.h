@@ -23,15 +23,9 @@ struct HemHandle {
     // phases residuals candidates stable failures fd successes analytic, then
     // (mixed arithmetic) FP32 phases and deferred cells
     unsigned long long* totals = nullptr;
-    // mixed arithmetic: candidate sets and the deferred-refinement queue
-    // (allocated on the first mixed batch), the last batch's FP32 phase
-    // evaluations and deferred cells
-    CandidateSet* sets = nullptr;
-    uint32_t* queue = nullptr;
-    unsigned* queueCount = nullptr;  // deferred cells; to search, to restart, to try again
-    SaturationTable* saturation = nullptr;
-    uint32_t* searchList = nullptr;
-    SearchScratch scratch = {};
+    // mixed arithmetic: candidate sets and lists (allocated on the first
+    // mixed batch), the last batch's FP32 phase evaluations and deferred cells
+    MixedScratch mixed;
     uint64_t lastSinglePhases = 0, lastQueued = 0;
     // host-path staging (allocated on the first host batch)
     bool hostReady = false;

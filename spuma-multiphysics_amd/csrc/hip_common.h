@@ -10,8 +10,10 @@
 namespace ramd {
 
 inline void hipCheck(hipError_t status, const char* what) {
-    if (status != hipSuccess)
+    if (status != hipSuccess) {
+        (void)hipGetLastError();  // reported here; the next launch's check must not find it again
         throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(status));
+    }
 }
 #define RAMD_HIP(call) ::ramd::hipCheck((call), #call)
 

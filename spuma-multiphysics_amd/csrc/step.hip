@@ -37,10 +37,6 @@
 namespace ramd {
 
 // ---------------------------------------------------------------- kernels
-// Counts of the mixed flash's lists: deferred cells, cells to search, cells to restart,
-// cells the directed search tries again, one-phase cells, slow starts.
-constexpr int kQueueCounts = 6;
-
 // Mixed precision, second half: FP64 refinement, stability and selection of
 // the listed cells' candidates.  Deferred cells go to the queue, or, where
 // the candidates came from the saturation table, to the list of cells to
@@ -85,7 +81,7 @@ __global__ __launch_bounds__(256, RAMD_REFINE_MIN_WAVES) void stepRefineKernel(c
 }
 
 __global__ void clearQueueKernel(unsigned* __restrict__ counts) {
-    if (threadIdx.x < kQueueCounts) counts[threadIdx.x] = 0;
+    if (threadIdx.x < kListCounts) counts[threadIdx.x] = 0;
 }
 __global__ void queueTotalKernel(const unsigned* __restrict__ count, unsigned long long* __restrict__ total) {
     if (threadIdx.x == 0) atomicAdd(total, (unsigned long long)*count);
@@ -644,14 +640,7 @@ struct Step {
     uint32_t* orderSearch = nullptr;
     uint16_t* costSearch = nullptr;
     bool haveCostSearch = false;
-    CandidateSet* sets = nullptr;
-    uint32_t* queue = nullptr;  // cells the refinement deferred
-    unsigned* queueCount = nullptr;  // kQueueCounts counts
-    // a pure fluid's saturation table and the cells it left to the search; the
-    // search's records and restart list
-    SaturationTable* saturation = nullptr;
-    uint32_t* searchList = nullptr;
-    SearchScratch scratch = {};
+    MixedScratch mixed;
     int mode = REACTIVE_AMD_FLASH_FP64;
     unsigned *bucketCount = nullptr, *bucketOffset = nullptr;
     // state order: bin keys, bin counts (kept zero between uses) and offsets, range
@@ -700,11 +689,17 @@ struct Step {
         allocations.push_back(p);
         return static_cast<T*>(p);
     }
+    // A buffer made on its first use.  Each of a group of buffers is asked for
+    // on every use, so that a use after one that ran out of memory between
+    // them makes the rest.
+    template <class T> void need(T*& p, size_t n) {
+        if (!p) p = alloc<T>(n);
+    }
 
     // Cell-major q on its way from or to the host (kept from the first load on).
     double* transferBuffer = nullptr;
     double* transfer() {
-        if (!transferBuffer) transferBuffer = alloc<double>(cells * nv);
+        need(transferBuffer, cells * nv);
         return transferBuffer;
     }
 
@@ -736,9 +731,14 @@ struct Step {
         sink.failMark = failMark;
         if (mode == REACTIVE_AMD_FLASH_MIXED) {
             const CellList whole = {order, uint32_t(cells), nullptr};
-            const CellList left = {searchList, 0, queueCount + 1};
+            const SearchScratch& scratch = mixed.search;
+            SaturationTable* const saturation = mixed.saturation;
+            CandidateSet* const sets = mixed.sets;
+            uint32_t *const queue = mixed.queue, *const searchList = mixed.searchList;
+            unsigned *const queueCount = mixed.counts + kDeferredCount, *const searchCount = mixed.counts + kSearchCount;
+            const CellList left = {searchList, 0, searchCount};
             uint16_t* searchCost = costOut ? costSearch : nullptr;
-            hipLaunchKernelGGL(clearQueueKernel, dim3(1), dim3(64), 0, stream, queueCount);
+            hipLaunchKernelGGL(clearQueueKernel, dim3(1), dim3(64), 0, stream, mixed.counts);
             if (saturation)
                 launchDirect(h->model, saturation, batch, orderSearch, uint32_t(cells), scratch, sets, searchCost,
                              counters + 6, stream);
@@ -753,14 +753,13 @@ struct Step {
 #define RAMD_STEP_REFINE(NS_, NL_)                                                                                 \
     hipLaunchKernelGGL((stepRefineKernel<NS_, NL_>), dim3(grid), dim3(block), 0, stream,                            \
                        static_cast<const HemModel<NS_>*>(h->model), batch, list, sets, out, pOut, cOut, rOut,      \
-                       costOut, counter, queue, queueCount, searchList, queueCount + 1,                     \
-                       failMark)
+                       costOut, counter, queue, queueCount, searchList, searchCount, failMark)
                 RAMD_STEP_SPECIES(RAMD_STEP_REFINE)
 #undef RAMD_STEP_REFINE
             };
             if (saturation) {
                 launchRefineTwoPhase(h->model, batch, orderSearch, uint32_t(cells), sets, sink, scratch,
-                                     searchList, queueCount + 1, stream);
+                                     searchList, searchCount, stream);
                 refine({scratch.single, 0, scratch.singleCount}, std::min(kListBlocks, blocksFor(cells, 64)), 64);
             } else {
                 refine(whole, blocks, flashBlock);
@@ -972,16 +971,14 @@ struct Step {
 // step-start state restored when the step cannot be completed.
 uint64_t attemptStep(Step& s, double cfl, double maximum, hipEvent_t* marks) {
     const int n = s.count;
-    if (!s.qKeep) {
-        s.qKeep = s.alloc<double>(s.all * s.nv);
-        s.pKeep = s.alloc<double>(s.all);
-        s.cKeep = s.alloc<double>(s.all);
-        s.rKeep = s.alloc<double>(s.all);
-        s.sKeep = s.alloc<ThermoOut>(s.cells);
-        s.failMarks = s.alloc<uint8_t>(s.cells);
-        s.boxFail = s.alloc<unsigned long long>(size_t(n));
-        s.limits = s.alloc<double>(size_t(n));
-    }
+    s.need(s.qKeep, s.all * s.nv);
+    s.need(s.pKeep, s.all);
+    s.need(s.cKeep, s.all);
+    s.need(s.rKeep, s.all);
+    s.need(s.sKeep, s.cells);
+    s.need(s.failMarks, s.cells);
+    s.need(s.boxFail, size_t(n));
+    s.need(s.limits, size_t(n));
     auto copy = [&](void* to, const void* from, size_t bytes) {
         RAMD_HIP(hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, s.stream));
     };
@@ -1282,36 +1279,22 @@ int reactive_amd_step_run(void* step, double cfl, double maximum, int steps, int
         require(!(retry && useGraph), "Retried steps run on the stream, not from a captured graph");
         require(flashMode == REACTIVE_AMD_FLASH_FP64 || flashMode == REACTIVE_AMD_FLASH_MIXED,
                 "Unknown flash arithmetic mode");
-        if (flashMode == REACTIVE_AMD_FLASH_MIXED && !s.sets) {
-            s.sets = s.alloc<CandidateSet>(s.cells);
-            s.queue = s.alloc<uint32_t>(s.cells);
-            s.queueCount = s.alloc<unsigned>(kQueueCounts);
-            if (!s.h->prune) {
-                // one record per start and cell; a pure fluid searches only the cells its table leaves
-                s.scratch.records = s.alloc<StartRecord>(kStarts * s.cells);
-                s.scratch.restarts = s.alloc<uint32_t>((s.h->ns > 1 ? kStarts : 1) * s.cells);
-                s.scratch.restartCount = s.queueCount + 2;
-                s.scratch.slowCount = s.queueCount + 5;
-            }
-            if (s.h->pure()) {
-                s.searchList = s.alloc<uint32_t>(s.cells);
-                s.scratch.again = s.alloc<uint32_t>(s.cells);
-                s.scratch.againCount = s.queueCount + 3;
-                s.scratch.single = s.alloc<uint32_t>(s.cells);
-                s.scratch.singleCount = s.queueCount + 4;
-                s.saturation = s.alloc<SaturationTable>(1);
-                launchSaturation(s.h->model, s.saturation, s.stream);
+        if (flashMode == REACTIVE_AMD_FLASH_MIXED) {
+            s.mixed.need(s.h->ns, s.h->prune, s.h->pure(), s.cells, [&s](auto*& p, size_t n) { s.need(p, n); });
+            if (s.mixed.saturation && !s.mixed.tableMade) {
+                launchSaturation(s.h->model, s.mixed.saturation, s.stream);
+                s.mixed.tableMade = true;
             }
         }
-        s.mode = flashMode;
-        if (reuse && !s.reuseTable) {
+        if (reuse) {
             uint32_t size = 1;
             while (size < 2 * s.cells) size <<= 1;
-            s.reuseTable = s.alloc<uint32_t>(size);
             s.reuseMask = size - 1;
-            s.reuseSlot = s.alloc<uint32_t>(s.cells);
-            s.reuseRep = s.alloc<uint32_t>(s.cells);
+            s.need(s.reuseTable, size);
+            s.need(s.reuseSlot, s.cells);
+            s.need(s.reuseRep, s.cells);
         }
+        s.mode = flashMode;
         s.rep = reuse ? s.reuseRep : nullptr;
         s.stateSide = s.stateSideOf[s.mode];
         s.stateLevels = s.stateLevelsOf[s.mode];
