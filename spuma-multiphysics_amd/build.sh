@@ -10,7 +10,9 @@
 # the ordinary allocation puts single lanes' moves and spills inside it (up to
 # 42 instructions in the FP64 flash's frozen solve), which overwrote other
 # lanes' values: a batch of binary cells, one per lane, read a wild pointer.
-# The other files' kernels have no such copy with anything inside it.
+# The other files' kernels have no such copy with anything inside it; a change
+# to the code around them can bring one (tests/test_whole_wave_registers.py
+# looks the built library over).
 set -euo pipefail
 here="$(cd -- "$(dirname -- "${BASH_SOURCE[0]}")" && pwd)"
 hipcc="${HIPCC:-/opt/rocm/bin/hipcc}"
