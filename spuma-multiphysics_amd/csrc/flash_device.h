@@ -502,39 +502,47 @@ struct Flash : FlashCap<CAP, R> {
     // What states at one temperature (and one pressure: the cubic's outer
     // roots) of one composition share: the gas probe's state at (T, rho) and
     // its check at (T, p), and, for one species with the same gas and liquid
-    // tables, the two phases of a mixture.
-    struct Shared {
+    // tables, the two phases of a mixture.  Whether a state shares anything
+    // (KEPT) is known at compile time: with a pointer that may be null the
+    // compiler kept the record on the stack (160^3 pure N2O in FP64: 432 ms
+    // a flash, now 388); with the ideal part kept for every state the search
+    // of two species is 5 % slower.
+    template <bool KEPT>
+    struct SharedT {
         M mx;
-        IdealT<NS, R> ideal;
+        IdealT<KEPT ? NS : 1, R> ideal;
         RootsT<R> r;
-        bool mixed, rooted;
+        bool mixed = false, rooted = false;
     };
+    using Shared = SharedT<true>;
+    using Alone = SharedT<false>;
     // Gas PR state at (T, p) on the gas root (evaluateTPTrusted, reactiveDevicePR.h:574-609).
-    // sh (may be null): what is known already, and kept for the next state;
-    // both: the cubic's smallest root too.
-    RAMD_NOINLINE int gasTP(R T, R p, const R* Y, S& s, R* mu) { return gasTPBody(T, p, Y, s, mu, nullptr, false); }
-    __device__ __attribute__((always_inline)) inline int gasTPBody(R T, R p, const R* Y, S& s, R* mu, Shared* sh,
+    // k: what is known already, and kept for the next state; both: the
+    // cubic's smallest root too.
+    RAMD_NOINLINE int gasTP(R T, R p, const R* Y, S& s, R* mu) {
+        Alone none;
+        return gasTPBody(T, p, Y, s, mu, none, false);
+    }
+    template <bool KEPT>
+    __device__ __attribute__((always_inline)) inline int gasTPBody(R T, R p, const R* Y, S& s, R* mu, SharedT<KEPT>& k,
                                                                    bool both) {
         if (!fin(T) || !fin(p) || T <= 0 || p <= 0) return kBadInput;
         R x[NS], W = 0;
         int st = massToMole(mod().gas, Y, x, W);
         if (st != kOk) return st;
-        Shared own;
-        Shared& k = sh ? *sh : own;
-        if (!sh || !sh->mixed) {
+        if (!k.mixed) {
             st = mixing(mod().gas, T, x, k.mx);
             if (st != kOk) return st;
-            if (sh) {
-                idealAt(mod().gas, T, sh->ideal);
-                sh->mixed = true;
-            }
+            if constexpr (KEPT) idealAt(mod().gas, T, k.ideal);
+            k.mixed = true;
         }
         if (both) st = roots<kOuterRoots>(T, p, k.mx.a, k.mx.b, k.mx.aa, k.r);
         else st = roots<kLargestRoot>(T, p, k.mx.a, k.mx.b, k.mx.aa, k.r);
         if (st != kOk) return st;
-        if (sh) sh->rooted = both;
+        k.rooted = both;
         if (!k.r.gas) return kUnavailable;
-        st = stateTrho(mod().gas, T, W / k.r.vLast, x, W, k.mx, s, mu, sh ? &sh->ideal : nullptr);
+        if constexpr (KEPT) st = stateTrho(mod().gas, T, W / k.r.vLast, x, W, k.mx, s, mu, &k.ideal);
+        else st = stateTrho(mod().gas, T, W / k.r.vLast, x, W, k.mx, s, mu);
         if (st != kOk) return st;
         st = finishState<NS>(gasHeuristic(x, W, k.mx), T, s, mu);
         if (st != kOk) return st;
@@ -580,7 +588,12 @@ struct Flash : FlashCap<CAP, R> {
     }
 
     // reactiveDeviceFlash.h:157-196 for index -1 (gas) and 0 (liquid).
-    RD int phaseStatus(int index, R p, R T, const R* Y, S& out, R* mu, Shared* sh = nullptr, bool both = false) {
+    RD int phaseStatus(int index, R p, R T, const R* Y, S& out, R* mu) {
+        Alone none;
+        return phaseStatus(index, p, T, Y, out, mu, none);
+    }
+    template <bool KEPT>
+    RD int phaseStatus(int index, R p, R T, const R* Y, S& out, R* mu, SharedT<KEPT>& known, bool both = false) {
         ++n.phases;
         if (!bounds(p, T)) return kBadInput;
         if (index >= 0 && T < liquidTmin) return kBadInput;
@@ -589,8 +602,12 @@ struct Flash : FlashCap<CAP, R> {
             for (int k = 0; k < NS; ++k)
                 if (Y[k] > 0 && (T < R(mod().gas.tlo[k]) || T > R(mod().gas.thi[k]))) return kBadInput;
         if constexpr (P::single ? RAMD_SEARCH_INLINE != 0 : RAMD_FLASH_INLINE != 0) {
-            if (index >= 0) return liquidTPBody(T, p, out, mu, sh);
-            return gasTPBody(T, p, Y, out, mu, sh, both);
+            if (index >= 0) {
+                const Shared* gas = nullptr;
+                if constexpr (KEPT) gas = known.rooted ? &known : nullptr;
+                return liquidTPBody(T, p, out, mu, gas);
+            }
+            return gasTPBody(T, p, Y, out, mu, known, both);
         }
         if (index >= 0) return liquidTP(T, p, out, mu);
         return gasTP(T, p, Y, out, mu);
@@ -743,14 +760,13 @@ struct Flash : FlashCap<CAP, R> {
         const R pg = gasPressure(p), pl = liquidPressure(p);
         const bool withLiquid = NL && (mass0 > 0 || (virtualLiquids && q[c] > 0));
         // one species, one table, one pressure: the liquid shares the gas's mixing, ideal part and cubic
-        Shared shared;
+        std::conditional_t<NS == 1 && NL != 0, Shared, Alone> shared;
         const bool share = NS == 1 && NL && withLiquid && mod().twin != 0 && pg == pl;
-        shared.mixed = shared.rooted = false;
         if (mg > 0) {
             for (int k = 0; k < NS; ++k) gas[k] /= mg;
             S prop;
             R mu[NS];
-            if (phaseStatus(-1, pg, T, gas, prop, virtualLiquids ? mu : nullptr, share ? &shared : nullptr, share) != kOk)
+            if (phaseStatus(-1, pg, T, gas, prop, virtualLiquids ? mu : nullptr, shared, share) != kOk)
                 return false;
             if constexpr (RJ) v.ref.gasMolarVolume = prop.V;
             accumulate(v, mg, prop, pg);
@@ -774,8 +790,7 @@ struct Flash : FlashCap<CAP, R> {
                     ++n.phases;
                     st = cacheStatus;
                 } else {
-                    st = phaseStatus(0, pl, T, nullptr, prop, virtualLiquids ? mu : nullptr,
-                                     shared.rooted ? &shared : nullptr);
+                    st = phaseStatus(0, pl, T, nullptr, prop, virtualLiquids ? mu : nullptr, shared);
                     if (unavailable(st) && T >= liquidTmin && T < liquidTc * (R(1) - R(1e-10))) {
                         cacheP = p; cacheT = T; cacheVirtual = virtualLiquids; cacheStatus = st;
                     }
@@ -832,7 +847,6 @@ struct Flash : FlashCap<CAP, R> {
         ++n.phases;
         S prop;
         Shared shared;
-        shared.mixed = shared.rooted = false;
         {
             if (!fin(T) || !fin(rho) || T <= 0 || rho <= 0) return false;
             R x[NS], W = 0;
@@ -849,7 +863,7 @@ struct Flash : FlashCap<CAP, R> {
         if (!bounds(p, T)) return false;
         if (check) {
             S gas;
-            if (phaseStatus(-1, gasP, T, Y, gas, nullptr, &shared) != kOk || ab(gas.rho - rho) > R(P::densityCheck) * rho)
+            if (phaseStatus(-1, gasP, T, Y, gas, nullptr, shared) != kOk || ab(gas.rho - rho) > R(P::densityCheck) * rho)
                 return false;
         }
         F = rho * prop.e - energy;
