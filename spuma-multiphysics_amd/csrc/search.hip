@@ -23,6 +23,11 @@
 #ifndef RAMD_SLOW_PHASES
 #define RAMD_SLOW_PHASES 64
 #endif
+// A list of up to this many such starts runs on groups of eight lanes, a
+// longer one a start per lane (searchSlowKernel).
+#ifndef RAMD_SLOW_GROUPS
+#define RAMD_SLOW_GROUPS 196608
+#endif
 
 namespace ramd {
 
@@ -91,34 +96,40 @@ __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchStartsKernel(
     if (threadIdx.x == 0) atomicAdd(phases, (unsigned long long)sum);
 }
 
-// The listed (list position, start) pairs, one per group of eight lanes: a
-// line search tries eight fractions at a time and the difference Jacobian its
-// six points, as the solve of one lane would one after the other.  A crawling
-// start's latency (ninety iterations of up to thirty fractions) is what the
-// search of a small or mid-size batch waits for: 40^3 binary cells 55 ms on
-// one lane per start, now 26 with both kernels.  A pure fluid's few starts
-// without a table point (47^3 cells) end as soon on one lane, 3.2 ms against
-// 3.6, and are not listed.
-template <int NS, int NL>
+// The listed (list position, start) pairs, each on GROUP lanes.  On a group
+// of eight a line search tries eight fractions at a time and the difference
+// Jacobian its six points, as the solve of one lane would one after the
+// other, with the same result.  A crawling start's latency (ninety iterations of
+// up to thirty fractions) is what the search of a small or mid-size batch
+// waits for: a 40^3 binary box's search (57,000 crawling starts a flash) 37
+// ms on groups, 68 with a start per lane.  A list that fills the chip with
+// one start per lane is bound by its evaluations instead, of which a group
+// makes several times as many: 160^3 (3.7 million) 1,500 ms on groups, 1,130
+// per lane.  The line: 56^3 (156,000) 75 and 80 ms, 64^3 (234,000) 105 and 93.
+// A pure fluid's few starts without a table point (47^3 cells) end as soon on
+// one lane, 3.2 ms against 3.6, and are not listed.  Both kernels are launched
+// and the count on the device chooses.
+template <int NS, int NL, int GROUP>
 __global__ __launch_bounds__(64, RAMD_SEARCH_MIN_WAVES) void searchSlowKernel(
     const HemModel<NS>* __restrict__ globalModel, FlashCells cells, CellList list, size_t stride,
     StartRecord* __restrict__ records, const uint32_t* __restrict__ slow, const unsigned* __restrict__ slowCount,
     unsigned long long* __restrict__ phases) {
+    constexpr uint32_t kEach = 64u / GROUP;  // starts per wave
     const uint32_t count = *slowCount;
-    if (blockIdx.x * 8u >= count) return;  // uniform per workgroup
+    if (blockIdx.x * kEach >= count || (count <= RAMD_SLOW_GROUPS) != (GROUP > 1)) return;  // uniform per workgroup
     const HemModel<NS>& model = workgroupModel(globalModel);
     uint32_t total = 0;
-    for (uint32_t base = blockIdx.x * 8u; base < count; base += gridDim.x * 8u) {
-        const uint32_t k = base + threadIdx.x / 8u;
+    for (uint32_t base = blockIdx.x * kEach; base < count; base += gridDim.x * kEach) {
+        const uint32_t k = base + threadIdx.x / GROUP;
         if (k < count) {
             const uint32_t i = slow[k] / 8u, start = slow[k] % 8u;
             Counts n = {0, 0, 0, 0, 0, 0, 0};
-            Flash<NS, NL, float, true, false, false, kModelLds, 8> f(model, n);
+            Flash<NS, NL, float, true, false, false, kModelLds, GROUP> f(model, n);
             cells.load<NS>(f, list.cells[i]);
             StartRecord r;
             r.bits = start >= 2 ? f.searchSeed(int(start), r.x) : f.searchFrozen(start == 1, r.x);
             r.bits |= n.phases << 2;
-            if (threadIdx.x % 8u == 0) {
+            if (threadIdx.x % GROUP == 0) {
                 records[size_t(start) * stride + i] = r;
                 total += n.phases;
             }
@@ -528,9 +539,16 @@ void launchSearchStarts(int ns, int nl, const void* model, const FlashCells& cel
     hipLaunchKernelGGL((searchStartsKernel<NS_, NL_>), dim3(blocks, kStarts), dim3(64), 0, stream,            \
                        static_cast<const HemModel<NS_>*>(model), cells, list, stride,                                   \
                        directed ? sets : nullptr, scratch.records, scratch.restarts, scratch.slowCount, phases); \
-    if constexpr (NS_ > 1 && NL_ > 0) hipLaunchKernelGGL((searchSlowKernel<NS_, NL_>), dim3(unsigned(std::min(size_t(kListWaves), (stride * kStarts + 7) / 8))), dim3(64), 0, \
-                       stream, static_cast<const HemModel<NS_>*>(model), cells, list, stride, scratch.records, \
-                       scratch.restarts, scratch.slowCount, phases);                                          \
+    if constexpr (NS_ > 1 && NL_ > 0) {                                                                       \
+        const size_t slow = std::min(stride * kStarts, size_t(RAMD_SLOW_GROUPS));                             \
+        hipLaunchKernelGGL((searchSlowKernel<NS_, NL_, 8>), dim3(unsigned(std::min(size_t(kListWaves), (slow + 7) / 8))), \
+                           dim3(64), 0, stream, static_cast<const HemModel<NS_>*>(model), cells, list, stride, \
+                           scratch.records, scratch.restarts, scratch.slowCount, phases);                     \
+        if (stride * kStarts > RAMD_SLOW_GROUPS)                                                              \
+            hipLaunchKernelGGL((searchSlowKernel<NS_, NL_, 1>), dim3(kListWaves), dim3(64), 0, stream,         \
+                               static_cast<const HemModel<NS_>*>(model), cells, list, stride, scratch.records, \
+                               scratch.restarts, scratch.slowCount, phases);                                  \
+    }                                                                                                         \
     hipLaunchKernelGGL((searchMergeKernel<NS_>), dim3(std::min(2048u, (waves + 3) / 4)), dim3(256), 0, stream, \
                        static_cast<const HemModel<NS_>*>(model), cells, list, stride, scratch.records, sets, cost, \
                        scratch.restarts, scratch.restartCount);                                              \
