@@ -5,11 +5,15 @@
 # Stack slots are not shared: where the lanes of a wave take both sides of a
 # branch around calls, the compiler keeps the scalar registers that one side
 # saves (stores of all 64 lanes) in slots that lanes of the other side still use.
-# lanes.hip: the registers that hold saved scalars are allocated without
+# lanes.hip, two.hip: the registers that hold saved scalars are allocated without
 # splitting (-wwm-regalloc=basic).  A split's copy runs for all 64 lanes, and
 # the ordinary allocation puts single lanes' moves and spills inside it (up to
 # 42 instructions in the FP64 flash's frozen solve), which overwrote other
 # lanes' values: a batch of binary cells, one per lane, read a wild pointer.
+# Constants stay in the loops that use them there (-disable-machine-licm):
+# hoisted, they are most of the scalars to save (of two.hip's 19,000 saves
+# 8,600 are left), and with it a batch of 80,000 binary cells takes 1,516 ms
+# instead of 1,798.
 # The other files' kernels have no such copy with anything inside it; a change
 # to the code around them can bring one (tests/test_whole_wave_registers.py
 # looks the built library over).
@@ -29,7 +33,7 @@ for src in "$here"/csrc/*.hip; do
   extra=()
   # the FP32 candidate search may use approximate reciprocals and transcendentals
   if [ "$(basename "$src")" = "search.hip" ]; then extra=(-freciprocal-math -fapprox-func); fi
-  if [ "$(basename "$src")" = "lanes.hip" ]; then extra=(-mllvm -wwm-regalloc=basic); fi
+  if [ "$(basename "$src")" = "lanes.hip" ] || [ "$(basename "$src")" = "two.hip" ]; then extra=(-mllvm -wwm-regalloc=basic -mllvm -disable-machine-licm); fi
   "$hipcc" "${flags[@]}" "${extra[@]}" -c "$src" -o "$obj" 2> >(grep -v "packed-fp32-ops" >&2) &
   objs+=("$obj")
   pids+=("$!")

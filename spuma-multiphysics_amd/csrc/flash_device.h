@@ -936,6 +936,21 @@ struct Flash : FlashCap<CAP, R> {
         }
         return volRes <= vtol && enRes <= etol;
     }
+    // How a lane left a solver's loop, in a vector register.  As a boolean it
+    // becomes a mask of the wave's lanes that the loop adds to; where the
+    // scalar registers are short that mask is kept in lanes of a vector
+    // register which the compiler (ROCm 7.2) takes for undefined again inside
+    // the loop, and the lanes that left in an earlier iteration than the last
+    // ones lost their result: of 884,736 binary cells two came out another
+    // way, one of them as a failure.  (A pure fluid's one-lane solvers have
+    // scalars enough, and are built without split copies only as they were.)
+    enum Left : int { kFailed = 0, kArrived = 1, kFinished = 2 };
+    static RD void keepInLanes(int& left) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        if constexpr (GROUP > 1 || NS > 1) asm volatile("" : "+v"(left));
+#endif
+        (void)left;
+    }
     // Fixed split, 2x2 Newton in (ln p, ln T) with line search (reactiveDeviceFlash.h:300-326).
     // polish > 0 (FP64 refinement only): up to that many further Newton steps
     // once the tolerances hold, while the residual is above 1e-3 of them; a
@@ -948,6 +963,7 @@ struct Flash : FlashCap<CAP, R> {
         if (!evaluate(mass0, p, T, value, false)) return false;
         int stalls = 0;
         bool polishing = false;
+        int left = -1;
         for (int it = 0; it < 70; ++it) {
             const R scale = energyScale(value), rv = value.volume - R(1), re = (value.energy - energy) / scale;
             if constexpr (E::kOutputs) {
@@ -960,14 +976,18 @@ struct Flash : FlashCap<CAP, R> {
                     --polish;
                     polishing = true;
                 } else {
-                    return true;
+                    left = 1;
+                    break;
                 }
             }
             R jac[3][3] = {};
             jac[0][0] = value.Vp * p; jac[0][1] = value.VT * T;
             jac[1][0] = value.Ep * p / scale; jac[1][1] = value.ET * T / scale;
             R rhs[2] = {-rv, -re}, step[2];
-            if (!solveN<2>(jac, rhs, step)) return polishing;
+            if (!solveN<2>(jac, rhs, step)) {
+                left = polishing;
+                break;
+            }
             const R limit = hi(R(1), hi(ab(step[0]) / R(.7), ab(step[1]) / R(.2)));
             step[0] /= limit; step[1] /= limit;
             const R previous = hi(ab(rv), ab(re));
@@ -1015,7 +1035,7 @@ struct Flash : FlashCap<CAP, R> {
                     if (pp == p && tt == T) break;
                 if constexpr (P::single) {
                     overrun = n.phases > phaseLimit;
-                    if (overrun) return false;
+                    if (overrun) break;
                 }
                 if (evaluate(mass0, pp, tt, trial, false)) {
                     const R next = hi(ab(trial.volume - R(1)), ab(trial.energy - energy) / scale);
@@ -1026,15 +1046,23 @@ struct Flash : FlashCap<CAP, R> {
                     }
                 }
             }
+            if (P::single && overrun) {
+                left = 0;
+                break;
+            }
             if (!accepted) {
                 stalled = P::single && previous <= R(P::handOver);
-                return polishing;
+                left = polishing;
+                break;
             }
             if (stallLimit > 0 && stalls >= stallLimit &&
-                !(ab(value.volume - R(1)) <= vtol && ab(value.energy - energy) / energyScale(value) <= etol))
-                return false;
+                !(ab(value.volume - R(1)) <= vtol && ab(value.energy - energy) / energyScale(value) <= etol)) {
+                left = 0;
+                break;
+            }
         }
-        return polishing;
+        keepInLanes(left);
+        return left < 0 ? polishing : left != 0;
     }
     // Residual [V-1, (E-e)/scale, mu_l/RT - mu_g/RT] in x = [ln p, ln T, beta]
     // (reactiveDeviceFlash.h:327-337).
@@ -1396,6 +1424,7 @@ struct Flash : FlashCap<CAP, R> {
         R f[3];
         if (!residual(x, scale, f, &value)) return false;
         bool polishing = false;  // converged already; a failed polishing step keeps the point
+        int left = kFailed;
         for (int it = 0; it < 90; ++it) {
             const R chemical = hi(R(0), ab(f[2]));
             R jac[3][3];
@@ -1406,27 +1435,29 @@ struct Flash : FlashCap<CAP, R> {
                     value.chemRes = chemical;
                     value.iterations = it;
                 }
-                if (P::single) return true;
+                if (P::single) {
+                    left = kArrived;
+                    break;
+                }
                 const bool tight = ab(f[0]) <= R(1e-3) * vtol && ab(f[1]) <= R(1e-3) * etol &&
                                    chemical <= R(1e-3) * mutol;
                 if (polish > 0 && !tight) {
                     --polish;
                     polishing = true;
                 } else {
-                    return activeFinish(x, scale, f, value);
+                    left = kFinished;
+                    break;
                 }
             }
             if constexpr (A && NS == 1) {
                 analyticJacobian(value, scale, jac);
             } else if constexpr (A) {
-                if (!analyticJacobianFinite(value, scale, jac) && !jacobian(x, scale, f, jac))
-                    return polishing && activeFinish(x, scale, f, value);
+                if (!analyticJacobianFinite(value, scale, jac) && !jacobian(x, scale, f, jac)) break;
             } else {
-                if (!referenceJacobian(x, scale, value, jac) && !jacobian(x, scale, f, jac))
-                    return polishing && activeFinish(x, scale, f, value);
+                if (!referenceJacobian(x, scale, value, jac) && !jacobian(x, scale, f, jac)) break;
             }
             R rhs[3] = {-f[0], -f[1], -f[2]}, step[3];
-            if (!solveN<3>(jac, rhs, step)) return polishing && activeFinish(x, scale, f, value);
+            if (!solveN<3>(jac, rhs, step)) break;
             R limiter = hi(R(1), hi(ab(step[0]) / R(.7), ab(step[1]) / R(.18)));
             bool vapourCoordinates = false;
             if constexpr (CAP) vapourCoordinates = this->adaptive;
@@ -1511,7 +1542,7 @@ struct Flash : FlashCap<CAP, R> {
                     if (tx[0] == x[0] && tx[1] == x[1] && tx[2] == x[2]) break;
                 if constexpr (P::single) {
                     overrun = n.phases > phaseLimit;
-                    if (overrun) return false;
+                    if (overrun) break;
                 }
                 E trial;
                 if (residual(tx, scale, tf, &trial) &&
@@ -1523,12 +1554,15 @@ struct Flash : FlashCap<CAP, R> {
                 }
             }
             }
+            if (P::single && overrun) break;
             if (!accepted) {
                 stalled = P::single && previous <= R(P::handOver);
-                return polishing && activeFinish(x, scale, f, value);
+                break;
             }
         }
-        return polishing && activeFinish(x, scale, f, value);
+        if (left == kFailed && polishing) left = kFinished;  // the converged point is kept
+        keepInLanes(left);
+        return left == kFinished ? activeFinish(x, scale, f, value) : left == kArrived;
     }
     // activeNewton of a pure fluid with this build's analytic Jacobian, as one
     // loop around one evaluation, so that all of it inlines and its state

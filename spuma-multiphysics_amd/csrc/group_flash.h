@@ -12,8 +12,8 @@
 // of those iterations; in a batch large enough to fill the chip with one cell
 // per lane, the lanes a cell's own starts leave idle cost more than that.
 //
-// Launched by group.hip; those of two species without a liquid by lanes.hip
-// (built otherwise, see lane_flash.h).
+// Launched by group.hip; those of two species by two.hip (built otherwise,
+// see lane_flash.h).
 #ifndef RAMD_GROUP_FLASH_H
 #define RAMD_GROUP_FLASH_H
 #include "flash_step.h"
@@ -101,11 +101,13 @@ __global__ __launch_bounds__(WIDE ? kQueueThreads : 64, RAMD_REFINE_MIN_WAVES) v
     }
 }
 
-// The launches of lanes.hip: two species without a liquid.
-void launchGasGroupFlash(bool capillaryFlash, const void* model, const FlashCells& cells, const uint32_t* order,
-                         uint32_t count, const HemCapillaryDev* capillary, const FlashSink& sink, hipStream_t stream);
-void launchGasRefineQueue(const void* model, const FlashCells& cells, const uint32_t* queue, const unsigned* queueCount,
-                          const CandidateSet* sets, const FlashSink& sink, hipStream_t stream);
+// The launches of two.hip: two species.
+void launchGroupFlashTwo(int nl, bool analytic, bool capillaryFlash, const void* model, const FlashCells& cells,
+                         const uint32_t* order, uint32_t count, const HemCapillaryDev* capillary,
+                         const FlashSink& sink, hipStream_t stream);
+void launchRefineQueueTwo(int nl, const void* model, const FlashCells& cells, const uint32_t* queue,
+                          const unsigned* queueCount, const CandidateSet* sets, const FlashSink& sink,
+                          hipStream_t stream);
 
 }  // namespace ramd
 #endif

@@ -25,6 +25,7 @@
 #include "hem_internal.h"
 #include "flash_step.h"
 #include "lane_flash.h"
+#include "refine_flash.h"
 #include "reactive_gpu_hem.h"
 #include "reactive_amd.h"
 
@@ -37,42 +38,6 @@ static_assert(sizeof(HemCapillaryDev) == sizeof(ReactiveGpuHemCapillaryInputV2) 
 static_assert(sizeof(HemOutputDev) == sizeof(ReactiveGpuHemOutputV1) &&
                   offsetof(HemOutputDev, success) == offsetof(ReactiveGpuHemOutputV1, success),
               "output layout");
-
-// Mixed arithmetic, second half: FP64 refinement, stability and selection of
-// the listed cells' candidates; deferred cells go to the queue, or, where the
-// candidates came from the saturation table, to the list of cells to search.
-template <int NS, int NL>
-__global__ __launch_bounds__(64, RAMD_REFINE_MIN_WAVES) void hemRefineKernel(const HemModel<NS>* __restrict__ globalModel,
-                                                     FlashCells cells, CellList list,
-                                                     const CandidateSet* __restrict__ sets,
-                                                     HemOutputDev* __restrict__ out,
-                                                     unsigned long long* __restrict__ totals,
-                                                     uint32_t* __restrict__ queue, unsigned* __restrict__ queueCount,
-                                                     uint32_t* __restrict__ search,
-                                                     unsigned* __restrict__ searchCount) {
-    const uint32_t count = list.size();
-    if (blockIdx.x * 64u >= count) return;  // uniform per workgroup
-    const HemModel<NS>& model = workgroupModel(globalModel);
-    Counts n = {0, 0, 0, 0, 0, 0, 0};
-    uint32_t succeeded = 0;
-    for (uint32_t i = blockIdx.x * 64u + threadIdx.x; i < count; i += gridDim.x * 64u) {
-        const uint32_t c = list.cells[i];
-        Flash<NS, NL, double, true, false, false, kModelLds> f(model, n);
-        cells.load<NS>(f, c);
-        EvalT<double, true> result;
-        zeroEval(result);
-        bool deferred = false;
-        const bool ok = f.refine(sets[c], result, &deferred);
-        if (deferred) {
-            if (sets[c].flags & kDirect) search[atomicAdd(searchCount, 1u)] = c;
-            else queue[atomicAdd(queueCount, 1u)] = c;
-        } else {
-            storeHemCell(ok, result, out[c]);
-            succeeded += ok ? 1u : 0u;
-        }
-    }
-    addTotals(n, succeeded, totals);
-}
 
 __global__ void clearCountsKernel(unsigned* __restrict__ counts) {
     if (threadIdx.x < kListCounts) counts[threadIdx.x] = 0;
@@ -195,21 +160,20 @@ void HemHandle::launchMixed(const double* q, const double* e, const ThermoOut* g
     else launchSearchStarts(ns, nl, model, cells, whole, count, scratch, false, sets, nullptr, totals + 8, s);
     if (saturation)
         launchRefineTwoPhase(model, cells, order, uint32_t(count), sets, sink, scratch, searchList, searchCount, s);
-#define RAMD_HEM_MIXED(NS_, NL_)                                                                                  \
-    hipLaunchKernelGGL((hemRefineKernel<NS_, NL_>), dim3(blocks), dim3(64), 0, s,                                   \
-                       static_cast<const HemModel<NS_>*>(model), cells, first, sets, out, totals, queue,          \
-                       queueCount, searchList, searchCount);                                                      \
-    if (saturation) {                                                                                             \
-        launchSearchStarts(ns, nl, model, cells, left, count, scratch, true, sets, nullptr, totals + 8, s);       \
-        hipLaunchKernelGGL((hemRefineKernel<NS_, NL_>), dim3(std::min(2048u, blocks)), dim3(64), 0, s,              \
-                           static_cast<const HemModel<NS_>*>(model), cells, left, sets, out, totals, queue,       \
-                           queueCount, searchList, searchCount);                                                  \
+    const auto refine = [&](const CellList& list, unsigned grid) {
+        if (ns == 2) return launchHemRefineTwo(nl, model, cells, list, sets, sink, queue, queueCount, grid, s);
+#define RAMD_HEM_REFINE(NL_)                                                                                      \
+    hipLaunchKernelGGL((hemRefineKernel<1, NL_>), dim3(grid), dim3(64), 0, s, static_cast<const HemModel<1>*>(model), \
+                       cells, list, sets, out, totals, queue, queueCount, searchList, searchCount)
+        if (nl == 0) RAMD_HEM_REFINE(0);
+        else RAMD_HEM_REFINE(1);
+#undef RAMD_HEM_REFINE
+    };
+    refine(first, blocks);
+    if (saturation) {
+        launchSearchStarts(ns, nl, model, cells, left, count, scratch, true, sets, nullptr, totals + 8, s);
+        refine(left, std::min(2048u, blocks));
     }
-    if (ns == 1 && nl == 0) { RAMD_HEM_MIXED(1, 0); }
-    else if (ns == 1) { RAMD_HEM_MIXED(1, 1); }
-    else if (nl == 0) { RAMD_HEM_MIXED(2, 0); }
-    else { RAMD_HEM_MIXED(2, 1); }
-#undef RAMD_HEM_MIXED
     launchRefineQueue(ns, nl, model, cells, queue, queueCount, sets, sink, s);
     hipLaunchKernelGGL(queueCountKernel, dim3(1), dim3(64), 0, s, queueCount, totals + 9);
     RAMD_HIP(hipGetLastError());

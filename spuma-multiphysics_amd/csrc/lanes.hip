@@ -1,10 +1,8 @@
 // SPDX-License-Identifier: GPL-3.0-or-later
 // FP64 flashes of one cell per lane of two species, the analytic-Jacobian mode
-// and the capillary / boundary-search flash (see lane_flash.h), and of one cell
-// per wave of two species without a liquid (group_flash.h).
+// and the capillary / boundary-search flash (see lane_flash.h).
 #include <hip/hip_runtime.h>
 #include "lane_flash.h"
-#include "group_flash.h"
 
 namespace ramd {
 
@@ -43,25 +41,6 @@ void launchLaneHem(int ns, int nl, bool analytic, bool boundary, const void* mod
         else RAMD_HEM_LAUNCH(2, 1, true, false);
     }
 #undef RAMD_HEM_LAUNCH
-    RAMD_HIP(hipGetLastError());
-}
-
-void launchGasGroupFlash(bool capillaryFlash, const void* model, const FlashCells& cells, const uint32_t* order,
-                         uint32_t count, const HemCapillaryDev* capillary, const FlashSink& sink, hipStream_t stream) {
-    const auto* m = static_cast<const HemModel<2>*>(model);
-    if (capillaryFlash)
-        hipLaunchKernelGGL((groupFlashKernel<2, 0, false, true>), dim3(count), dim3(64), 0, stream, m, cells, order,
-                           capillary, sink);
-    else
-        hipLaunchKernelGGL((groupFlashKernel<2, 0, false, false>), dim3(count), dim3(64), 0, stream, m, cells, order,
-                           capillary, sink);
-    RAMD_HIP(hipGetLastError());
-}
-
-void launchGasRefineQueue(const void* model, const FlashCells& cells, const uint32_t* queue, const unsigned* queueCount,
-                          const CandidateSet* sets, const FlashSink& sink, hipStream_t stream) {
-    hipLaunchKernelGGL((refineQueueKernel<2, 0, false>), dim3(RAMD_QUEUE_BLOCKS), dim3(64), 0, stream,
-                       static_cast<const HemModel<2>*>(model), cells, queue, queueCount, sets, sink);
     RAMD_HIP(hipGetLastError());
 }
 

@@ -32,54 +32,12 @@
 #include "cartesian_kernels.h"
 #include "flash_step.h"
 #include "lane_flash.h"
+#include "refine_flash.h"
 #include "reactive_amd.h"
 
 namespace ramd {
 
 // ---------------------------------------------------------------- kernels
-// Mixed precision, second half: FP64 refinement, stability and selection of
-// the listed cells' candidates.  Deferred cells go to the queue, or, where
-// the candidates came from the saturation table, to the list of cells to
-// search.  A list counted on the device is swept in rounds.
-template <int NS, int NL>
-__global__ __launch_bounds__(256, RAMD_REFINE_MIN_WAVES) void stepRefineKernel(const HemModel<NS>* __restrict__ globalModel,
-                                                       FlashCells cells, CellList list,
-                                                       const CandidateSet* __restrict__ sets,
-                                                       ThermoOut* __restrict__ out, double* __restrict__ pOut,
-                                                       double* __restrict__ cOut, double* __restrict__ rOut,
-                                                       uint16_t* __restrict__ cost,
-                                                       unsigned long long* __restrict__ counters,
-                                                       uint32_t* __restrict__ queue, unsigned* __restrict__ queueCount,
-                                                       uint32_t* __restrict__ search, unsigned* __restrict__ searchCount,
-                                                       uint8_t* __restrict__ failMark) {
-    const uint32_t count = list.size();
-    if (blockIdx.x * blockDim.x >= count) return;  // uniform per workgroup
-    const HemModel<NS>& model = workgroupModel(globalModel);
-    uint32_t failed = 0, phases = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
-        const uint32_t c = list.cells[i];
-        if (!cells.flashed(c)) continue;
-        Counts n = {0, 0, 0, 0, 0, 0, 0};
-        Flash<NS, NL, double, true, false, false, kModelLds> f(model, n);
-        cells.load<NS>(f, c);
-        EvalT<double, true> result;
-        zeroEval(result);
-        bool deferred = false;
-        const bool ok = f.refine(sets[c], result, &deferred);
-        if (deferred) {
-            if (sets[c].flags & kDirect) search[atomicAdd(searchCount, 1u)] = c;
-            else queue[atomicAdd(queueCount, 1u)] = c;
-        } else {
-            storeCell(ok, result, cells.seeds[c], c, out, pOut, cOut, rOut);
-            if (!ok && failMark) failMark[c] = 1;
-            failed += ok ? 0u : 1u;
-            if (cost) cost[c] = uint16_t(n.phases < 65535u ? n.phases : 65535u);
-        }
-        phases += n.phases;
-    }
-    countFlash(failed, phases, counters);
-}
-
 __global__ void clearQueueKernel(unsigned* __restrict__ counts) {
     if (threadIdx.x < kListCounts) counts[threadIdx.x] = 0;
 }
@@ -581,11 +539,6 @@ __global__ void copyFixedKernel(const double* __restrict__ tq, const ReactiveTra
 inline unsigned blocksFor(size_t n, unsigned b) { return unsigned((n + b - 1) / b); }
 // Waves of the refinement over the searched remainder (two fit a SIMD).
 constexpr unsigned kListBlocks = 2048;
-#define RAMD_STEP_SPECIES(LAUNCH)                     \
-    if (h->ns == 1 && h->nl == 0) { LAUNCH(1, 0); }   \
-    else if (h->ns == 1) { LAUNCH(1, 1); }            \
-    else if (h->nl == 0) { LAUNCH(2, 0); }            \
-    else { LAUNCH(2, 1); }
 constexpr int kMarks = 11;  // events per step
 
 // ---------------------------------------------------------------- handle
@@ -750,11 +703,15 @@ struct Step {
                                    false, sets, searchCost, counters + 6, stream);
             if (split) RAMD_HIP(hipEventRecord(split, stream));
             const auto refine = [&](const CellList& list, unsigned grid, unsigned block) {
-#define RAMD_STEP_REFINE(NS_, NL_)                                                                                 \
-    hipLaunchKernelGGL((stepRefineKernel<NS_, NL_>), dim3(grid), dim3(block), 0, stream,                            \
-                       static_cast<const HemModel<NS_>*>(h->model), batch, list, sets, out, pOut, cOut, rOut,      \
+                if (ns == 2)
+                    return launchStepRefineTwo(h->nl, h->model, batch, list, sets, sink, queue, queueCount, grid, block,
+                                               stream);
+#define RAMD_STEP_REFINE(NL_)                                                                                      \
+    hipLaunchKernelGGL((stepRefineKernel<1, NL_>), dim3(grid), dim3(block), 0, stream,                              \
+                       static_cast<const HemModel<1>*>(h->model), batch, list, sets, out, pOut, cOut, rOut,        \
                        costOut, counter, queue, queueCount, searchList, searchCount, failMark)
-                RAMD_STEP_SPECIES(RAMD_STEP_REFINE)
+                if (h->nl == 0) RAMD_STEP_REFINE(0);
+                else RAMD_STEP_REFINE(1);
 #undef RAMD_STEP_REFINE
             };
             if (saturation) {
