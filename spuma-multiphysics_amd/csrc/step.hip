@@ -798,7 +798,13 @@ struct Step {
     // 4, 8 (stage 0 from q0, three launches each after a warm-up).  Flash (the
     // current arithmetic, into the scratch state buffers): state-order bins
     // per axis 32, 64, 128 with 64-lane workgroups, then workgroups of 64,
-    // 128, 256 lanes with the chosen bins.  Nothing it computes is kept.
+    // 128, 256 lanes with the chosen bins where the flash has a choice.
+    // Nothing it computes is kept.
+    // Whether any launch of the current flash takes its workgroup size from
+    // flashBlock: one wave per cell and a pure fluid's directed search do not.
+    bool blockChosen() const {
+        return mode == REACTIVE_AMD_FLASH_MIXED ? !h->pure() : cells > RAMD_GROUP_CELLS;
+    }
     float timeIt(const std::function<void()>& work, int reps) {
         RAMD_HIP(hipEventRecord(tuneEvents[0], stream));
         for (int r = 0; r < reps; ++r) work();
@@ -841,6 +847,7 @@ struct Step {
         stateLevels = bestLevels;
         unsigned bestBlock = 64;
         for (unsigned b : {64u, 128u, 256u}) {
+            if (b > 64u && !blockChosen()) break;
             flashBlock = b;
             const float ms = b == 64u ? best : timeIt(trial, 1);
             if (ms < best || b == 64u) { best = ms; bestBlock = b; }
