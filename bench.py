@@ -13,11 +13,10 @@ the plain FP64 path is timed on the same case for the comparison, and the
 two are compared cell by cell after one step from the same states.
 
 Prints one JSON line (the bench contract) with:
-  roofline       the dominant kernel of the step (the mixed flash's FP32
-                 candidate search, about two thirds of the step): VALU FLOPs
-                 (phase evaluations x FLOPs per evaluation) / event-timed
-                 launch duration vs the 157.3 TFLOP/s FP32 vector peak, and
-                 its measured HBM traffic per launch
+  roofline       the mixed flash's FP32 candidate search (about a third of
+                 the step): VALU FLOPs (phase evaluations x FLOPs per
+                 evaluation, an upper figure: see flop_source) / event-timed
+                 duration of its launches vs the 157.3 TFLOP/s FP32 vector peak
   roofline_stage fused flux sweep (both SSPRK2 stages): algorithmic bytes per
                  cell per stage / event-timed kernel duration vs 8 TB/s HBM
   roofline_flash all flash kernels: time per launch, phase evaluations
@@ -366,7 +365,9 @@ def distance(s, states0, root, ok):
 def flash_roofline(rep, rep64, cells, steps, mixed):
     """VALU rate of the flash kernels against the vector peaks (see FLOP_PER_PHASE)."""
     flashes = 2 * steps
-    out = {"bound": "valu", "unit": "TFLOP/s", "flop_source": "profiles/flash_valu_uniform32.txt",
+    out = {"bound": "valu", "unit": "TFLOP/s",
+           "flop_source": "profiles/flash_valu_uniform32.txt, measured before two states of an evaluation shared what "
+                          "they have in common: achieved and frac are upper figures",
            "profiled_commit": PROFILED_COMMIT}
     t64 = (rep64.flashSeconds[0] + rep64.flashSeconds[1]) / flashes
     a64 = rep64.phaseEvaluations / flashes * FLOP_PER_PHASE["fp64_flash"] / t64 / 1e12

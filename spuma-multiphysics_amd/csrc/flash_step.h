@@ -35,9 +35,10 @@
 #define RAMD_WIDE_CELLS 4096
 #endif
 // FP64 batches of up to this many cells run one cell per wave, its starts on
-// groups of eight lanes (group.hip); larger ones one cell per lane.
-// Measured, per lane and per wave: pure, 16,384 cells 45.9 and 15.7 ms, 65,536
-// cells 55.7 and 56.7; binary, 65,536 cells 1,812 and 461 ms.
+// groups of eight lanes (group_flash.h); larger ones one cell per lane.
+// Measured, per lane and per wave: pure, 16,384 cells 43.2 and 14.9 ms, 65,536
+// cells 51.4 and 54.1, where the line lies; binary, 65,536 cells 1,708 and 453
+// ms: two species cross later, at a size not measured.
 #ifndef RAMD_GROUP_CELLS
 #define RAMD_GROUP_CELLS 65536
 #endif
@@ -214,7 +215,7 @@ __device__ inline void countFlash(uint32_t failed, uint32_t phases, unsigned lon
     }
 }
 
-// ---- one cell per wave (group.hip) -----------------------------------------
+// ---- one cell per wave (group_flash.h) -------------------------------------
 // Where a cell's result and counts go: a HEM batch's records and totals (or a
 // slot of eight sums per workgroup in partials), or the step's arrays.
 struct FlashSink {

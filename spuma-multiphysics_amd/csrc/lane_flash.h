@@ -6,6 +6,8 @@
 // lanes.hip, whose compilation differs (build.sh): these kernels hold more
 // scalars than the registers take, and the ordinary allocation of the
 // registers that keep the rest let one lane's spills overwrite another's.
+// (Two species' flashes of one cell per wave, group_flash.h, and their
+// refinement, refine_flash.h, are built so in two.hip.)
 // That allocation costs the pure fluid's flash 30 % (64^3 cells, two steps:
 // 312 ms, 418 with it).
 #ifndef RAMD_LANE_FLASH_H

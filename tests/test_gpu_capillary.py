@@ -1,5 +1,6 @@
 """The capillary / boundary-search flash on the GPU (Flash<..., CAP> in
-csrc/flash_device.h, hemFlashKernel<..., CAP>): capillary recoveries with a
+csrc/flash_device.h, groupFlashKernel<..., CAP>; hemFlashKernel<..., CAP>, for
+long batches, in test_gpu_long_batches.py): capillary recoveries with a
 fixed interface (reactive_gpu_hem_run_v2 from host arrays and
 run_resident_v1 from device pointers) and boundaryRecovery = 1 models
 (reactive_gpu_hem_run_v1), on the reference-written fixtures
